@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstring>
 #include <numeric>
+#include <queue>
 
 namespace femhip {
 
@@ -60,23 +61,116 @@ __global__ void k_colscale(int n, const int* rp, const int* ci, const TI* Si, co
 // Barrier epochs restart at 1 every launch.  Barrier e uses buffer e & 3 and
 // tag (e >> 2) & 1 in the lowest mantissa bit, so before a launch buffer 0
 // must carry tag 0 and buffers 1-3 tag 1 (none of them looks "arrived").
+// One thread per value.
 // (A fill kernel rather than a memset node, so the launch sequence can be
 // captured in a graph.)
-__global__ void k_reset(Slot* slots, int nslots, double* scal, int nteams, int* abort_flag, Inst* insts,
-                        int ninst) {
+__global__ void k_reset(double* slots, int nrec, int rec_vals, int* abort_flag, Inst* insts, int ninst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const double tag1 = __longlong_as_double(1ll);  // smallest denormal: value 0, tag 1
-  const int per = kSlotBufs * kMaxRed;
-  if (i < nslots + nteams) {
-    double* v = (i < nslots) ? &slots[i].vals[0][0] : scal + (size_t)(i - nslots) * per;
-    for (int q = 0; q < per; q++) v[q] = (q < kMaxRed) ? 0.0 : tag1;
-  }
+  const int per = nrec * rec_vals;                // values of one buffer
+  if (i < 2 * kSlotBufs * per) slots[i] = (i / per) % kSlotBufs == 0 ? 0.0 : tag1;
   if (i == 0) *abort_flag = 0;
   if (i < ninst) {
     insts[i].counters[0] = 0;
     insts[i].counters[1] = 0;
     insts[i].counters[2] = 0;
     *insts[i].status = 0;
+  }
+}
+
+// Workgroups of k_reset.
+unsigned reset_grid(int nrec, int rec_vals, int ninst) {
+  return div_up(std::max(2LL * kSlotBufs * nrec * rec_vals, (long long)ninst), kBlock);
+}
+
+// Halos of one team-instance whose workgroups keep their rows in LDS
+// (HaloRef): workgroup `rank` collects the distinct columns outside its rows
+// in a hash table (at most rows x kCacheE of them, under two thirds of the
+// table), sorts them, and writes for every lane and entry the place of its
+// value in the staging area.  A halo beyond the capacity clears ref->ok: the
+// team then reads its neighbours from memory.  Run once per plan.
+constexpr int kHaloHash = 16384;
+__global__ void __launch_bounds__(kTeamBlock) k_halo(HaloRef* ref, int n, const int* rp, const int* ci,
+                                                     int rows_per_wg, int passes, int K, int* cnt_out, int* list,
+                                                     unsigned short* place) {
+  __shared__ int hash[kHaloHash], keys[kHaloHash];
+  __shared__ int cnt;
+  const int rank = blockIdx.x, tid = threadIdx.x;
+  const int lo = min(n, rank * rows_per_wg), hi = min(n, lo + rows_per_wg);
+  for (int i = tid; i < kHaloHash; i += kTeamBlock) hash[i] = -1;
+  if (tid == 0) cnt = 0;
+  __syncthreads();
+  for (int row = lo + tid; row < hi; row += kTeamBlock)
+    for (int s = rp[row]; s < rp[row + 1]; s++) {
+      const int c = ci[s];
+      if (c >= lo && c < hi) continue;
+      unsigned h = ((unsigned)c * 2654435761u) >> 18;
+      while (true) {
+        const int was = atomicCAS(&hash[h], -1, c);
+        if (was == -1) keys[atomicAdd(&cnt, 1)] = c;
+        if (was == -1 || was == c) break;
+        h = (h + 1) & (kHaloHash - 1);
+      }
+    }
+  __syncthreads();
+  const int total = cnt;
+  int m = 1;
+  while (m < total) m <<= 1;
+  for (int i = total + tid; i < m; i += kTeamBlock) keys[i] = INT32_MAX;
+  for (int k = 2; k <= m; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      __syncthreads();
+      for (int i = tid; i < m; i += kTeamBlock) {
+        const int p = i ^ j;
+        if (p > i) {
+          const int a = keys[i], b = keys[p];
+          if ((a > b) == ((i & k) == 0)) {
+            keys[i] = b;
+            keys[p] = a;
+          }
+        }
+      }
+    }
+  __syncthreads();
+  const int cap = ref->cap;
+  if (total > cap) {
+    if (tid == 0) {
+      ref->ok = 0;
+      cnt_out[rank] = 0;
+    }
+    return;
+  }
+  if (tid == 0) {
+    cnt_out[rank] = total;
+    atomicMax(&ref->max_n, total);
+  }
+  for (int i = tid; i < total; i += kTeamBlock) list[(size_t)rank * cap + i] = keys[i];
+  const int rpp = kTeamBlock / K;
+  for (int q = 0; q < passes; q++) {
+    const int row = lo + tid / K + q * rpp;
+    int s0 = 0, s1 = 0;
+    if (row < hi) {
+      s0 = rp[row];
+      s1 = rp[row + 1];
+    }
+    for (int e = 0; e < kCacheE; e++) {
+      int at = 0;
+      if (s0 + e < s1) {
+        const int c = ci[s0 + e];
+        if (c >= lo && c < hi) {
+          at = c - lo;
+        } else {
+          int a = 0, b = total;
+          while (a < b) {
+            const int mid = (a + b) >> 1;
+            if (keys[mid] < c) a = mid + 1;
+            else b = mid;
+          }
+          at = hi - lo + a;
+        }
+      }
+      place[(size_t)rank * ref->place_n + (q * kCacheE + e) * kTeamBlock + tid] = (unsigned short)at;
+    }
   }
 }
 
@@ -99,7 +193,7 @@ __global__ void k_get_cols(const double* src, int k, int col0, double* dst, int 
 void free_inst(InstHost& h) {
   void* ptrs[] = {h.d_S64, h.d_Si,    h.d_dinv64, h.d_dinvi, h.d_SDi, h.d_u, h.d_v,   h.d_a,
                   h.d_h3,  h.d_h4,    h.d_xnext,  h.d_hpre,  h.d_hvec, h.d_x, h.d_b, h.d_vec,
-                  h.d_surf, h.d_h5, h.d_h6};
+                  h.d_surf, h.d_h5, h.d_h6, h.d_xch};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (h.surf_done) (void)hipEventSynchronize(h.surf_done);
@@ -271,6 +365,7 @@ void fill_dev(fem_batch* b, InstHost& h) {
   I.h4 = h.d_h4;
   I.h5 = h.d_h5;
   I.h6 = h.d_h6;
+  I.xch = h.d_xch;
   I.xnext = h.d_xnext;
   I.hpre = h.d_hpre;
   I.hvec = h.d_hvec;
@@ -307,7 +402,8 @@ void fill_dev(fem_batch* b, InstHost& h) {
 }
 
 void free_plan(fem_batch* b) {
-  void* ptrs[] = {b->d_insts, b->d_teams, b->d_wg_team, b->d_team_inst, b->d_slots, b->d_scal};
+  void* ptrs[] = {b->d_insts, b->d_teams, b->d_wg_team, b->d_team_inst, b->d_slots, b->d_halo,
+                  b->d_halo_mem};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   b->d_insts = nullptr;
@@ -315,7 +411,8 @@ void free_plan(fem_batch* b) {
   b->d_wg_team = nullptr;
   b->d_team_inst = nullptr;
   b->d_slots = nullptr;
-  b->d_scal = nullptr;
+  b->d_halo = nullptr;
+  b->d_halo_mem = nullptr;
   b->uploaded.clear();
   b->plan_ready = false;
 }
@@ -323,27 +420,110 @@ void free_plan(fem_batch* b) {
 }  // namespace
 
 // Workgroups of the team of a lone instance, within maxb co-resident
-// workgroups: team_size when given and it fits, else about one row per lane
-// (at most 1024).
+// workgroups: team_size when given and it fits, else one per 128 rows x
+// columns, up to one per CU.  Few rows per workgroup leave most of its waves
+// to the halo and the control wave.  Where that would leave the flat reduction
+// (flat_reduction), its largest team is kept while its workgroups stay short:
+// the second level costs an iteration more than the longer gathers do (one
+// column, us per iteration: 9,801 rows 4.7 at 64 workgroups, 5.3 at 128;
+// 39,601 rows 4.3 and 4.5; 89,401 rows take two-level teams; two columns:
+// 2,562 rows 5.4 at 20 workgroups and 6.3 at 40, 10,242 rows 9.1 at 40 and
+// 7.6 at 160).
 int single_team_size(long long n, int k, int team_size, int maxb) {
   if (team_size > 0 && team_size <= maxb) return team_size;
   const long long lanes = n * k;
-  const int g = (int)std::max(1LL, (lanes + kBlock - 1) / kBlock);
-  return std::min(g, std::min(maxb, 1024));
+  int g = (int)std::min<long long>(1024, std::max(1LL, (lanes + 127) / 128));
+  const int flat = std::max(kGroup, 256 / (4 * k));
+  if (g > flat && lanes <= (long long)flat * (k == 1 ? 640 : 320)) g = flat;
+  return std::min(g, maxb);
 }
 
-// A workgroup of a multi-workgroup team whose rows exceed two per lane (the
-// kernel's LDS row cache) streams its phases.
+// Whether every workgroup of a team sums all records: one group's worth, or up
+// to 256 values, four per lane of the control wave; beyond, two levels.  The
+// flat form is one publish and poll, but every workgroup reads every record
+// (pipelined CG on 39,601 rows: 4.3 us an iteration flat at 64 workgroups, 5.3
+// at 128 and 6.8 at 256; in two levels 4.5 and 4.7).
+int flat_reduction(int size, int k) { return size <= kGroup || (long long)size * 4 * k <= 256 ? 1 : 0; }
+
+// Barrier records of a launch of `grid` workgroups, and a team's among them.
+size_t slot_bytes(int grid, int k) { return sizeof(double) * 2 * kSlotBufs * (size_t)grid * slot_vals(k); }
+void team_slots(Team* T, double* slots, int grid, int k) {
+  T->rec_vals = slot_vals(k);
+  T->buf_records = grid;
+  T->slots = slots + (size_t)T->first_wg * T->rec_vals;
+  T->groups = T->slots + (size_t)kSlotBufs * grid * T->rec_vals;
+}
+
+// A workgroup of a multi-workgroup team whose rows exceed kCacheP per lane (the
+// kernel's row cache) streams its phases.
 bool team_streams(long long n, int k, int size) {
   const long long rows = (n + size - 1) / size;
-  return rows * k > 2LL * kBlock;
+  return rows * k > (long long)kCacheP * kTeamBlock;
+}
+
+// Whether the workgroups of a team can keep the instance's rows in LDS, but
+// for the halo (HaloRef::ok): at most kCacheP rows per lane, rows of at most
+// kCacheE entries, and not classic CG.
+bool rows_fit(const fem_ctx* c, int k, int size, int kr) {
+  const long long rows = (c->n + size - 1) / size;
+  const int block = size == 1 ? kBlock : kTeamBlock;
+  return kr != 2 && c->max_row <= kCacheE && rows * k <= (long long)kCacheP * block;
+}
+
+// Co-resident workgroups that both variants of an exchange mode (rows in LDS
+// or not) hold.
+int variant_coresident(int k, int inner_fp32, int kr, int coh, int* blocks) {
+  int rc = step_max_coresident(k, inner_fp32, kr, coh, 0, blocks);
+  int with_rows = *blocks;
+  if (!rc && kr != 2) rc = step_max_coresident(k, inner_fp32, kr, coh, 1, &with_rows);
+  *blocks = std::min(*blocks, with_rows);
+  return rc;
 }
 
 // Exchange mode of a plan: plain for one-workgroup teams only; else forced,
-// then the autotuner's choice, then fenced for streaming teams, coherent
-// otherwise.
+// then the autotuner's choice, then fenced for teams that stream their phases
+// (more rows than the row cache holds), coherent otherwise.
 int exchange_mode(bool multi, bool streaming, int forced, int tuned) {
   return !multi ? 0 : forced ? forced : tuned ? tuned : streaming ? kExchangeFenced : kExchangeCoherent;
+}
+
+// The halos of one team-instance: whether its workgroups can keep their rows
+// in LDS at all, how many halo rows fit beside them (4 bytes of list and four
+// values of ti bytes per column each: the staged one and three Krylov
+// vectors), and the bytes its tables take.
+bool halo_shape(const fem_ctx* c, int k, int size, int ti, int kr, HaloShape* h) {
+  if (size <= 1 || c->n == 0 || !rows_fit(c, k, size, kr)) return false;
+  h->rows = (c->n + size - 1) / size;
+  h->passes = (int)div_up((long long)h->rows * k, kTeamBlock);
+  const int room = kTeamPool - rows_cells_bytes(h->passes, kTeamBlock, ti) - ti * h->rows * k;
+  h->cap = std::min(room / (4 + 4 * ti * k), h->rows * kCacheE);
+  h->place_n = h->passes * kCacheE * kTeamBlock;
+  h->n_bytes = (sizeof(int) * (size_t)size + 255) & ~size_t(255);
+  h->list_bytes = (sizeof(int) * (size_t)size * h->cap + 255) & ~size_t(255);
+  h->place_bytes = (sizeof(unsigned short) * (size_t)size * h->place_n + 255) & ~size_t(255);
+  return h->cap > 0;
+}
+
+// Its descriptor over `mem` (n_bytes + list_bytes + place_bytes).
+HaloRef halo_ref(const HaloShape& h, void* mem) {
+  HaloRef r{};
+  char* at = (char*)mem;
+  r.n = (const int*)at;
+  r.list = (const int*)(at + h.n_bytes);
+  r.place = (const unsigned short*)(at + h.n_bytes + h.list_bytes);
+  r.cap = h.cap;
+  r.place_n = h.place_n;
+  r.ok = 1;
+  return r;
+}
+
+// Fill the tables of `ref` (already at d_ref).
+int launch_halo(const fem_ctx* c, int k, int size, const HaloShape& h, const HaloRef& ref, HaloRef* d_ref,
+                hipStream_t st) {
+  hipLaunchKernelGGL(k_halo, dim3(size), dim3(kTeamBlock), 0, st, d_ref, c->n, c->d_rp, c->d_ci, h.rows, h.passes, k,
+                     const_cast<int*>(ref.n), const_cast<int*>(ref.list), const_cast<unsigned short*>(ref.place));
+  FEM_HIP(hipGetLastError());
+  return 0;
 }
 
 // S = coef[0] M + coef[1] K + coef[2] A (one value column) and its Jacobi
@@ -368,10 +548,10 @@ int form_system(fem_ctx* c, const double coef[3], int fp32, double* S64, void* S
 
 // Barrier slots, team sums, abort flag and the instances' outcome records
 // reset before a launch of the stepping kernel (a fill kernel).
-int launch_slot_reset(Slot* slots, int nslots, double* scal, int nteams, int* abort_flag, Inst* insts, int ninst,
+int launch_slot_reset(double* slots, int nrec, int rec_vals, int* abort_flag, Inst* insts, int ninst,
                       hipStream_t st) {
-  hipLaunchKernelGGL(k_reset, dim3(div_up(std::max(nteams + nslots, ninst), kBlock)), dim3(kBlock), 0, st, slots,
-                     nslots, scal, nteams, abort_flag, insts, ninst);
+  hipLaunchKernelGGL(k_reset, dim3(reset_grid(nrec, rec_vals, ninst)), dim3(kBlock), 0, st, slots, nrec, rec_vals,
+                     abort_flag, insts, ninst);
   FEM_HIP(hipGetLastError());
   return 0;
 }
@@ -412,7 +592,7 @@ int build_plan(fem_batch* b) {
   // coherent and fenced exchange; they differ in registers
   int maxv[3] = {0, 0, 0};
   int rc = 0;
-  for (int m = 0; m < 3 && !rc; m++) rc = step_max_coresident(k, inner_fp32, kr, m, &maxv[m]);
+  for (int m = 0; m < 3 && !rc; m++) rc = variant_coresident(k, inner_fp32, kr, m, &maxv[m]);
   if (rc) return rc;
   if (std::min(maxv[0], std::min(maxv[1], maxv[2])) <= 0) {
     set_error("persistent kernel cannot be resident on this device");
@@ -440,28 +620,33 @@ int build_plan(fem_batch* b) {
       }
     } else {
       const int budget = (b->grid_budget > 0) ? std::min(b->grid_budget, maxb) : maxb;
+      // Instances of at least one workgroup's share get teams of their own,
+      // one workgroup more at a time to the team with the most work per
+      // workgroup; the others share the workgroups their work amounts to.
       const double share = W / budget;
       std::vector<int> small;
-      int used = 0;
-      for (int i = 0; i < ninst; i++) {
-        int g = (int)std::floor(work[i] / share);
-        if (g >= 2) {
-          teams.push_back({i});
-          sizes.push_back(g);
-          used += g;
-        } else {
+      double wsmall = 0.0;
+      for (int i = 0; i < ninst; i++)
+        if (work[i] < share) {
           small.push_back(i);
+          wsmall += work[i];
+        } else {
+          teams.push_back({i});
+          sizes.push_back(1);
         }
+      const int big = (int)teams.size();
+      int bins = std::max(1, std::min((int)small.size(), std::max(1, std::min((int)std::lround(wsmall / share),
+                                                                            budget - big))));
+      int left = budget - big - (small.empty() ? 0 : bins);
+      using Load = std::pair<double, int>;  // work per workgroup, team
+      std::priority_queue<Load> heaviest;
+      for (int t = 0; t < big; t++) heaviest.push(Load(work[teams[t][0]], t));
+      for (; left > 0 && big > 0; left--) {
+        const int t = heaviest.top().second;
+        heaviest.pop();
+        sizes[t]++;
+        heaviest.push(Load(work[teams[t][0]] / sizes[t], t));
       }
-      if (used > budget) {  // rounding guard
-        double f = (double)budget / (used + (double)small.size());
-        used = 0;
-        for (auto& g : sizes) {
-          g = std::max(1, (int)(g * f));
-          used += g;
-        }
-      }
-      int bins = std::max(1, std::min((int)small.size(), std::max(1, budget - used)));
       std::sort(small.begin(), small.end(), [&](int x, int y) { return work[x] > work[y]; });
       std::vector<double> load(bins, 0.0);
       std::vector<std::vector<int>> lists(bins);
@@ -477,43 +662,24 @@ int build_plan(fem_batch* b) {
         }
     }
   };
-  // Exchange mode of a plan: a workgroup of a multi-workgroup team whose rows
-  // exceed two per lane (the LDS row cache) streams its phases: fenced
-  // barriers.  Plans of one-workgroup teams run the plain variant.
-  const int forced = (b->opts.exchange == FEM_EXCHANGE_COHERENT || b->opts.exchange == FEM_EXCHANGE_FENCED)
-                         ? b->opts.exchange : 0;
-  auto plan_mode = [&]() {
-    bool multi = false, streaming = false;
-    for (size_t t = 0; t < teams.size(); t++) {
-      if (sizes[t] <= 1) continue;
-      multi = true;
-      for (int i : teams[t])
-        if (team_streams(b->insts[i].ctx->n, k, sizes[t])) streaming = true;
-    }
-    return exchange_mode(multi, streaming, forced, b->mode_override);
-  };
   auto plan_grid = [&]() {
     int g = 0;
     for (int s_ : sizes) g += s_;
     return g;
   };
-  // Size for the coherent variant first; if the variant the plan then picks
-  // holds fewer workgroups, re-plan within the smallest limit of all three,
-  // which any mode fits.
-  make_plan(maxv[kExchangeCoherent]);
-  int mode = plan_mode();
-  if (plan_grid() > maxv[mode]) {
-    make_plan(std::min(maxv[0], std::min(maxv[1], maxv[2])));
-    mode = plan_mode();
+  auto any_multi = [&]() { return std::any_of(sizes.begin(), sizes.end(), [](int g) { return g > 1; }); };
+  // One-workgroup teams only: the plain variant (smaller workgroups, more of
+  // them); else within what both exchange modes hold.
+  make_plan(maxv[0]);
+  bool multi = any_multi();
+  if (multi) {
+    make_plan(std::min(maxv[kExchangeCoherent], maxv[kExchangeFenced]));
+    multi = any_multi();
   }
-  const int maxb = maxv[mode];
+  const int forced = (b->opts.exchange == FEM_EXCHANGE_COHERENT || b->opts.exchange == FEM_EXCHANGE_FENCED)
+                         ? b->opts.exchange : 0;
   const int nteams = (int)teams.size();
-  int grid = 0;
-  for (int g : sizes) grid += g;
-  if (grid > maxb) {
-    set_error("team plan exceeds the co-resident grid");
-    return FEM_ERR_INVALID;
-  }
+  const int grid = plan_grid();
   std::vector<Team> ht(nteams);
   std::vector<int> wg_team(grid), team_inst;
   int wg = 0;
@@ -529,21 +695,60 @@ int build_plan(fem_batch* b) {
   b->d_teams = dalloc<Team>(nteams, &rc);
   b->d_wg_team = dalloc<int>(grid, &rc);
   b->d_team_inst = dalloc<int>(team_inst.size(), &rc);
-  b->d_slots = dalloc<Slot>(grid, &rc);
-  b->d_scal = dalloc<double>((size_t)nteams * kSlotBufs * kMaxRed, &rc);
+  b->d_slots = dalloc<double>(slot_bytes(grid, k) / sizeof(double), &rc);
   if (rc) return rc;
-  int poff = 0;
+  // halos of the teams whose workgroups keep their rows in LDS
+  std::vector<HaloRef> halo(team_inst.size());
+  std::vector<HaloShape> shape(team_inst.size());
+  size_t halo_bytes = 0;
+  for (int t = 0; t < nteams; t++)
+    for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++)
+      if (halo_shape(b->insts[team_inst[q]].ctx, k, sizes[t], inner_fp32 ? 4 : 8, kr, &shape[q]))
+        halo_bytes += shape[q].n_bytes + shape[q].list_bytes + shape[q].place_bytes;
+      else
+        shape[q].cap = 0;
+  if (halo_bytes > 0) {
+    b->d_halo = dalloc<HaloRef>(halo.size(), &rc);
+    b->d_halo_mem = dalloc<char>(halo_bytes, &rc);
+    if (rc) return rc;
+    size_t at = 0;
+    for (size_t q = 0; q < halo.size(); q++) {
+      if (shape[q].cap == 0) continue;
+      halo[q] = halo_ref(shape[q], b->d_halo_mem + at);
+      at += shape[q].n_bytes + shape[q].list_bytes + shape[q].place_bytes;
+    }
+    const size_t bytes = sizeof(HaloRef) * halo.size();
+    FEM_HIP(hipMemcpyAsync(b->d_halo, halo.data(), bytes, hipMemcpyHostToDevice, b->stream));
+    for (int t = 0; t < nteams; t++)
+      for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++)
+        if (shape[q].cap > 0 &&
+            (rc = launch_halo(b->insts[team_inst[q]].ctx, k, sizes[t], shape[q], halo[q], b->d_halo + q, b->stream)))
+          return rc;
+    FEM_HIP(hipMemcpyAsync(halo.data(), b->d_halo, bytes, hipMemcpyDeviceToHost, b->stream));
+    FEM_HIP(hipStreamSynchronize(b->stream));
+  }
+  // Whether any instance keeps its rows in LDS (the kernel variant), and the
+  // exchange mode: teams of several workgroups with more rows than the row
+  // cache holds stream their phases: fenced barriers.  Plans of one-workgroup teams run the plain
+  // variant.
+  bool rows = false, streaming = false;
+  for (int t = 0; t < nteams; t++)
+    for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++) {
+      const bool fits = sizes[t] == 1 ? rows_fit(b->insts[team_inst[q]].ctx, k, 1, kr) : halo[q].ok != 0;
+      rows |= fits;
+      streaming |= sizes[t] > 1 && team_streams(b->insts[team_inst[q]].ctx->n, k, sizes[t]);
+    }
+  const int mode = exchange_mode(multi, streaming, forced, b->mode_override);
+  if (grid > maxv[mode]) {
+    set_error("team plan exceeds the co-resident grid");
+    return FEM_ERR_INVALID;
+  }
   for (int t = 0; t < nteams; t++) {
-    ht[t].slots = b->d_slots + poff;
-    ht[t].scal = b->d_scal + (size_t)t * kSlotBufs * kMaxRed;
+    ht[t].halo = b->d_halo;
+    team_slots(&ht[t], b->d_slots, grid, k);
     ht[t].abort_flag = b->d_abort;
     ht[t].wait_ticks = b->wait_ticks;
-    // every workgroup reading every partial costs size^2 * nvals loads per
-    // barrier; beyond ~16 KB per workgroup rank 0 reduces and publishes
-    ht[t].allpoll = b->poll_override == 1   ? 1
-                    : b->poll_override == 2 ? 0
-                                            : ((long long)sizes[t] * 3 * k <= 2048) ? 1 : 0;
-    poff += sizes[t];
+    ht[t].allpoll = b->poll_override == 1 ? 1 : b->poll_override == 2 ? 0 : flat_reduction(sizes[t], k);
   }
   std::vector<Inst> hi(ninst);
   for (int i = 0; i < ninst; i++) hi[i] = persistent_desc(b->insts[i].dev);
@@ -563,6 +768,7 @@ int build_plan(fem_batch* b) {
   b->launch.inner_fp32 = inner_fp32;
   b->launch.kr = kr;
   b->launch.coh = mode;
+  b->launch.rows = rows;
   b->nteams = nteams;
   b->grid = grid;
   b->team_sizes = sizes;
@@ -1042,6 +1248,12 @@ int batch_prepare(fem_batch* b, bool need_plan) {
       if (!rc && need_plan && !h.d_hvec) h.d_hvec = dalloc<double>((size_t)h.ctx->n * h.k, &rc);
       if (rc) return rc;
     }
+    // exchange words of the persistent plans
+    if (need_plan && !h.d_xch) {
+      int rc = 0;
+      h.d_xch = dalloc<unsigned long long>((size_t)h.ctx->n * h.k * xch_words((int)inner_bytes(b)), &rc);
+      if (rc) return rc;
+    }
     // Newmark on the streaming engine: each update forms the next step's
     // displacement predictor (Inst::hvec)
     if (h.eq == FEM_WAVE_NEWMARK && !need_plan && !h.d_hvec) {
@@ -1052,7 +1264,7 @@ int batch_prepare(fem_batch* b, bool need_plan) {
     if (h.dirty || h.formed_version != h.ctx->version) {
       int rc = form_inst(b, h);
       if (rc) return rc;
-      b->plan_ready = false;
+      b->plan_gen++;  // the plan stays (no value enters it), a recorded advance goes stale
     }
     fill_dev(b, h);
   }
@@ -1164,7 +1376,7 @@ int batch_plan_info(fem_batch* b, fem_plan_info* info) {
   int rc = batch_prepare(b, true);
   if (rc) return rc;
   int maxb = 0;
-  rc = step_max_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, b->launch.coh, &maxb);
+  rc = step_max_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, b->launch.coh, b->launch.rows, &maxb);
   if (rc) return rc;
   info->grid = b->grid;
   info->teams = b->nteams;
@@ -1184,9 +1396,9 @@ int batch_advance(fem_batch* b, int nsteps, fem_step_stats* stats) {
   int rc = batch_prepare(b, true);
   if (rc) return rc;
   const int ninst = (int)b->insts.size();
-  hipLaunchKernelGGL(k_reset, dim3(div_up(std::max(b->nteams + b->grid, ninst), kBlock)), dim3(kBlock), 0,
-                     b->stream, b->d_slots, b->grid, b->d_scal, b->nteams, b->d_abort, b->d_insts, ninst);
-  FEM_HIP(hipGetLastError());
+  rc = launch_slot_reset(b->d_slots, b->grid, slot_vals(b->launch.k), b->d_abort, b->d_insts, ninst,
+                         b->stream);
+  if (rc) return rc;
   FEM_HIP(hipEventRecord(b->ev0, b->stream));
   if (nsteps > 0) {
     rc = launch_step(b->launch, nsteps, b->stream);
@@ -1236,16 +1448,14 @@ int batch_graph_capture(fem_batch* b, int nsteps) {
   hipGraph_t g = nullptr;
   FEM_HIP(hipGraphCreate(&g, 0));
   int ninst = (int)b->insts.size();
-  Slot* slots = b->d_slots;
-  int nslots = b->grid, nteams = b->nteams;
-  double* scal = b->d_scal;
+  double* slots = b->d_slots;
+  int nslots = b->grid, rec_vals = slot_vals(b->launch.k);
   int* abort_flag = b->d_abort;
   Inst* insts = b->d_insts;
-  void* rargs[] = {(void*)&slots, (void*)&nslots, (void*)&scal, (void*)&nteams, (void*)&abort_flag, (void*)&insts,
-                   (void*)&ninst};
+  void* rargs[] = {(void*)&slots, (void*)&nslots, (void*)&rec_vals, (void*)&abort_flag, (void*)&insts, (void*)&ninst};
   hipKernelNodeParams prm{};
   prm.func = (void*)k_reset;
-  prm.gridDim = dim3(div_up(std::max(b->nteams + b->grid, ninst), kBlock));
+  prm.gridDim = dim3(reset_grid(nslots, rec_vals, ninst));
   prm.blockDim = dim3(kBlock);
   prm.sharedMemBytes = 0;
   prm.kernelParams = rargs;
@@ -1486,7 +1696,7 @@ int batch_autotune(fem_batch* b, int probe, int* chosen, double* best_ms) {
   int rc = batch_prepare(b, true);
   if (rc) return rc;
   int maxb = 0;
-  rc = step_max_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, 1, &maxb);
+  rc = variant_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, kExchangeCoherent, &maxb);
   if (rc) return rc;
   const bool single = b->insts.size() == 1;
   // Rows x columns per lane of the whole co-resident grid: beyond ~64 every
@@ -1495,7 +1705,7 @@ int batch_autotune(fem_batch* b, int probe, int* chosen, double* best_ms) {
   // such batches only try the streaming engine.
   double lanes_work = 0.0;
   for (auto& h : b->insts) lanes_work += (double)h.ctx->n * h.k;
-  const bool persistent_hopeless = lanes_work > 64.0 * maxb * kBlock;
+  const bool persistent_hopeless = lanes_work > 64.0 * maxb * kTeamBlock;
   std::vector<int> cands;
   if (persistent_hopeless) {
     // no persistent candidates
@@ -1555,7 +1765,7 @@ int batch_autotune(fem_batch* b, int probe, int* chosen, double* best_ms) {
     for (int c : cands) {
       for (int m : {kExchangeCoherent, kExchangeFenced}) {
         if (b->opts.exchange != FEM_EXCHANGE_AUTO && m != kExchangeCoherent) continue;  // mode fixed by opts
-        // one instance: both barrier reductions (all workgroups sum, or rank 0 publishes)
+        // one instance: both barrier reductions (flat, or in two levels)
         for (int pl : {1, 2}) {
           if (!single && pl == 2) continue;
           if (single) b->opts.team_size = c;

@@ -14,6 +14,7 @@
 namespace femhip {
 
 constexpr int kBlock = 256;          // threads per workgroup (4 wave64)
+constexpr int kTeamBlock = 512;      // threads per workgroup of the stepping kernel's multi-workgroup variants
 constexpr int kWave = 64;
 constexpr int kMaxK = 16;            // right-hand sides per instance
 constexpr int kMaxSlots = 4;         // reduction slots per phase
@@ -56,16 +57,18 @@ enum : int {
   ST_BARRIER_TIMEOUT = 8,
 };
 
-// Per-workgroup barrier slot: the partial sums of the last four barriers.
+// Per-workgroup barrier records: the partial sums of the last four barriers.
 // Barrier e writes buffer e & 3, and the lowest mantissa bit of every value
 // carries the tag (e >> 2) & 1, so a reader recognises this barrier's values
-// without a separate flag.  Arrivals go to the workgroup's own slot and never
-// contend on one address.
+// without a separate flag.  Arrivals go to the workgroup's own record and
+// never contend on one address.  A record holds slot_vals(k) doubles, at
+// least one 128-byte line, and the records of one buffer are adjacent: every
+// workgroup polls all of them, and 512 bytes apart (the four buffers of a
+// workgroup together) a barrier of 128 workgroups took 0.4 us longer.
 constexpr int kSlotBufs = 4;
-struct alignas(128) Slot {
-  double vals[kSlotBufs][kMaxRed];
-};
-
+__host__ __device__ constexpr int slot_vals(int k) { return 4 * k < 16 ? 16 : 4 * k; }
+// Ranks per group of a two-level reduction.
+constexpr int kGroup = 16;
 
 // Device-side description of one instance (a mesh, its parameters and its
 // state) advanced by one team of workgroups inside the persistent kernel.
@@ -125,20 +128,58 @@ struct Inst {
   double* hvec;          // [n][k] history part of the next initial guess, formed with the update:
                          //   phase_res gathers it instead of the history levels; Newmark on the
                          //   streaming engine: the next u + dt v + (1/2 - beta) dt^2 a
+  unsigned long long* xch;  // exchange words between the workgroups of a team (xch_words per value; null:
+                         //   the teams read their neighbours from memory)
   double* h5;            // [n][k] x_{n-5}, x_{n-6} (quintic and sextic predictors, streaming engine)
   double* h6;
 };
+
+// Rows that a workgroup of the stepping kernel keeps in LDS for the launch
+// (step_kernel.h): at most kCacheP per lane and kCacheE entries each.
+constexpr int kCacheE = 10, kCacheP = 2;
+// LDS of a workgroup's entries (a weight of ti bytes and a 16-bit place each)
+// over `passes` rows per lane of `block` lanes, and the pool they share with
+// the staging area and the halo's list.  One-workgroup teams (kBlock) have no
+// halo: the staging area holds the own rows.  Multi-workgroup variants run one
+// workgroup per CU and take most of its 160 KB.
+__host__ __device__ constexpr int rows_cells_bytes(int passes, int block, int ti) {
+  return (passes * kCacheE * block * (ti + 2) + 15) & ~15;
+}
+__host__ __device__ constexpr int rows_pool_bytes(int block, int ti) {
+  return rows_cells_bytes(kCacheP, block, ti) + 16 * kCacheP * block;
+}
+constexpr int kTeamPool = 145 * 1024;
+
+// The halos of one team-instance (k_halo): per rank the rows of other
+// workgroups that its rows read, ascending, and per lane and entry the place
+// of the value in the workgroup's staging area (own rows first, then the
+// halo's, in rows).
+struct HaloRef {
+  const int* n;                   // [team size]
+  const int* list;                // [team size][cap]
+  const unsigned short* place;    // [team size][place_n]
+  int cap, place_n;
+  int ok;                         // every rank's halo fits
+  int max_n;                      // the longest
+};
+
+// Words per value of Inst::xch: two buffers of an inner-precision product (or
+// two products) and one of an FP64 candidate, 4 bytes of value each.
+__host__ __device__ constexpr int xch_words(int ti) { return 2 * (ti / 4) + 2; }
 
 // A team: a contiguous range of workgroups that advances a list of instances
 // one after the other, synchronising through its own barrier.
 struct Team {
   int first_wg, size;
   int inst_begin, inst_end;  // range in the team-instance list
-  int allpoll;               // 1: every workgroup polls all slots and reduces;
-                             // 0: rank 0 reduces and releases through gen
+  int allpoll;               // 1: every workgroup polls and sums all records;
+                             // 0: in two levels, by groups of kGroup ranks
   int pad_;
-  Slot* slots;               // [size]
-  double* scal;             // [kSlotBufs][kMaxRed] tagged sums published by rank 0
+  double* slots;             // the team's first record of buffer 0
+  int rec_vals;              // doubles per record (slot_vals)
+  int buf_records;           // records per buffer (workgroups of the launch)
+  double* groups;            // the team's first group record of buffer 0 (as slots)
+  const HaloRef* halo;       // by position in the team-instance list (null: no halos)
   int* abort_flag;
   long long wait_ticks;      // longest barrier wait (wall_clock64 ticks, 100 MHz) before the launch
                              // aborts; 0: abort at the first wait not already satisfied

@@ -16,6 +16,7 @@ struct StepLaunch {
   int inner_fp32 = 1;
   int kr = 0;   // Krylov method: 0 pipelined CG, 1 BiCGSTAB, 2 classic CG
   int coh = 1;  // exchange mode: 0 one-workgroup teams only, 1 coherent, 2 fenced
+  int rows = 0; // the variant that keeps instances' rows in LDS where they fit
 };
 
 // Exchange mode for teams spanning several workgroups: coherent accesses
@@ -27,10 +28,25 @@ int launch_step(const StepLaunch& L, int nsteps, hipStream_t st);
 
 // Plan rules shared by the batch plans and the allocation-free solve (batch.hip).
 int single_team_size(long long n, int k, int team_size, int maxb);
+int flat_reduction(int size, int k);
+size_t slot_bytes(int grid, int k);
+void team_slots(Team* T, double* slots, int grid, int k);
 bool team_streams(long long n, int k, int size);
+bool rows_fit(const fem_ctx* c, int k, int size, int kr);
+int variant_coresident(int k, int inner_fp32, int kr, int coh, int* blocks);
 int exchange_mode(bool multi, bool streaming, int forced, int tuned);
-int launch_slot_reset(Slot* slots, int nslots, double* scal, int nteams, int* abort_flag, Inst* insts, int ninst,
+int launch_slot_reset(double* slots, int nrec, int rec_vals, int* abort_flag, Inst* insts, int ninst,
                       hipStream_t st);
+
+// Halos of the teams whose workgroups keep their rows in LDS (batch.hip).
+struct HaloShape {
+  int rows = 0, passes = 0, cap = 0, place_n = 0;  // rows per workgroup, rows per lane, halo rows that fit
+  size_t n_bytes = 0, list_bytes = 0, place_bytes = 0;
+};
+bool halo_shape(const fem_ctx* c, int k, int size, int ti, int kr, HaloShape* h);
+HaloRef halo_ref(const HaloShape& h, void* mem);
+int launch_halo(const fem_ctx* c, int k, int size, const HaloShape& h, const HaloRef& ref, HaloRef* d_ref,
+                hipStream_t st);
 
 // Streaming engine (stream.hip): row-block table and per-instance scalars.
 struct StreamPlan;
@@ -62,7 +78,7 @@ int stream_run(const StreamPlan* p, const Inst* d_insts, int max_sweeps, int max
 // Column counts whose stream phases use the multi-column layout with the
 // staged pattern (one value column, Inst::SDi present).
 bool stream_vec_layout(int k);
-int step_max_coresident(int k, int inner_fp32, int kr, int coh, int* blocks);
+int step_max_coresident(int k, int inner_fp32, int kr, int coh, int rows, int* blocks);
 int step_graph_node(const StepLaunch& L, int nsteps, hipGraph_t g, hipGraphNode_t dep, hipGraphNode_t* out);
 
 // Per-instance host bookkeeping.
@@ -86,6 +102,7 @@ struct InstHost {
   double* d_xnext = nullptr; // Inst::xnext, Inst::hpre
   double* d_hpre = nullptr;
   double* d_hvec = nullptr;  // Inst::hvec
+  unsigned long long* d_xch = nullptr;  // Inst::xch
   double* d_S64 = nullptr;
   void* d_Si = nullptr;
   double* d_dinv64 = nullptr;
@@ -130,8 +147,9 @@ struct fem_batch {
   femhip::Team* d_teams = nullptr;
   int* d_wg_team = nullptr;
   int* d_team_inst = nullptr;
-  femhip::Slot* d_slots = nullptr;
-  double* d_scal = nullptr;
+  double* d_slots = nullptr;    // barrier records of the workgroups, then of the groups: 2 x [kSlotBufs][grid][slot_vals]
+  femhip::HaloRef* d_halo = nullptr;  // by position in the team-instance list; tables in d_halo_mem
+  char* d_halo_mem = nullptr;
   int grid = 0;
   int* d_abort = nullptr;       // in the info block
   char* d_info = nullptr;       // [ninst][kInfoBytes] + abort flag
@@ -142,8 +160,8 @@ struct fem_batch {
   long long wait_ticks = femhip::kDefaultWaitTicks;  // longest barrier wait of the persistent kernel
   int grid_budget = 0;          // multi-instance plans: workgroups to spread over (0 = all co-resident)
   int mode_override = 0;        // exchange mode forced by the autotuner (0 = by the row-cache rule)
-  int poll_override = 0;        // barrier reduction forced by the autotuner: 1 every workgroup sums all
-                                // partials, 2 rank 0 sums and publishes (0 = by the traffic rule)
+  int poll_override = 0;        // barrier reduction forced by the autotuner: 1 flat, 2 in two levels
+                                // (0 = by flat_reduction)
   std::vector<int> team_sizes;  // for reporting
   // plain-engine scratch
   double* d_plain = nullptr;

@@ -30,8 +30,8 @@ static __device__ __align__(256) unsigned char scratch[size_t(32) << 20];
 namespace {
 
 // Largest footprint a call may lay out: 32 MiB per GPU.  One right-hand side
-// of an FP32 + refinement solve uses about 12 nnz + 80 N bytes plus 2 KiB
-// per workgroup of barrier slots, so meshes up to roughly 180,000 unknowns
+// of an FP32 + refinement solve uses about 12 nnz + 80 N bytes plus 0.5 KiB
+// per workgroup of barrier records, so meshes up to roughly 180,000 unknowns
 // fit at one column (about 25,000 at sixteen).
 constexpr size_t kScratchBytes = size_t(32) << 20;
 
@@ -76,13 +76,14 @@ struct Layout {
 // Writes the launch descriptors of the one-team plan and zeroes the buffer
 // the update phase reads as the previous state (a fill kernel: no memset, so
 // the sequence stays capturable).
-__global__ void k_noalloc_setup(Team team, Inst inst, int grid, Team* d_team, int* d_wg_team, int* d_team_inst,
-                                Inst* d_inst, double* zero, long long nzero) {
+__global__ void k_noalloc_setup(Team team, Inst inst, HaloRef halo, int grid, Team* d_team, int* d_wg_team,
+                                int* d_team_inst, Inst* d_inst, HaloRef* d_halo, double* zero, long long nzero) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     *d_team = team;
     *d_inst = inst;
     *d_team_inst = 0;
+    if (team.halo) *d_halo = halo;
   }
   if (i < grid) d_wg_team[i] = 0;
   for (long long q = i; q < nzero; q += (long long)gridDim.x * blockDim.x) zero[q] = 0.0;
@@ -120,7 +121,7 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   // plan: one team, sized and moded as a one-instance batch plan
   int maxv[3] = {0, 0, 0};
   for (int m = 0; m < 3; m++) {
-    const int rc = step_max_coresident(k, fp32, kri, m, &maxv[m]);
+    const int rc = variant_coresident(k, fp32, kri, m, &maxv[m]);
     if (rc) return rc;
   }
   const int forced = (o.exchange == FEM_EXCHANGE_COHERENT || o.exchange == FEM_EXCHANGE_FENCED) ? o.exchange : 0;
@@ -137,8 +138,7 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
 
   // footprint
   Layout L;
-  const size_t o_slots = L.take(sizeof(Slot) * (size_t)grid);
-  const size_t o_scal = L.take(sizeof(double) * kSlotBufs * kMaxRed);
+  const size_t o_slots = L.take(slot_bytes(grid, k));
   const size_t o_team = L.take(sizeof(Team));
   const size_t o_wgt = L.take(sizeof(int) * (size_t)grid);
   const size_t o_ti = L.take(sizeof(int));
@@ -152,6 +152,19 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   const size_t o_x = L.take(sizeof(double) * (size_t)n * k);
   const size_t o_b = L.take(sizeof(double) * (size_t)n * k);
   const size_t o_vec = L.take(tb * (size_t)n * k * 11);
+  // the halo tables, where the scratch array still has room for them (without
+  // them the workgroups read their neighbours' rows from memory)
+  HaloShape hs;
+  bool halos = halo_shape(c, k, grid, (int)tb, kri, &hs);
+  size_t o_halo = 0, o_halo_mem = 0, o_xch = 0;
+  if (halos) {
+    Layout H = L;
+    o_halo = H.take(sizeof(HaloRef));
+    o_halo_mem = H.take(hs.n_bytes + hs.list_bytes + hs.place_bytes);
+    o_xch = H.take(8 * (size_t)xch_words((int)tb) * (size_t)n * k);
+    halos = H.used <= kScratchBytes;
+    if (halos) L = H;
+  }
   static_assert(sizeof(scratch) == kScratchBytes, "scratch size");
   if (L.used > kScratchBytes) {
     set_error("fem_ctx_solve_noalloc: this system needs " + std::to_string(L.used) + " bytes of scratch, more than the " +
@@ -162,8 +175,7 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   int rc = scratch_ptr(&base);
   if (rc) return rc;
 
-  Slot* slots = (Slot*)(base + o_slots);
-  double* scal = (double*)(base + o_scal);
+  double* slots = (double*)(base + o_slots);
   Team* d_team = (Team*)(base + o_team);
   int* d_wg_team = (int*)(base + o_wgt);
   int* d_team_inst = (int*)(base + o_ti);
@@ -215,6 +227,7 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   I.status = (int*)(info + kInfoStatus);
   I.last_res = (double*)(info + kInfoLastRes);
   I.traj_every = 1;
+  if (halos) I.xch = (unsigned long long*)(base + o_xch);
 
   Team T;
   std::memset(&T, 0, sizeof(T));
@@ -222,10 +235,12 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   T.size = grid;
   T.inst_begin = 0;
   T.inst_end = 1;
-  T.allpoll = ((long long)grid * 3 * k <= 2048) ? 1 : 0;
-  T.slots = slots;
-  T.scal = scal;
+  T.allpoll = flat_reduction(grid, k);
+  team_slots(&T, slots, grid, k);
   T.abort_flag = abort_flag;
+  HaloRef* d_halo = (HaloRef*)(base + o_halo);
+  const HaloRef halo = halos ? halo_ref(hs, base + o_halo_mem) : HaloRef{};
+  if (halos) T.halo = d_halo;
   T.wait_ticks = kDefaultWaitTicks;
 
   hipStream_t st = c->stream;
@@ -236,11 +251,15 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   const long long nzero = n * k;
   hipLaunchKernelGGL(k_noalloc_setup, dim3(div_up(std::max<long long>(grid, std::min<long long>(nzero, 1 << 20)),
                                                   kBlock)),
-                     dim3(kBlock), 0, st, T, I, grid, d_team, d_wg_team, d_team_inst, d_inst, I.u, nzero);
+                     dim3(kBlock), 0, st, T, I, halo, grid, d_team, d_wg_team, d_team_inst, d_inst, d_halo, I.u, nzero);
   FEM_HIP(hipGetLastError());
+  if (halos) {
+    rc = launch_halo(c, k, grid, hs, halo, d_halo, st);
+    if (rc) return rc;
+  }
   rc = form_system(c, coef, fp32, (double*)I.S64, (void*)I.Si, (double*)I.dinv64, (void*)I.dinvi, st);
   if (rc) return rc;
-  rc = launch_slot_reset(slots, grid, scal, 1, abort_flag, d_inst, 1, st);
+  rc = launch_slot_reset(slots, grid, slot_vals(k), abort_flag, d_inst, 1, st);
   if (rc) return rc;
   StepLaunch SL;
   SL.teams = d_team;
@@ -252,6 +271,7 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   SL.inner_fp32 = fp32;
   SL.kr = kri;
   SL.coh = mode;
+  SL.rows = grid == 1 ? rows_fit(c, k, 1, kri) : halos;
   rc = launch_step(SL, 1, st);
   if (rc) return rc;
   alignas(8) char rec[kInfoBytes + sizeof(int)];

@@ -11,22 +11,29 @@ namespace femhip {
 const void* step_kernel_plain(int k, int fp32, int kr);
 const void* step_kernel_coherent(int k, int fp32, int kr);
 const void* step_kernel_fenced(int k, int fp32, int kr);
+const void* step_kernel_plain_rows(int k, int fp32, int kr);
+const void* step_kernel_coherent_rows(int k, int fp32, int kr);
+const void* step_kernel_fenced_rows(int k, int fp32, int kr);
 
 namespace {
 
-// Kernel instantiation for (columns, inner precision, Krylov method, exchange mode).
-const void* pick_kernel(int k, int fp32, int kr, int coh) {
+// Kernel instantiation for (columns, inner precision, Krylov method, exchange
+// mode, rows in LDS).
+const void* pick_kernel(int k, int fp32, int kr, int coh, int rows) {
   switch (coh) {
-    case 0: return step_kernel_plain(k, fp32, kr);
-    case kExchangeCoherent: return step_kernel_coherent(k, fp32, kr);
-    case kExchangeFenced: return step_kernel_fenced(k, fp32, kr);
+    case 0: return rows ? step_kernel_plain_rows(k, fp32, kr) : step_kernel_plain(k, fp32, kr);
+    case kExchangeCoherent: return rows ? step_kernel_coherent_rows(k, fp32, kr) : step_kernel_coherent(k, fp32, kr);
+    case kExchangeFenced: return rows ? step_kernel_fenced_rows(k, fp32, kr) : step_kernel_fenced(k, fp32, kr);
     default: return nullptr;
   }
 }
 
-// Workgroups of kernel `fn` that fit the current device at once.  Cached per
+// Threads per workgroup of the variants of one exchange mode.
+int team_block(int coh) { return coh == 0 ? kBlock : kTeamBlock; }
+
+// Workgroups of kernel `fn` (of `block` threads) that fit the current device at once.  Cached per
 // (device, kernel): the answer depends only on the code object.
-int kernel_max_coresident(const void* fn, int* blocks) {
+int kernel_max_coresident(const void* fn, int block, int* blocks) {
   constexpr int kMaxDev = 16, kMaxFn = 128;
   struct Entry { const void* fn; int blocks; };
   static std::mutex mu;
@@ -44,7 +51,7 @@ int kernel_max_coresident(const void* fn, int* blocks) {
   }
   int per_cu = 0, cus = 0;
   FEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  FEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0));
+  FEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, block, 0));
   *blocks = per_cu * cus;
   if (dev >= 0 && dev < kMaxDev) {
     std::lock_guard<std::mutex> lk(mu);
@@ -57,7 +64,7 @@ int kernel_max_coresident(const void* fn, int* blocks) {
 // resident at once: refuse a grid the launched variant cannot hold.
 int check_resident(const StepLaunch& L, const void* fn) {
   int maxb = 0;
-  const int rc = kernel_max_coresident(fn, &maxb);
+  const int rc = kernel_max_coresident(fn, team_block(L.coh), &maxb);
   if (rc) return rc;
   if (L.grid > maxb) {
     set_error("stepping kernel: grid of " + std::to_string(L.grid) + " workgroups exceeds the " +
@@ -72,14 +79,14 @@ int check_resident(const StepLaunch& L, const void* fn) {
 // Launch one persistent cooperative grid for a prepared batch.
 int launch_step(const StepLaunch& L, int nsteps, hipStream_t st) {
   void* args[] = {(void*)&L.teams, (void*)&L.wg_team, (void*)&L.insts, (void*)&L.team_inst, (void*)&nsteps};
-  const void* fn = pick_kernel(L.k, L.inner_fp32, L.kr, L.coh);
+  const void* fn = pick_kernel(L.k, L.inner_fp32, L.kr, L.coh, L.rows);
   if (!fn) {
     set_error("unsupported kernel configuration (number of right-hand sides must be 1, 2, 4 or 16)");
     return FEM_ERR_INVALID;
   }
   const int rc = check_resident(L, fn);
   if (rc) return rc;
-  hipError_t e = hipLaunchCooperativeKernel(fn, dim3(L.grid), dim3(kBlock), args, 0, st);
+  hipError_t e = hipLaunchCooperativeKernel(fn, dim3(L.grid), dim3(team_block(L.coh)), args, 0, st);
   if (e != hipSuccess) return hip_fail(e, "hipLaunchCooperativeKernel(k_step)");
   return 0;
 }
@@ -89,7 +96,7 @@ int launch_step(const StepLaunch& L, int nsteps, hipStream_t st) {
 // cooperative launch checks is checked here against the same limit
 // (check_resident); every barrier wait of the kernel is also bounded.
 int step_graph_node(const StepLaunch& L, int nsteps, hipGraph_t g, hipGraphNode_t dep, hipGraphNode_t* out) {
-  const void* fn = pick_kernel(L.k, L.inner_fp32, L.kr, L.coh);
+  const void* fn = pick_kernel(L.k, L.inner_fp32, L.kr, L.coh, L.rows);
   if (!fn) {
     set_error("unsupported kernel configuration (number of right-hand sides must be 1, 2, 4 or 16)");
     return FEM_ERR_INVALID;
@@ -100,7 +107,7 @@ int step_graph_node(const StepLaunch& L, int nsteps, hipGraph_t g, hipGraphNode_
   hipKernelNodeParams prm{};
   prm.func = const_cast<void*>(fn);
   prm.gridDim = dim3(L.grid);
-  prm.blockDim = dim3(kBlock);
+  prm.blockDim = dim3(team_block(L.coh));
   prm.sharedMemBytes = 0;
   prm.kernelParams = args;
   prm.extra = nullptr;
@@ -109,13 +116,13 @@ int step_graph_node(const StepLaunch& L, int nsteps, hipGraph_t g, hipGraphNode_
 }
 
 // coh: 0 plain (one-workgroup teams), 1 coherent, 2 fenced.
-int step_max_coresident(int k, int inner_fp32, int kr, int coh, int* blocks) {
-  const void* fn = pick_kernel(k, inner_fp32, kr, coh);
+int step_max_coresident(int k, int inner_fp32, int kr, int coh, int rows, int* blocks) {
+  const void* fn = pick_kernel(k, inner_fp32, kr, coh, rows);
   if (!fn) {
     set_error("unsupported kernel configuration (number of right-hand sides must be 1, 2, 4 or 16)");
     return FEM_ERR_INVALID;
   }
-  return kernel_max_coresident(fn, blocks);
+  return kernel_max_coresident(fn, team_block(coh), blocks);
 }
 
 }  // namespace femhip

@@ -134,7 +134,6 @@ struct VLay {
 // S_ij D^-1_jj (classic CG's phase A: S_ij).  The Krylov gathers then read
 // only the vectors from global memory: one dependent memory level instead of
 // three (row pointer -> column index -> vector).
-#define LA __attribute__((address_space(3)))
 template <typename TI>
 struct Stage {
   const int LA* rp;  // [rows + 1]
@@ -650,9 +649,7 @@ __device__ inline void vblock_partials(const vec<double, V>* acc, Shared& sh) {
   for (int q = 0; q < NS; q++)
 #pragma unroll
     for (int v = 0; v < V; v++) {
-      double x = acc[q][v];
-#pragma unroll
-      for (int m = kWave / 2; m >= G; m >>= 1) x += __shfl_xor(x, m, kWave);
+      const double x = wave_sum<G>(acc[q][v]);
       if (lane < G) sh.wred[wave][q * K + lane * V + v] = x;
     }
   __syncthreads();

@@ -20,8 +20,8 @@ CSRC = os.path.join(PKG, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 OUT = os.path.join(HERE, "libfemhip.so")
 
-SOURCES = ["api.hip", "scan.hip", "ctx.hip", "batch.hip", "step.hip", "step_plain.hip", "step_coherent.hip",
-           "step_fenced.hip", "stream.hip", "plain.hip", "adjoint.hip", "operator.hip", "gl_compat.hip", "noalloc.hip", "surface.cpp"]
+SOURCES = ["step_coherent_rows.hip", "step_fenced_rows.hip", "step_plain_rows.hip", "stream.hip", "step_coherent.hip",
+           "step_fenced.hip", "step_plain.hip", "api.hip", "scan.hip", "ctx.hip", "batch.hip", "step.hip", "plain.hip", "adjoint.hip", "operator.hip", "gl_compat.hip", "noalloc.hip", "surface.cpp"]
 
 # -packed-fp32-ops: keep v_pk_*_f32 out of every code object.
 HIPCC_FLAGS = [
