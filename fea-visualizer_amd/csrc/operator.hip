@@ -15,6 +15,7 @@
 #include "femhip_ctx.h"
 
 #include <algorithm>
+#include <cstdint>
 
 namespace femhip {
 
@@ -74,7 +75,27 @@ __global__ void __launch_bounds__(kBlock) k_spmv(int n, const int* __restrict__ 
 // the LDS capacity (rows averaging more than kCapRow entries) reads its rows
 // from global memory instead.  NT marks the stream loads non-temporal, so the
 // single-use matrix bytes do not displace x from the caches.
+//
+// Bound by HBM for one column and by the gathers of x (7 segments of 64 or
+// 128 bytes a row) for 16.  Workgroups are dealt round-robin to the 8 XCDs,
+// so in launch order every x line is read by the XCDs of its own block and of
+// the blocks one lattice row away.  Groups of 8 kDeal blocks are therefore
+// dealt so that an XCD takes kDeal consecutive blocks: its L2 then holds both
+// lattice neighbours of most rows, while the XCDs still stream one short
+// stretch of memory together (one contiguous eighth of the matrix per XCD lost
+// 3 to 7 points of roofline).  16 columns, 700 x 700 nodes, FP64: 61 us a
+// product in launch order, 56 with kDeal 64 (32 to 250: 56 to 57); 600 x 600
+// FP32 34 -> 31; one column unchanged within 1%.
 constexpr int kCapRow = 10;
+constexpr int kDeal = 64;
+
+// The row block of this workgroup; the blocks past the last whole group stay
+// in launch order.
+__device__ inline int dealt_block() {
+  const int b = (int)blockIdx.x, g = 8 * kDeal;
+  const int first = b / g * g, w = b - first;
+  return first + g <= (int)gridDim.x ? first + (w & 7) * kDeal + (w >> 3) : b;
+}
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -103,7 +124,7 @@ __global__ void __launch_bounds__(kBlock) k_spmv_stream(int n, long long nnz, co
   typedef T vec __attribute__((ext_vector_type(V)));
   __shared__ int s_ci[CAP];
   __shared__ T s_val[CAP];
-  const int row0 = blockIdx.x * R;
+  const int row0 = dealt_block() * R;
   const int row1 = min(n, row0 + R);
   const int row = row0 + (int)threadIdx.x / LPR;
   const int c = ((int)threadIdx.x % LPR) * V;
@@ -356,7 +377,19 @@ int stream_rows(int k) {
   }
 }
 
-int default_lanes(int k) { return k >= 16 ? 16 : FEM_SPMV_STREAM_NT; }
+// Schedule of a column count that was neither tuned nor set: the row-block
+// stream with non-temporal matrix loads.  16 lanes per row with 16 columns is
+// one column per lane, 4 bytes a gather where the stream has 16: 1000 x 1100
+// nodes, FP32, 120 us a product against 61; 700 x 700 FP64 116 against 56;
+// 64 x 64 FP32 3.3 against 2.7.  It takes x and y at any alignment of their
+// type, and keeps those that the stream's 16-byte accesses cannot.  Below 256
+// x 256 nodes and one column 4 lanes per row take 2.2 us against 2.8, both
+// under the launch's own cost; the other stream variants lie within 10% of
+// this one either way.
+int default_schedule(int k, const void* x, const void* y) {
+  if (k >= 16 && (((uintptr_t)x | (uintptr_t)y) & 15)) return 16;
+  return FEM_SPMV_STREAM_NT;
+}
 
 template <typename T>
 int pipe_grid_k(int k, bool nt, int nblk, int* grid) {
@@ -468,7 +501,7 @@ int operator_apply_device(fem_operator* op, int k, const void* x, void* y) {
     set_error("operator: nrhs must be 1, 2, 4 or 16");
     return FEM_ERR_INVALID;
   }
-  const int g = op->lanes[k] ? op->lanes[k] : default_lanes(k);
+  const int g = op->lanes[k] ? op->lanes[k] : default_schedule(k, x, y);
   return launch(op, k, g, x, y);
 }
 
@@ -535,7 +568,7 @@ int operator_time(fem_operator* op, int k, const void* x, void* y, int reps, dou
     set_error("operator_time: nrhs must be 1, 2, 4 or 16 and reps >= 1");
     return FEM_ERR_INVALID;
   }
-  const int g = op->lanes[k] ? op->lanes[k] : default_lanes(k);
+  const int g = op->lanes[k] ? op->lanes[k] : default_schedule(k, x, y);
   return time_lanes(op, k, g, x, y, reps, ms);
 }
 
@@ -554,7 +587,7 @@ int operator_autotune(fem_operator* op, int k, const void* x, void* y, int reps,
     return FEM_ERR_INVALID;
   }
   double best = 1e300;
-  int bg = default_lanes(k);
+  int bg = default_schedule(k, x, y);
   for (int g : {1, 2, 4, 8, 16, (int)FEM_SPMV_STREAM, (int)FEM_SPMV_STREAM_NT, (int)FEM_SPMV_PIPE,
                 (int)FEM_SPMV_PIPE_NT}) {
     if (g < k) continue;

@@ -84,6 +84,48 @@ def test_operator_pipe_many_blocks_per_workgroup(gpu, precision):
     op.close()
 
 
+@pytest.mark.parametrize("precision", [_lib.FEM_PREC_FP64, _lib.FEM_PREC_FP32_IR])
+@pytest.mark.parametrize("cells", [5, 128, 129, 130, 182, 183, 364])
+def test_operator_default_schedule(gpu, precision, cells):
+    """The schedule of an operator that was not tuned, at sizes below, at and
+    past one group of 512 row blocks ((cells - 1)^2 rows; 32 rows a block at 16
+    FP64 columns, 64 at 16 FP32, 256 at one column), with a ragged rest, and
+    with 16 columns at an address that is aligned to the value type alone.
+    Against the context's own matrices: an entry is three rounded terms, two
+    sums and one conversion, and a row of m entries rounds each product and
+    sum once, so |y - ref| <= (m + 6) u (W |x|) with u the unit roundoff and W
+    the sum of the terms' magnitudes."""
+    import scipy.sparse as sp
+    import torch
+    m = meshes.jittered_square(cells, seed=6)
+    print("case operator default", precision, cells, flush=True)
+    ctx = FEMContext(m, 0)
+    coef = (1.0 / 2e-3, 1.0, -1.0)
+    rp, ci = ctx.pattern()
+    M, K, A = (sp.csr_matrix((ctx.matrix(w), ci, rp), shape=(len(rp) - 1, len(rp) - 1))
+               for w in (_lib.FEM_MATRIX_M, _lib.FEM_MATRIX_K, _lib.FEM_MATRIX_A))
+    n = M.shape[0]
+    S = coef[0] * M + coef[1] * K + coef[2] * A
+    W = abs(coef[0] * M) + abs(coef[1] * K) + abs(coef[2] * A)
+    dt = torch.float64 if precision == _lib.FEM_PREC_FP64 else torch.float32
+    u = torch.finfo(dt).eps / 2
+    bound = (np.diff(rp).max() + 6) * u
+    rng = np.random.Generator(np.random.PCG64(13))
+    for k in (1, 4, 16):
+        op = Operator(ctx, coef, precision)
+        for shift in ((0, 1) if k == 16 else (0,)):
+            buf = torch.zeros(2, n * k + 4, dtype=dt, device="cuda")
+            xd, yd = buf[0, shift:shift + n * k], buf[1, shift:shift + n * k]
+            xd.copy_(torch.from_numpy(rng.standard_normal(n * k)))
+            torch.cuda.synchronize()
+            op.apply_device(k, xd.data_ptr(), yd.data_ptr())
+            torch.cuda.synchronize()
+            x = xd.cpu().double().numpy().reshape(n, k)
+            err = abs(yd.cpu().double().numpy().reshape(n, k) - S @ x)
+            assert (err <= bound * (W @ abs(x)) + 1e-300).all(), (k, shift)
+        op.close()
+
+
 def test_operator_transpose_dot_product(gpu):
     m, ve, kappa = c5_like(20, 5)
     ctx = FEMContext(m, 0, velocity_e=ve, normalize_velocity=False, kappa_e=kappa)
