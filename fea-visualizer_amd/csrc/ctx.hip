@@ -78,111 +78,228 @@ __global__ void k_inc_sort(const int* inc_ptr, int nv, int* inc) {
   }
 }
 
-// Distinct columns of row r (vertex i) in ascending order, by repeated
-// minimum search over the incident triangles (rows hold ~7 entries, so this
-// needs no per-thread list).  mode 0 counts, mode 1 writes col_idx and the
-// diagonal position.
-__global__ void k_row_cols(const uint32_t* tri, const uint8_t* onb, const int* idx, const int* row2v,
-                           const int* inc_ptr, const int* inc, int n, int bc, int mode, int* cnt,
-                           const int* rp, int* ci, int* diag) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
+// Distinct columns of row r (vertex i) in ascending order: the unknowns of the
+// incident triangles' vertices (those that pass the boundary filter, which for
+// a vertex that has a row are the ones with an unknown).  mode 0 counts, mode 1
+// writes col_idx and the diagonal position.
+//
+// Bound by latency: a thread's chain is incidence -> triangle -> unknown, then
+// the merge.  kChunk triangles are loaded at once and merged into a sorted list
+// of the thread's own in LDS (rows hold ~7 entries); a row past kListCap
+// entries searches its next larger column over the triangles again and again.
+// The search alone, for every row, took 131 us a launch at 261K rows, the list
+// 23.
+constexpr int kChunk = 3;
+constexpr int kListCap = 16;
+__global__ void __launch_bounds__(kBlock) k_row_cols(const uint32_t* __restrict__ tri, const int* __restrict__ idx,
+                                                     const int* __restrict__ row2v, const int* __restrict__ inc_ptr,
+                                                     const int* __restrict__ inc, int n, int mode,
+                                                     int* __restrict__ cnt, const int* __restrict__ rp,
+                                                     int* __restrict__ ci, int* __restrict__ diag) {
+  __shared__ int list[kListCap][kBlock];
+  const int r = blockIdx.x * kBlock + threadIdx.x, tid = threadIdx.x;
   if (r >= n) return;
-  int i = row2v[r];
-  bool bi = onb[i] != 0;
-  int lo = inc_ptr[i], hi = inc_ptr[i + 1];
-  int last = -1, c = 0, out = (mode == 1) ? rp[r] : 0, dpos = -1;
-  while (true) {
-    int best = INT32_MAX;
-    for (int e = lo; e < hi; e++) {
-      int t = inc[e];
+  const int i = row2v[r];
+  const int lo = inc_ptr[i], hi = inc_ptr[i + 1];
+  int c = 0;
+  bool fits = true;
+  for (int e0 = lo; e0 < hi && fits; e0 += kChunk) {
+    int col[kChunk][3];
+#pragma unroll
+    for (int u = 0; u < kChunk; u++) {
+      const size_t t = 3 * (size_t)inc[min(e0 + u, hi - 1)];
+#pragma unroll
+      for (int b = 0; b < 3; b++) col[u][b] = idx[tri[t + b]];
+    }
+#pragma unroll
+    for (int u = 0; u < kChunk; u++)
+#pragma unroll
       for (int b = 0; b < 3; b++) {
-        uint32_t w = tri[3 * (size_t)t + b];
-        if (!(bc == FEM_NEUMANN || (!bi && !onb[w]))) continue;
-        int col = idx[w];
-        if (col > last && col < best) best = col;
+        const int w = col[u][b];
+        if (w < 0) continue;
+        int q = c;  // list[0..q) < w
+        while (q > 0 && list[q - 1][tid] > w) q--;
+        if (q > 0 && list[q - 1][tid] == w) continue;
+        if (c == kListCap) {
+          fits = false;
+          continue;
+        }
+        for (int m = c; m > q; m--) list[m][tid] = list[m - 1][tid];
+        list[q][tid] = w;
+        c++;
       }
+  }
+  const int out = mode == 1 ? rp[r] : 0;
+  int dpos = -1;
+  if (fits) {
+    if (mode == 1)
+      for (int q = 0; q < c; q++) {
+        const int w = list[q][tid];
+        ci[out + q] = w;
+        if (w == r) dpos = out + q;
+      }
+  } else {
+    c = 0;
+    for (int last = -1;; c++) {
+      int best = INT32_MAX;
+      for (int e = lo; e < hi; e++)
+        for (int b = 0; b < 3; b++) {
+          const int w = idx[tri[3 * (size_t)inc[e] + b]];
+          if (w > last && w < best) best = w;
+        }
+      if (best == INT32_MAX) break;
+      if (mode == 1) {
+        ci[out + c] = best;
+        if (best == r) dpos = out + c;
+      }
+      last = best;
     }
-    if (best == INT32_MAX) break;
-    if (mode == 1) {
-      ci[out + c] = best;
-      if (best == r) dpos = out + c;
-    }
-    c++;
-    last = best;
   }
   if (mode == 0) cnt[r] = c;
   else diag[r] = dpos;
 }
 
-__device__ inline int find_slot(const int* ci, int lo, int hi, int col) {
-  for (int s = lo; s < hi; s++)
-    if (ci[s] == col) return s;
-  return -1;
+// Position of col in the ascending cols[0..m); col is there.
+__device__ inline int find_slot(const int* cols, int m, int col) {
+  int lo = 0;
+  while (m > 1) {
+    const int half = m >> 1;
+    if (cols[lo + half] <= col) lo += half;
+    m -= half;
+  }
+  return lo;
 }
 
-__global__ void k_assemble(const float* xyz, const uint32_t* tri, const uint8_t* onb, const int* idx,
-                           const int* row2v, const int* inc_ptr, const int* inc, const int* rp,
-                           const int* ci, int n, int bc, double vx, double vy, double vz,
-                           const double* vel_e, int normalize, const double* kappa_e, double* K,
-                           double* M, double* A, double* lumped) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  int i = row2v[r];
-  int lo = rp[r], hi = rp[r + 1];
-  for (int s = lo; s < hi; s++) {
-    K[s] = 0.0;
-    M[s] = 0.0;
-    A[s] = 0.0;
-  }
-  bool bi = onb[i] != 0;
-  for (int e = inc_ptr[i]; e < inc_ptr[i + 1]; e++) {
-    int t = inc[e];
-    const uint32_t* tv3 = tri + 3 * (size_t)t;
-    Geo G;
-    elem_geom(xyz, tv3, G);
-    double kap = kappa_e ? kappa_e[t] : 1.0;
-    double mo = G.jdet / 24.0;
-    double vel[3] = {vx, vy, vz};
-    if (vel_e) {
-      vel[0] = vel_e[3 * (size_t)t];
-      vel[1] = vel_e[3 * (size_t)t + 1];
-      vel[2] = vel_e[3 * (size_t)t + 2];
+// K, M, A of the mesh and M's row sums.  A thread owns a row and walks the row
+// vertex's triangles in ascending element order.
+//
+// Bound by latency and by the FP64 divides of the geometry (each triangle is
+// formed by its three rows).  The workgroup's rows are one stretch of the CSR
+// arrays, so their columns and sums stay in LDS and the stretch is written
+// once, in whole lines; kChunk triangles' vertices are in flight at once.
+// Accumulating in global memory instead chained a search of the row's columns
+// and three read-modify-writes per triangle corner: 409 us at 261K rows, 68
+// now.  Blocks whose rows average more than kAsmRow entries (~7 on a surface)
+// still accumulate there.
+constexpr int kAsmBlock = 64, kAsmRow = 8, kAsmCap = kAsmBlock * kAsmRow;
+__global__ void __launch_bounds__(kAsmBlock) k_assemble(
+    const float* __restrict__ xyz, const uint32_t* __restrict__ tri, const uint8_t* __restrict__ onb,
+    const int* __restrict__ idx, const int* __restrict__ row2v, const int* __restrict__ inc_ptr,
+    const int* __restrict__ inc, const int* __restrict__ rp, const int* __restrict__ ci, int n, int bc, double vx,
+    double vy, double vz, const double* __restrict__ vel_e, int normalize, const double* __restrict__ kappa_e,
+    double* __restrict__ K, double* __restrict__ M, double* __restrict__ A, double* __restrict__ lumped) {
+  __shared__ int s_ci[kAsmCap];
+  __shared__ double s_K[kAsmCap], s_M[kAsmCap], s_A[kAsmCap];
+  const int row0 = blockIdx.x * kAsmBlock, tid = threadIdx.x;
+  const int base = rp[row0], end = rp[min(n, row0 + kAsmBlock)];
+  const bool staged = end - base <= kAsmCap;
+  if (staged)
+    for (int s = tid; s < end - base; s += kAsmBlock) {
+      s_ci[s] = ci[base + s];
+      s_K[s] = 0.0;
+      s_M[s] = 0.0;
+      s_A[s] = 0.0;
     }
-    // FEMContext.cpp:179-180: tangential projection, then normalised
-    double nn = G.nrm[0] * G.nrm[0] + G.nrm[1] * G.nrm[1] + G.nrm[2] * G.nrm[2];
-    double vd = (vel[0] * G.nrm[0] + vel[1] * G.nrm[1] + vel[2] * G.nrm[2]) / nn;
-    double tvel[3];
-    for (int q = 0; q < 3; q++) tvel[q] = vel[q] - vd * G.nrm[q];
-    if (normalize) {
-      double z = tvel[0] * tvel[0] + tvel[1] * tvel[1] + tvel[2] * tvel[2];
-      if (z > 0.0) {
-        double sz = sqrt(z);
-        for (int q = 0; q < 3; q++) tvel[q] = tvel[q] / sz;
-      }
-    }
-    double jd6 = G.jdet / 6.0;
-    for (int a = 0; a < 3; a++) {
-      if (tv3[a] != (uint32_t)i) continue;
-      for (int b = 0; b < 3; b++) {
-        uint32_t w = tv3[b];
-        bool bw = onb[w] != 0;
-        bool keep_km = (bc == FEM_NEUMANN) || (!bi && !bw);  // FEMContext.cpp:99,136
-        bool keep_a = !bi && !bw;                              // FEMContext.cpp:188
-        if (!keep_km && !keep_a) continue;
-        int s = find_slot(ci, lo, hi, idx[w]);
-        if (s < 0) continue;
-        if (keep_km) {
-          double kab = elem_kab(G, a, b);
-          K[s] += kap * kab;
-          M[s] += (a == b) ? 2.0 * mo : mo;
+  __syncthreads();
+  const int r = row0 + tid;
+  // cols, k, m, a: the row's m_row columns and sums, in LDS or in memory
+  auto row = [&](const int* cols, int m_row, double* k, double* m, double* a) __attribute__((always_inline)) {
+    const int i = row2v[r];
+    const bool bi = onb[i] != 0;
+    const int hi = inc_ptr[i + 1];
+    for (int e0 = inc_ptr[i]; e0 < hi; e0 += kChunk) {
+      int t[kChunk];
+      uint32_t v[kChunk][3];
+      float p[kChunk][3][3];
+      int col[kChunk][3];
+      bool bw[kChunk][3];
+#pragma unroll
+      for (int u = 0; u < kChunk; u++) t[u] = inc[min(e0 + u, hi - 1)];
+#pragma unroll
+      for (int u = 0; u < kChunk; u++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) v[u][b] = tri[3 * (size_t)t[u] + b];
+#pragma unroll
+      for (int u = 0; u < kChunk; u++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+          for (int q = 0; q < 3; q++) p[u][b][q] = xyz[3 * (size_t)v[u][b] + q];
+          col[u][b] = idx[v[u][b]];
+          bw[u][b] = onb[v[u][b]] != 0;
         }
-        if (keep_a) A[s] += jd6 * (tvel[0] * G.g[b][0] + tvel[1] * G.g[b][1] + tvel[2] * G.g[b][2]);
+#pragma unroll
+      for (int u = 0; u < kChunk; u++) {
+        if (e0 + u >= hi) break;
+        Geo G;
+        elem_geom_at(p[u], G);
+        const double kap = kappa_e ? kappa_e[t[u]] : 1.0;
+        const double mo = G.jdet / 24.0;
+        double vel[3] = {vx, vy, vz};
+        if (vel_e)
+          for (int q = 0; q < 3; q++) vel[q] = vel_e[3 * (size_t)t[u] + q];
+        // FEMContext.cpp:179-180: tangential projection, then normalised
+        const double nn = G.nrm[0] * G.nrm[0] + G.nrm[1] * G.nrm[1] + G.nrm[2] * G.nrm[2];
+        const double vd = (vel[0] * G.nrm[0] + vel[1] * G.nrm[1] + vel[2] * G.nrm[2]) / nn;
+        double tvel[3];
+        for (int q = 0; q < 3; q++) tvel[q] = vel[q] - vd * G.nrm[q];
+        if (normalize) {
+          const double z = tvel[0] * tvel[0] + tvel[1] * tvel[1] + tvel[2] * tvel[2];
+          if (z > 0.0) {
+            const double sz = sqrt(z);
+            for (int q = 0; q < 3; q++) tvel[q] = tvel[q] / sz;
+          }
+        }
+        const double jd6 = G.jdet / 6.0;
+        // the row vertex is one corner (a degenerate triangle may repeat it)
+        unsigned corners = 0;
+#pragma unroll
+        for (int c = 0; c < 3; c++) corners |= v[u][c] == (uint32_t)i ? 1u << c : 0u;
+        while (corners) {
+          const int c = __ffs(corners) - 1;
+          corners &= corners - 1;
+          double gc[3];
+#pragma unroll
+          for (int q = 0; q < 3; q++) gc[q] = c == 0 ? G.g[0][q] : c == 1 ? G.g[1][q] : G.g[2][q];
+#pragma unroll
+          for (int b = 0; b < 3; b++) {
+            const bool keep_km = (bc == FEM_NEUMANN) || (!bi && !bw[u][b]);  // FEMContext.cpp:99,136
+            const bool keep_a = !bi && !bw[u][b];                            // FEMContext.cpp:188
+            if (!keep_km && !keep_a) continue;
+            const int s = find_slot(cols, m_row, col[u][b]);
+            if (keep_km) {
+              const double kab = G.area * (gc[0] * G.g[b][0] + gc[1] * G.g[b][1] + gc[2] * G.g[b][2]);  // elem_kab
+              k[s] += kap * kab;
+              m[s] += (c == b) ? 2.0 * mo : mo;
+            }
+            if (keep_a) a[s] += jd6 * (tvel[0] * G.g[b][0] + tvel[1] * G.g[b][1] + tvel[2] * G.g[b][2]);
+          }
+        }
       }
     }
+    double acc = 0.0;
+    for (int s = 0; s < m_row; s++) acc += m[s];
+    lumped[r] = acc;
+  };
+  if (r < n) {
+    const int lo = rp[r], m_row = rp[r + 1] - lo;
+    if (staged) {
+      row(s_ci + (lo - base), m_row, s_K + (lo - base), s_M + (lo - base), s_A + (lo - base));
+    } else {
+      for (int s = lo; s < lo + m_row; s++) {
+        K[s] = 0.0;
+        M[s] = 0.0;
+        A[s] = 0.0;
+      }
+      row(ci + lo, m_row, K + lo, M + lo, A + lo);
+    }
   }
-  double acc = 0.0;
-  for (int s = lo; s < hi; s++) acc += M[s];
-  lumped[r] = acc;
+  __syncthreads();
+  if (staged)
+    for (int s = tid; s < end - base; s += kAsmBlock) {
+      K[base + s] = s_K[s];
+      M[base + s] = s_M[s];
+      A[base + s] = s_A[s];
+    }
 }
 
 // Position of (c, r) for every CSR entry (r, c); the pattern is structurally
@@ -240,7 +357,7 @@ int ctx_assemble(fem_ctx* c, const fem_assembly_params* prm) {
   c->normalize = p.normalize_velocity;
   for (int q = 0; q < 3; q++) c->velocity[q] = p.velocity[q];
   if (c->n > 0) {
-    hipLaunchKernelGGL(k_assemble, dim3(div_up(c->n, kBlock)), dim3(kBlock), 0, c->stream, c->d_xyz, c->d_tri,
+    hipLaunchKernelGGL(k_assemble, dim3(div_up(c->n, kAsmBlock)), dim3(kAsmBlock), 0, c->stream, c->d_xyz, c->d_tri,
                        c->d_onb, c->d_idx, c->d_row2v, c->d_inc_ptr, c->d_inc, c->d_rp, c->d_ci, c->n, c->bc,
                        p.velocity[0], p.velocity[1], p.velocity[2], c->d_vel_e, p.normalize_velocity,
                        c->d_kappa_e, c->d_K, c->d_M, c->d_A, c->d_lumped);
@@ -329,8 +446,8 @@ int ctx_create(const fem_mesh* mesh, int bc, fem_ctx** out) {
   if (rc) { ctx_free(c); return rc; }
   int nnz = 0;
   if (n > 0) {
-    hipLaunchKernelGGL(k_row_cols, dim3(div_up(n, kBlock)), dim3(kBlock), 0, st, c->d_tri, c->d_onb, c->d_idx,
-                       c->d_row2v, c->d_inc_ptr, c->d_inc, n, bc, 0, c->d_rp, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(k_row_cols, dim3(div_up(n, kBlock)), dim3(kBlock), 0, st, c->d_tri, c->d_idx,
+                       c->d_row2v, c->d_inc_ptr, c->d_inc, n, 0, c->d_rp, nullptr, nullptr, nullptr);
     CKH(hipMemsetAsync(c->d_rp + n, 0, sizeof(int), st));
     CKH(hipGetLastError());
     CK(exclusive_scan_i32(c->d_rp, c->d_rp, n + 1, &nnz, st));
@@ -345,8 +462,8 @@ int ctx_create(const fem_mesh* mesh, int bc, fem_ctx** out) {
   c->d_A = dalloc<double>((size_t)nnz + 1, &rc);
   if (rc) { ctx_free(c); return rc; }
   if (n > 0) {
-    hipLaunchKernelGGL(k_row_cols, dim3(div_up(n, kBlock)), dim3(kBlock), 0, st, c->d_tri, c->d_onb, c->d_idx,
-                       c->d_row2v, c->d_inc_ptr, c->d_inc, n, bc, 1, nullptr, c->d_rp, c->d_ci, c->d_diag);
+    hipLaunchKernelGGL(k_row_cols, dim3(div_up(n, kBlock)), dim3(kBlock), 0, st, c->d_tri, c->d_idx,
+                       c->d_row2v, c->d_inc_ptr, c->d_inc, n, 1, nullptr, c->d_rp, c->d_ci, c->d_diag);
     hipLaunchKernelGGL(k_tperm, dim3(div_up(n, kBlock)), dim3(kBlock), 0, st, c->d_rp, c->d_ci, n, c->d_tperm);
     CKH(hipGetLastError());
   }

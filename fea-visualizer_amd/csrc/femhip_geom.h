@@ -17,12 +17,13 @@ struct Geo {
 // FEMContext.cpp:73-95: n = normalize(cross(b-a, c-a)), area = |cross|/2,
 // J = [b-a, c-a, n], gradients = rows of J^{-1} applied to the reference
 // gradients {(-1,-1,0),(1,0,0),(0,1,0)}; J^{-1} by cofactors.
-__device__ inline void elem_geom(const float* xyz, const uint32_t* t, Geo& G) {
+// p: the three vertices' positions.
+__device__ inline void elem_geom_at(const float p[3][3], Geo& G) {
   double a[3], e1[3], e2[3];
   for (int k = 0; k < 3; k++) {
-    a[k] = (double)xyz[3 * (size_t)t[0] + k];
-    e1[k] = (double)xyz[3 * (size_t)t[1] + k] - a[k];
-    e2[k] = (double)xyz[3 * (size_t)t[2] + k] - a[k];
+    a[k] = (double)p[0][k];
+    e1[k] = (double)p[1][k] - a[k];
+    e2[k] = (double)p[2][k] - a[k];
   }
   double cr0 = e1[1] * e2[2] - e1[2] * e2[1];
   double cr1 = e1[2] * e2[0] - e1[0] * e2[2];
@@ -47,6 +48,13 @@ __device__ inline void elem_geom(const float* xyz, const uint32_t* t, Geo& G) {
   G.g[2][1] = (m00 * m22 - m02 * m20) / det;
   G.g[2][2] = (m02 * m10 - m00 * m12) / det;
   for (int k = 0; k < 3; k++) G.g[0][k] = -G.g[1][k] - G.g[2][k];
+}
+
+__device__ inline void elem_geom(const float* xyz, const uint32_t* t, Geo& G) {
+  float p[3][3];
+  for (int a = 0; a < 3; a++)
+    for (int k = 0; k < 3; k++) p[a][k] = xyz[3 * (size_t)t[a] + k];
+  elem_geom_at(p, G);
 }
 
 // Unit-diffusivity element stiffness area * grad(phi_a) . grad(phi_b)

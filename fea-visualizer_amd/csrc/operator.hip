@@ -21,19 +21,18 @@ namespace femhip {
 
 namespace {
 
-__global__ void k_op_form(int n, const int* rp, const int* tperm, const double* M, const double* Kk,
-                          const double* A, double cM, double cK, double cA, int fp32, void* val) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  for (int s = rp[r]; s < rp[r + 1]; s++) {
-    const int t = tperm ? tperm[s] : s;
-    double v = 0.0;
-    if (cM != 0.0) v += cM * M[t];
-    if (cK != 0.0) v += cK * Kk[t];
-    if (cA != 0.0) v += cA * A[t];
-    if (fp32) ((float*)val)[s] = (float)v;
-    else ((double*)val)[s] = v;
-  }
+__global__ void k_op_form(int nnz, const int* __restrict__ tperm, const double* __restrict__ M,
+                          const double* __restrict__ Kk, const double* __restrict__ A, double cM, double cK, double cA,
+                          int fp32, void* val) {
+  const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= nnz) return;
+  const int t = tperm ? tperm[s] : (int)s;
+  double v = 0.0;
+  if (cM != 0.0) v += cM * M[t];
+  if (cK != 0.0) v += cK * Kk[t];
+  if (cA != 0.0) v += cA * A[t];
+  if (fp32) ((float*)val)[s] = (float)v;
+  else ((double*)val)[s] = v;
 }
 
 template <typename T, int K, int G>
@@ -481,8 +480,8 @@ int operator_create(fem_ctx* c, const double coef[3], int precision, int transpo
     operator_free(op);
     return rc;
   }
-  if (c->n > 0) {
-    hipLaunchKernelGGL(k_op_form, dim3(div_up(c->n, kBlock)), dim3(kBlock), 0, op->stream, c->n, c->d_rp,
+  if (c->nnz > 0) {
+    hipLaunchKernelGGL(k_op_form, dim3(div_up(c->nnz, kBlock)), dim3(kBlock), 0, op->stream, (int)c->nnz,
                        transpose ? c->d_tperm : nullptr, c->d_M, c->d_K, c->d_A, coef[0], coef[1], coef[2],
                        precision == FEM_PREC_FP32_IR ? 1 : 0, op->d_val);
     e = hipGetLastError();

@@ -55,6 +55,36 @@ def test_pattern_and_matrices(gpu, name):
         assert np.max(np.abs(got - ref)) <= 1e-12 * max(1e-300, np.max(np.abs(ref)))
 
 
+@pytest.mark.parametrize("bc", [0, 1])
+@pytest.mark.parametrize("rims", [(3,), (14, 15, 16, 17), (40, 3, 21, 9), (600, 5, 16), (9,) * 80])
+def test_pattern_and_matrices_fans(gpu, rims, bc):
+    """Disjoint fans of a hub and its rim, vertices and triangles shuffled: rows
+    of up to 601 entries, on either side of what a row's list and a block's
+    stretch hold in fast memory, and a last block with a rest."""
+    print("case fans", rims, bc, flush=True)
+    rng = np.random.Generator(np.random.PCG64(sum(rims)))
+    xyz, tri, at = [], [], 0
+    for q, d in enumerate(rims):
+        t = 2 * np.pi * np.arange(d) / d
+        xyz += [np.array([[3.0 * q, 0, 0.5]]), np.stack([3.0 * q + np.cos(t), np.sin(t), 0.1 * np.cos(3 * t)], 1)]
+        tri.append(at + np.stack([np.zeros(d, int), 1 + np.arange(d), 1 + (np.arange(d) + 1) % d], 1))
+        at += d + 1
+    perm = rng.permutation(at)
+    pos = np.empty((at, 3), np.float32)
+    pos[perm] = np.concatenate(xyz)
+    m = {"xyz": pos, "tri": np.ascontiguousarray(rng.permutation(perm[np.concatenate(tri)]).astype(np.uint32)),
+         "on_boundary": (rng.random(at) < 0.2).astype(np.uint8)}
+    ve = rng.standard_normal((len(m["tri"]), 3))
+    kappa = rng.uniform(0.5, 2.0, len(m["tri"]))
+    ctx = FEMContext(m, bc, velocity_e=ve, normalize_velocity=True, kappa_e=kappa)
+    s = oracle.System(m, bc=bc, velocity_e=ve, normalize=True, kappa_e=kappa)
+    rp, ci = ctx.pattern()
+    assert np.array_equal(ctx.idx_map, s.idx_map)
+    assert np.array_equal(rp, s.row_ptr) and np.array_equal(ci, s.col_idx)
+    for which, ref in ((_lib.FEM_MATRIX_K, s.K), (_lib.FEM_MATRIX_M, s.M), (_lib.FEM_MATRIX_A, s.A)):
+        assert np.max(np.abs(ctx.matrix(which) - ref)) <= 1e-12 * max(1e-300, np.max(np.abs(ref)))
+
+
 def test_golden_square_matrices(gpu):
     g = dict(np.load(os.path.join(GOLD, "square64.npz")))
     m = {"xyz": g["xyz"], "tri": g["tri"], "on_boundary": g["on_boundary"]}
