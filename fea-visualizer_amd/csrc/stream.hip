@@ -39,6 +39,7 @@ struct SState {
   int sweep_done, solve_done, redo, bkd;
   int it_s, its, sweeps, status;
   long long its_total, sweeps_total;
+  int vote;  // reduction workgroups of the running phase that have their sums (k_sreduce)
 };
 
 enum Phase : int {
@@ -70,6 +71,7 @@ struct SArgs {
   int pass;             // FP64 residual: 0 normal, 1 redo with the correction dropped
   int more;             // update: another step follows in this launch (it reads xnext)
   double* partials;     // [nblocks][kPartW K]
+  double* sums;         // [instances][kPartW K]: sums of an instance's reduction workgroups (k_sreduce)
   const int* act_blk;   // launched block -> row block (null: every row block, in order)
   const int* act_inst;  // reduction block -> instance (null: every instance)
   const int* act_cnt;   // {instances, blocks} of the lists (device); the grid may be larger
@@ -396,12 +398,20 @@ __global__ void __launch_bounds__(kBlock) k_sphase(SArgs a) {
 // row blocks, and the sum is bound by how many partials are in flight.
 constexpr int kRedBlock = 1024;
 
-// Sum of the instance's block partials in a fixed order: thread (q, c) sums
-// blocks c, c + chunks, ... of value q, kR loads in flight at a time; a fixed
-// pairwise tree combines the chunk sums.
-template <int K, int NS>
-__device__ void sum_blocks(const SArgs& a, const int* inst_blk, int i, double* red, double* scratch) {
-  constexpr int nv = NS * K;
+// Reduction workgroups per instance: 16 columns with several sums each have
+// as many values per row block, so each sum gets a workgroup of its own and
+// the last one to finish advances the scalars; one workgroup read the 80
+// values of BiCGSTAB's phase S over 2,048 row blocks in 27 us, the five take 8.
+template <int K, int PH>
+constexpr int red_parts() {
+  return K >= 16 ? (nsums<K, PH>() > 1 ? nsums<K, PH>() : 1) : 1;
+}
+
+// Sums of nv of the values, from q0, over the instance's row blocks in a fixed
+// order: thread (q, c) sums blocks c, c + chunks, ... of value q0 + q, kR loads
+// in flight at a time; a fixed pairwise tree combines the chunk sums.
+template <int K, int nv>
+__device__ void sum_blocks(const SArgs& a, const int* inst_blk, int i, int q0, double* red, double* scratch) {
   constexpr int chunks = kRedBlock / nv;
   const int q = threadIdx.x % nv, c = threadIdx.x / nv;
   const int b0 = inst_blk[i], b1 = inst_blk[i + 1];
@@ -413,7 +423,7 @@ __device__ void sum_blocks(const SArgs& a, const int* inst_blk, int i, double* r
 #pragma unroll
       for (int u = 0; u < kR; u++) {
         const int w = w0 + u * chunks;
-        v[u] = (w < b1) ? a.partials[(size_t)w * kPartW * K + q] : 0.0;
+        v[u] = (w < b1) ? a.partials[(size_t)w * kPartW * K + q0 + q] : 0.0;
       }
 #pragma unroll
       for (int u = 0; u < kR; u++) s += v[u];
@@ -446,189 +456,208 @@ __device__ inline void post_flag_word(const SArgs& a, int v) {
                      __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// One block per instance: reduce the phase's partials and advance the scalar
-// recurrences exactly as the persistent drivers do after their barriers.
+// Reduce the phase's partials (red_parts workgroups per instance) and advance
+// the scalar recurrences exactly as the persistent drivers do after their
+// barriers: lane j of the first wave (of the last workgroup to have its sums)
+// advances column j.  One thread advancing the columns in turn took 4 us of
+// the 10 of a 16-column reduction.
 template <int K, int PH>
 __global__ void __launch_bounds__(kRedBlock) k_sreduce(SArgs a, const int* inst_blk, int ninst, int fp32) {
+  constexpr int NS = nsums<K, PH>();
+  constexpr int parts = red_parts<K, PH>();
+  constexpr int nv = NS * K / parts;  // values of this workgroup
+  static_assert(nv * parts == NS * K && (parts == 1 || nv <= kWave), "reduction workgroups");
   __shared__ double scratch[kRedBlock];
-  __shared__ double red[kPartW * kMaxK];
-  if ((int)blockIdx.x >= ninst || (a.act_cnt && (int)blockIdx.x >= a.act_cnt[0])) return;
-  const int i = a.act_inst ? a.act_inst[blockIdx.x] : blockIdx.x;
+  __shared__ double red[nv];
+  const int slot = (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;
+  if (slot >= ninst || (a.act_cnt && slot >= a.act_cnt[0])) return;
+  const int i = a.act_inst ? a.act_inst[slot] : slot;
   const Inst& I = a.insts[i];
   SState& S = a.ss[i];
+  const int j = threadIdx.x;
   if constexpr (PH == PH_RES) {
     if (a.pass ? !S.redo : S.solve_done) return;
   } else if constexpr (PH != PH_RHS) {
     if (S.sweep_done) {
       if constexpr (ends_iteration<PH>())
-        if (a.post && threadIdx.x == 0) post_flag_word(a, 1);
+        if (a.post && part == 0 && j == 0) post_flag_word(a, 1);
       return;
     }
   }
-  // pipelined CG, few columns: thread 0 loads the recurrence's scalars before
-  // the sums, so the loads overlap them (no dependent round trip at the end)
-  constexpr bool pre = PH == PH_PCG_ITER && K <= 4;
-  double p_gamma[pre ? K : 1], p_alpha[pre ? K : 1], p_ithr[pre ? K : 1];
-  int p_active[pre ? K : 1], p_it_s = 0, p_its = 0, p_max_inner = 0, p_max_iters = 0;
-  if constexpr (pre) {
-    if (threadIdx.x == 0) {
-      for (int j = 0; j < K; j++) {
-        p_gamma[j] = S.gamma[j];
-        p_alpha[j] = S.alpha[j];
-        p_ithr[j] = S.ithr[j];
-        p_active[j] = S.active[j];
-      }
-      p_it_s = S.it_s;
-      p_its = S.its;
-      p_max_inner = I.max_inner;
-      p_max_iters = I.max_iters;
-    }
+  // the recurrence's scalars, loaded before the sums so that the loads overlap
+  // them (no dependent round trip at the end)
+  double p_gamma = 0, p_alpha = 0, p_omega = 0, p_thr = 0, p_ithr = 0, p_bb = 0;
+  int p_active = 0, p_bbad = 0, p_it_s = 0, p_its = 0, p_bkd = 0, p_max_inner = 0, p_max_iters = 0;
+  if (j < K) {
+    p_gamma = S.gamma[j];
+    p_alpha = S.alpha[j];
+    p_omega = S.omega[j];
+    p_thr = S.thr[j];
+    p_ithr = S.ithr[j];
+    p_bb = S.bb[j];
+    p_active = S.active[j];
+    p_bbad = S.bbad[j];
+    p_it_s = S.it_s;
+    p_its = S.its;
+    p_bkd = S.bkd;
+    p_max_inner = I.max_inner;
+    p_max_iters = I.max_iters;
   }
-  sum_blocks<K, nsums<K, PH>()>(a, inst_blk, i, red, scratch);
-  if (threadIdx.x != 0) return;
+  sum_blocks<K, nv>(a, inst_blk, i, part * nv, red, scratch);
+  if (j >= kWave) return;
+  double v[NS];  // column j's sums
+  if constexpr (parts > 1) {
+    double* sums = a.sums + (size_t)i * kPartW * K;
+    if (j < nv) __hip_atomic_store(sums + part * nv + j, red[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);  // they are in memory before the vote is
+    int last = 0;
+    if (j == 0)
+      last = __hip_atomic_fetch_add(&S.vote, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+    if (!__shfl(last, 0)) return;
+    if (j == 0) __hip_atomic_store(&S.vote, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (j >= K) return;
+#pragma unroll
+    for (int q = 0; q < NS; q++)
+      v[q] = __hip_atomic_load(sums + q * K + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    if (j >= K) return;
+#pragma unroll
+    for (int q = 0; q < NS; q++) v[q] = red[q * K + j];
+  }
+  auto any = [](bool x) { return __ballot(x) != 0; };  // over the columns
   if constexpr (PH == PH_RHS) {
-    int any = 0;
-    for (int j = 0; j < K; j++) {
-      const double bb = red[j], rr = red[K + j];
-      S.bb[j] = bb;
-      S.thr[j] = fmax(I.tol2 * bb, DBL_MIN);
-      S.active[j] = (bb != 0.0) && (rr >= S.thr[j]);
-      S.gamma[j] = red[2 * K + j];
-      S.ithr[j] = rr;
-      S.reset[j] = 0;
-      any |= S.active[j];
+    const double bb = v[0], rr = v[1], thr = fmax(I.tol2 * bb, DBL_MIN);
+    const bool active = (bb != 0.0) && (rr >= thr);
+    S.bb[j] = bb;
+    S.thr[j] = thr;
+    S.active[j] = active;
+    S.gamma[j] = v[2];
+    S.ithr[j] = rr;
+    S.reset[j] = 0;
+    const bool go = any(active);
+    if (j == 0) {
+      S.solve_done = !go;
+      S.sweep_done = 1;
+      S.redo = 0;
+      S.sweeps = 0;
+      S.its = 0;
     }
-    S.solve_done = !any;
-    S.sweep_done = 1;
-    S.redo = 0;
-    S.sweeps = 0;
-    S.its = 0;
   } else if constexpr (PH == PH_RES) {
-    int redo = 0;
+    const double rr = v[0];
+    bool redo = false;
     if (!a.pass) {
-      for (int j = 0; j < K; j++) {
-        const bool bad = !(red[j] <= DBL_MAX);  // NaN or infinite: drop the sweep's correction
-        redo |= bad;
-        S.reset[j] = bad;
-      }
+      const bool bad = !(rr <= DBL_MAX);  // NaN or infinite: drop the sweep's correction
+      redo = any(bad);
+      S.reset[j] = bad;
     }
-    S.redo = redo;
+    if (j == 0) S.redo = redo;
     if (redo) return;  // finalised by the second pass
-    int any = 0;
-    for (int j = 0; j < K; j++) {
-      const double rr = red[j];
-      S.active[j] = (S.bb[j] != 0.0) && (rr >= S.thr[j]) && (rr == rr);
-      S.gamma[j] = red[K + j];
-      S.ithr[j] = rr;
-      S.reset[j] = 0;
-      any |= S.active[j];
+    const bool active = (p_bb != 0.0) && (rr >= p_thr) && (rr == rr);
+    S.active[j] = active;
+    S.gamma[j] = v[1];
+    S.ithr[j] = rr;
+    S.reset[j] = 0;
+    const bool go = any(active);
+    if (j == 0) {
+      S.sweeps++;
+      S.solve_done = !go;
     }
-    S.sweeps++;
-    S.solve_done = !any;
   } else if constexpr (PH == PH_PCG_INIT) {
-    for (int j = 0; j < K; j++) {
-      const double g = red[j], d = red[K + j];
-      S.gamma[j] = g;
-      S.alpha[j] = (S.active[j] && d != 0.0) ? g / d : 0.0;
-      S.beta[j] = 0.0;
-    }
+    const double g = v[0], d = v[1];
+    S.gamma[j] = g;
+    S.alpha[j] = (p_active && d != 0.0) ? g / d : 0.0;
+    S.beta[j] = 0.0;
   } else if constexpr (PH == PH_PCG_ITER) {
-    const int it_s = (pre ? p_it_s : S.it_s) + 1, its = (pre ? p_its : S.its) + 1;
-    S.it_s = it_s;
-    S.its = its;
-    int alldone = 1;
-    for (int j = 0; j < K; j++) {
-      const double g = red[j], d = red[K + j], rr = red[2 * K + j];
-      const double gold = pre ? p_gamma[j] : S.gamma[j], aold = pre ? p_alpha[j] : S.alpha[j];
-      const bool done = !(pre ? p_active[j] : S.active[j]) || rr < (pre ? p_ithr[j] : S.ithr[j]) || !(rr == rr);
-      double be = 0.0, al = 0.0;
-      if (!done && gold != 0.0 && aold != 0.0) {
-        be = g / gold;
-        const double den = d - be * g / aold;
-        al = (den != 0.0) ? g / den : 0.0;
-      }
-      S.beta[j] = be;
-      S.alpha[j] = al;
-      S.gamma[j] = g;
-      alldone &= done;
+    const double g = v[0], d = v[1], rr = v[2];
+    const bool done = !p_active || rr < p_ithr || !(rr == rr);
+    double be = 0.0, al = 0.0;
+    if (!done && p_gamma != 0.0 && p_alpha != 0.0) {
+      be = g / p_gamma;
+      const double den = d - be * g / p_alpha;
+      al = (den != 0.0) ? g / den : 0.0;
     }
-    S.sweep_done = alldone || it_s >= (pre ? p_max_inner : I.max_inner) || its >= (pre ? p_max_iters : I.max_iters);
+    S.beta[j] = be;
+    S.alpha[j] = al;
+    S.gamma[j] = g;
+    const bool go = any(!done);
+    if (j == 0) {
+      const int it_s = p_it_s + 1, its = p_its + 1;
+      S.it_s = it_s;
+      S.its = its;
+      const int sweep_done = !go || it_s >= p_max_inner || its >= p_max_iters;
+      S.sweep_done = sweep_done;
+      if (a.post) post_flag_word(a, sweep_done);
+    }
   } else if constexpr (PH == PH_CG_A) {
-    for (int j = 0; j < K; j++) {
-      const double pq = red[j];
-      S.alpha[j] = (S.active[j] && pq != 0.0) ? S.gamma[j] / pq : 0.0;
-    }
+    const double pq = v[0];
+    S.alpha[j] = (p_active && pq != 0.0) ? p_gamma / pq : 0.0;
   } else if constexpr (PH == PH_CG_B) {
-    S.it_s++;
-    S.its++;
-    int alldone = 1;
-    for (int j = 0; j < K; j++) {
-      const double rz = red[j], rr = red[K + j];
-      const double g = S.gamma[j];
-      S.beta[j] = (g != 0.0) ? rz / g : 0.0;
-      S.gamma[j] = rz;
-      alldone &= (!S.active[j]) || (rr < S.ithr[j]) || !(rr == rr);
+    const double rz = v[0], rr = v[1];
+    S.beta[j] = (p_gamma != 0.0) ? rz / p_gamma : 0.0;
+    S.gamma[j] = rz;
+    const bool go = any(p_active && !(rr < p_ithr) && rr == rr);
+    if (j == 0) {
+      const int it_s = p_it_s + 1, its = p_its + 1;
+      S.it_s = it_s;
+      S.its = its;
+      const int sweep_done = !go || it_s >= p_max_inner || its >= p_max_iters;
+      S.sweep_done = sweep_done;
+      if (a.post) post_flag_word(a, sweep_done);
     }
-    S.sweep_done = alldone || S.it_s >= I.max_inner || S.its >= I.max_iters;
   } else if constexpr (PH == PH_BI_P) {
-    S.bkd = 0;
-    for (int j = 0; j < K; j++) {
-      const double rv = red[j];
-      const double al = (S.active[j] && rv != 0.0) ? S.gamma[j] / rv : 0.0;
-      const bool fine = fabs(al) < 1e30;
-      S.alpha[j] = fine ? al : 0.0;
-      if (!fine) S.bkd = 1;
-    }
+    const double rv = v[0];
+    const double al = (p_active && rv != 0.0) ? p_gamma / rv : 0.0;
+    const bool fine = fabs(al) < 1e30;
+    S.alpha[j] = fine ? al : 0.0;
+    const bool bkd = any(!fine);
+    if (j == 0) S.bkd = bkd;
   } else if constexpr (PH == PH_BI_S) {
-    for (int j = 0; j < K; j++) {
-      const double ts = red[j], tt = red[K + j], ssv = red[2 * K + j];
-      const double om = (S.active[j] && tt > 0.0 && !(ssv < S.ithr[j])) ? ts / tt : 0.0;
-      const bool fine = fabs(om) < 1e30;
-      S.omega[j] = fine ? om : 0.0;
-      if (!fine) S.bkd = 1;
-      if constexpr (vec_layout<K>()) {
-        // next rho = <rh, s - omega t>, and beta for the x phase's new p;
-        // a breakdown stops the sweep only if the column goes on (phase X)
-        const double w = S.omega[j], rho = S.gamma[j];
-        const double rho_new = red[3 * K + j] - w * red[4 * K + j];
-        const double be = (w == 0.0 || rho == 0.0) ? 0.0 : (rho_new / rho) * (S.alpha[j] / w);
-        const bool bad = be == 0.0 || !(fabs(be) < 1e30);
-        S.bbad[j] = bad;
-        S.beta[j] = bad ? 0.0 : be;
-        S.gamma[j] = rho_new;
-      }
+    const double ts = v[0], tt = v[1], ssv = v[2];
+    const double om = (p_active && tt > 0.0 && !(ssv < p_ithr)) ? ts / tt : 0.0;
+    const bool fine = fabs(om) < 1e30;
+    const double w = fine ? om : 0.0;
+    S.omega[j] = w;
+    const bool bkd = any(!fine);
+    if (j == 0 && bkd) S.bkd = 1;
+    if constexpr (vec_layout<K>()) {
+      // next rho = <rh, s - omega t>, and beta for the x phase's new p;
+      // a breakdown stops the sweep only if the column goes on (phase X)
+      const double rho = p_gamma;
+      const double rho_new = v[3] - w * v[4];
+      const double be = (w == 0.0 || rho == 0.0) ? 0.0 : (rho_new / rho) * (p_alpha / w);
+      const bool bad = be == 0.0 || !(fabs(be) < 1e30);
+      S.bbad[j] = bad;
+      S.beta[j] = bad ? 0.0 : be;
+      S.gamma[j] = rho_new;
     }
-  } else if constexpr (PH == PH_BI_X && vec_layout<K>()) {
-    S.it_s++;
-    S.its++;
-    int alldone = 1, brk = S.bkd;
-    for (int j = 0; j < K; j++) {
-      const double rr = red[j];
-      const bool done = !S.active[j] || rr < S.ithr[j] || !(rr == rr);
-      alldone &= done;
-      if (!done && S.bbad[j]) brk = 1;
-    }
-    S.sweep_done = alldone || brk || S.it_s >= I.max_inner || S.its >= I.max_iters;
-  } else if constexpr (PH == PH_BI_X) {
-    S.it_s++;
-    S.its++;
-    int alldone = 1, brk = S.bkd;
-    for (int j = 0; j < K; j++) {
-      const double rho_new = red[j], rr = red[K + j];
-      const bool done = !S.active[j] || rr < S.ithr[j] || !(rr == rr);
-      alldone &= done;
+  } else {  // PH_BI_X
+    bool done, broke;
+    if constexpr (vec_layout<K>()) {
+      const double rr = v[0];
+      done = !p_active || rr < p_ithr || !(rr == rr);
+      broke = !done && p_bbad;
+    } else {
+      const double rho_new = v[0], rr = v[1];
+      done = !p_active || rr < p_ithr || !(rr == rr);
+      broke = false;
       if (!done) {
-        const double om = S.omega[j], rho = S.gamma[j];
-        const double be = (om == 0.0 || rho == 0.0) ? 0.0 : (rho_new / rho) * (S.alpha[j] / om);
-        if (be == 0.0 || !(fabs(be) < 1e30)) brk = 1;
-        else S.beta[j] = be;
+        const double be =
+            (p_omega == 0.0 || p_gamma == 0.0) ? 0.0 : (rho_new / p_gamma) * (p_alpha / p_omega);
+        broke = be == 0.0 || !(fabs(be) < 1e30);
+        if (!broke) S.beta[j] = be;
       }
       S.gamma[j] = rho_new;
     }
-    S.sweep_done = alldone || brk || S.it_s >= I.max_inner || S.its >= I.max_iters;
+    const bool go = any(!done), brk = any(broke) || p_bkd;
+    if (j == 0) {
+      const int it_s = p_it_s + 1, its = p_its + 1;
+      S.it_s = it_s;
+      S.its = its;
+      const int sweep_done = !go || brk || it_s >= p_max_inner || its >= p_max_iters;
+      S.sweep_done = sweep_done;
+      if (a.post) post_flag_word(a, sweep_done);
+    }
   }
-  if constexpr (ends_iteration<PH>())
-    if (a.post) post_flag_word(a, S.sweep_done);
   (void)fp32;
 }
 
@@ -762,6 +791,80 @@ __global__ void k_expand(const int* blk_inst, const int* inst_blk, const int* ac
   if (base >= 0) act_blk[base + gb - inst_blk[i]] = gb;
 }
 
+// k_compact, k_expand and k_post in one launch, for up to kListInsts
+// instances: every workgroup scans the instances itself and then lists its own
+// row blocks; the first also writes the instances, the counts and the host's
+// read (post, else null).  4.6 us where the three took 14.
+constexpr int kListInsts = 1024;
+__global__ void __launch_bounds__(kBlock) k_lists(const SState* ss, const int* inst_blk, const int* blk_inst, int ninst,
+                                                  int nblocks, int pred, int* act_inst, int* act_blk, int* cnt,
+                                                  unsigned long long* post, unsigned seq) {
+  constexpr int E = kListInsts / kBlock;  // instances per thread
+  __shared__ int base[kListInsts];        // an active instance's first position less its first row block
+  __shared__ int wsum[kBlock / kWave][2];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  const int gb = blockIdx.x * kBlock + t;
+  const int mine = gb < nblocks ? blk_inst[gb] : 0;
+  int on[E], first[E], nb[E], sb = 0, si = 0;
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const int i = t * E + e;
+    on[e] = first[e] = nb[e] = 0;
+    if (i < ninst) {
+      const SState& S = ss[i];
+      on[e] = pred == 0 ? !S.sweep_done : pred == 1 ? !S.solve_done : S.redo != 0;
+      first[e] = inst_blk[i];
+      nb[e] = on[e] ? inst_blk[i + 1] - first[e] : 0;
+    }
+    sb += nb[e];
+    si += on[e];
+  }
+  int ib = sb, ii = si;  // inclusive scans over the workgroup
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int vb = __shfl_up(ib, d), vi = __shfl_up(ii, d);
+    if (lane >= d) {
+      ib += vb;
+      ii += vi;
+    }
+  }
+  if (lane == kWave - 1) {
+    wsum[wave][0] = ib;
+    wsum[wave][1] = ii;
+  }
+  __syncthreads();
+  int tot_b = 0, tot_i = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / kWave; w++) {
+    if (w < wave) {
+      ib += wsum[w][0];
+      ii += wsum[w][1];
+    }
+    tot_b += wsum[w][0];
+    tot_i += wsum[w][1];
+  }
+  int pb = ib - sb, pi = ii - si;
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const int i = t * E + e;
+    base[i] = on[e] ? pb - first[e] : INT32_MIN;
+    if (on[e] && blockIdx.x == 0) act_inst[pi] = i;
+    pb += nb[e];
+    pi += on[e];
+  }
+  __syncthreads();
+  if (gb < nblocks && base[mine] != INT32_MIN) act_blk[base[mine] + gb] = gb;
+  if (blockIdx.x == 0 && t == 0) {
+    cnt[0] = tot_i;
+    cnt[1] = tot_b;
+    if (post) {
+      const unsigned long long tag = (unsigned long long)seq << 32;
+      __hip_atomic_store(post, tag | (unsigned)tot_i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(post + 1, tag | (unsigned)tot_b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+}
+
 template <int K, typename TI>
 const void* phase_fn(int ph, bool walk) {
   if (walk) {  // the phases a budgeted run launches over its fixed grid
@@ -817,6 +920,21 @@ const void* pick_phase(int k, int fp32, int ph, bool walk) {
   }
 }
 
+template <int K>
+int reduce_parts(int ph) {
+  switch (ph) {
+    case PH_RHS: return red_parts<K, PH_RHS>();
+    case PH_RES: return red_parts<K, PH_RES>();
+    case PH_PCG_INIT: return red_parts<K, PH_PCG_INIT>();
+    case PH_PCG_ITER: return red_parts<K, PH_PCG_ITER>();
+    case PH_CG_A: return red_parts<K, PH_CG_A>();
+    case PH_CG_B: return red_parts<K, PH_CG_B>();
+    case PH_BI_P: return red_parts<K, PH_BI_P>();
+    case PH_BI_S: return red_parts<K, PH_BI_S>();
+    default: return red_parts<K, PH_BI_X>();
+  }
+}
+
 const void* pick_reduce(int k, int ph) {
   switch (k) {
     case 1: return reduce_fn<1>(ph);
@@ -865,6 +983,7 @@ struct StreamPlan {
   int* d_blk_end = nullptr;
   int* d_inst_blk = nullptr;
   double* d_partials = nullptr;
+  double* d_sums = nullptr;
   int* d_act_inst = nullptr;  // [ninst]
   int* d_act_base = nullptr;  // [ninst]
   int* d_act_blk = nullptr;   // [nblocks]
@@ -879,7 +998,7 @@ struct StreamPlan {
 void stream_plan_free(StreamPlan* p) {
   if (!p) return;
   void* ptrs[] = {p->d_ss,       p->d_blk_inst, p->d_blk_row,  p->d_blk_end, p->d_inst_blk,
-                  p->d_partials, p->d_act_inst, p->d_act_base, p->d_act_blk,  p->d_cnt};
+                  p->d_partials, p->d_sums,     p->d_act_inst, p->d_act_base, p->d_act_blk,  p->d_cnt};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   if (p->h_post) (void)hipHostFree(p->h_post);
@@ -949,6 +1068,7 @@ int stream_plan_build(const std::vector<InstHost>& insts, const Inst* d_insts, i
   p->d_blk_end = dalloc<int>(std::max(1, p->nblocks), &rc);
   p->d_inst_blk = dalloc<int>(p->ninst + 1, &rc);
   p->d_partials = dalloc<double>((size_t)std::max(1, p->nblocks) * kPartW * k, &rc);
+  p->d_sums = dalloc<double>((size_t)p->ninst * kPartW * k, &rc);
   p->d_act_inst = dalloc<int>(p->ninst, &rc);
   p->d_act_base = dalloc<int>(p->ninst, &rc);
   p->d_act_blk = dalloc<int>(std::max(1, p->nblocks), &rc);
@@ -1023,7 +1143,8 @@ int launch_phase(const StreamPlan* p, const SArgs& a, int ph, const Cover& cv, h
   const int* ib = p->d_inst_blk;
   int fp32 = p->fp32;
   void* rargs[] = {(void*)&aa, (void*)&ib, (void*)&nact, (void*)&fp32};
-  FEM_HIP(hipLaunchKernel(rf, dim3(nact), dim3(kRedBlock), rargs, 0, st));
+  const int parts = p->k == 16 ? reduce_parts<16>(ph) : 1;
+  FEM_HIP(hipLaunchKernel(rf, dim3(nact * parts), dim3(kRedBlock), rargs, 0, st));
   return 0;
 }
 
@@ -1045,10 +1166,19 @@ int post_read(const StreamPlan* p, const int* src, int nvals, int slot, hipStrea
 }
 
 // Compact the instances and row blocks that satisfy `pred` into the device
-// lists (k_compact, k_expand).  post >= 0: also queue the read of the lists'
-// counts into that pinned slot (read back by wait_counts).  The launch sizes
+// lists (k_lists, or k_compact and k_expand).  post >= 0: also queue the read
+// of the lists' counts into that pinned slot (wait_counts).  The launch sizes
 // in *cv are left as they are: a superset.
 int compact(const StreamPlan* p, int pred, hipStream_t st, Cover* cv, int post = -1) {
+  cv->all = false;
+  if (p->ninst <= kListInsts) {
+    const unsigned seq = post >= 0 ? claim_slot(p, post, 2) : 0;
+    hipLaunchKernelGGL(k_lists, dim3(std::max(1u, div_up(p->nblocks, kBlock))), dim3(kBlock), 0, st, p->d_ss,
+                       p->d_inst_blk, p->d_blk_inst, p->ninst, p->nblocks, pred, p->d_act_inst, p->d_act_blk, p->d_cnt,
+                       post >= 0 ? p->d_post + kPostWords * post : nullptr, seq);
+    FEM_HIP(hipGetLastError());
+    return 0;
+  }
   hipLaunchKernelGGL(k_compact, dim3(1), dim3(kBlock), 0, st, p->d_ss, p->d_inst_blk, p->ninst, pred, p->d_act_inst,
                      p->d_act_base, p->d_cnt);
   FEM_HIP(hipGetLastError());
@@ -1061,7 +1191,6 @@ int compact(const StreamPlan* p, int pred, hipStream_t st, Cover* cv, int post =
                        p->d_act_base, p->nblocks, p->d_act_blk);
     FEM_HIP(hipGetLastError());
   }
-  cv->all = false;
   return 0;
 }
 
@@ -1144,6 +1273,7 @@ int stream_run(const StreamPlan* p, const Inst* d_insts, int max_sweeps, int max
   a.rhs_stage = p->lds_rhs > 0;
   a.res_stage = p->lds_res > 0;
   a.partials = p->d_partials;
+  a.sums = p->d_sums;
   hipLaunchKernelGGL(k_hist_load, dim3(div_up(p->ninst, kBlock)), dim3(kBlock), 0, st, const_cast<Inst*>(d_insts),
                      p->ninst);
   hipLaunchKernelGGL(k_sinit, dim3(div_up(p->ninst, kBlock)), dim3(kBlock), 0, st, p->d_ss, d_insts, p->ninst);
@@ -1221,7 +1351,9 @@ int stream_run(const StreamPlan* p, const Inst* d_insts, int max_sweeps, int max
       };
       // one iteration queued: refresh the lists (several instances), take
       // the counts read after the previous iteration, and every
-      // kCheckEvery-th time queue another read (budgeted: refresh only)
+      // kCheckEvery-th time queue another read (budgeted: refresh only).  A
+      // refresh every fourth iteration alone saves its launch but leaves the
+      // finished instances' blocks in the others: no faster.
       int since = 0, it_run = 0, pend = -1, pend_it = 0, need = 0;
       const int expect = sw < (int)prev_its.size() ? prev_its[sw] : 0;
       // before an iteration's launches: whether it ends with a read (the slot,
