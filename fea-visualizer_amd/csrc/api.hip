@@ -476,7 +476,8 @@ int fem_solver_smooth_normals(fem_solver* s, const float* normals_nv3, float ext
     const size_t nv = (size_t)c->nv;
     if (nv == 0) return FEM_OK;
     int rc = 0;
-    float* d = dalloc<float>(7 * nv, &rc);
+    float*& d = b->insts[0].d_normals;  // kept: a viewer asks every frame
+    if (!d) d = dalloc<float>(7 * nv, &rc);
     if (!d) return rc;
     float *dn = d, *dv = d + 3 * nv, *dout = d + 4 * nv;
     hipError_t e = hipMemcpyAsync(dn, normals_nv3, sizeof(float) * 3 * nv, hipMemcpyHostToDevice, b->stream);
@@ -486,7 +487,6 @@ int fem_solver_smooth_normals(fem_solver* s, const float* normals_nv3, float ext
       if (!rc) e = hipMemcpyAsync(out_nv3, dout, sizeof(float) * 3 * nv, hipMemcpyDeviceToHost, b->stream);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    (void)hipFree(d);
     if (e != hipSuccess) return hip_fail(e, "fem_solver_smooth_normals");
     return rc;
   })

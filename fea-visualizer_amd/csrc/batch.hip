@@ -202,10 +202,20 @@ __global__ void k_get_cols(const double* src, int k, int col0, double* dst, int 
   dst[i] = src[r * k + col0 + j];
 }
 
+// A new instance's vectors and outcome record cleared in one launch: ten
+// memsets, most of a few KB, took 50 us of a one-off solve.
+__global__ void __launch_bounds__(kBlock) k_clear_inst(double* u, double* v, double* a, double* x, double* b,
+                                                       long long n, float* vec, long long nvec, int* info) {
+  const long long step = (long long)gridDim.x * kBlock, t = (long long)blockIdx.x * kBlock + threadIdx.x;
+  for (long long i = t; i < n; i += step) u[i] = v[i] = a[i] = x[i] = b[i] = 0.0;
+  for (long long i = t; i < nvec; i += step) vec[i] = 0.0f;
+  if (t < (long long)(kInfoBytes / sizeof(int))) info[t] = 0;
+}
+
 void free_inst(InstHost& h) {
   void* ptrs[] = {h.d_S64, h.d_Si,    h.d_dinv64, h.d_dinvi, h.d_SDi, h.d_u, h.d_v,   h.d_a,
                   h.d_h3,  h.d_h4,    h.d_xnext,  h.d_hpre,  h.d_hvec, h.d_x, h.d_b, h.d_vec,
-                  h.d_surf, h.d_h5, h.d_h6, h.d_xch};
+                  h.d_surf, h.d_h5, h.d_h6, h.d_xch, h.d_normals};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (h.surf_done) (void)hipEventSynchronize(h.surf_done);
@@ -219,6 +229,17 @@ void free_inst(InstHost& h) {
 }
 
 size_t inner_bytes(const fem_batch* b) { return b->opts.precision == FEM_PREC_FP32_IR ? 4 : 8; }
+
+// Staging of the surface-space state calls.
+int alloc_surface(InstHost& h) {
+  int rc = 0;
+  const size_t len = std::max<size_t>(1, (size_t)h.ctx->nv * h.k);
+  if (!h.d_surf) h.d_surf = dalloc<float>(len, &rc);
+  if (rc) return rc;
+  if (!h.h_surf) FEM_HIP(hipHostMalloc((void**)&h.h_surf, sizeof(float) * len, hipHostMallocDefault));
+  if (!h.surf_done) FEM_HIP(hipEventCreateWithFlags(&h.surf_done, hipEventDisableTiming));
+  return 0;
+}
 
 int alloc_inst(fem_batch* b, InstHost& h, int k, int kv) {
   free_inst(h);
@@ -238,30 +259,20 @@ int alloc_inst(fem_batch* b, InstHost& h, int k, int kv) {
   h.d_x = dalloc<double>((size_t)n * k, &rc);
   h.d_b = dalloc<double>((size_t)n * k, &rc);
   h.d_vec = (void*)dalloc<char>((size_t)n * k * tb * 11, &rc);
-  h.d_surf = dalloc<float>((size_t)h.ctx->nv * k, &rc);
   if (rc) return rc;
   char* info = b->d_info + (size_t)(&h - b->insts.data()) * kInfoBytes;
   h.d_counters = (long long*)info;
   h.d_status = (int*)(info + kInfoStatus);
   h.d_last_res = (double*)(info + kInfoLastRes);
   h.d_hist = (int*)(info + kInfoHist);
-  {
-    hipError_t e = hipHostMalloc((void**)&h.h_surf, sizeof(float) * std::max<size_t>(1, (size_t)h.ctx->nv * k),
-                                 hipHostMallocDefault);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&h.surf_done, hipEventDisableTiming);
-    if (e != hipSuccess) return hip_fail(e, "alloc_inst: surface staging");
+  if (!b->once) {  // a one-off solve has no surface state
+    rc = alloc_surface(h);
+    if (rc) return rc;
   }
-  const size_t vb = (size_t)n * k * sizeof(double);
-  FEM_HIP(hipMemsetAsync(h.d_u, 0, vb, b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_v, 0, vb, b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_a, 0, vb, b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_x, 0, vb, b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_b, 0, vb, b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_vec, 0, (size_t)n * k * tb * 11, b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_status, 0, 4 * sizeof(int), b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_counters, 0, 4 * sizeof(long long), b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_last_res, 0, kMaxK * sizeof(double), b->stream));
-  FEM_HIP(hipMemsetAsync(h.d_hist, 0, sizeof(int), b->stream));
+  const long long nk = n * k, nvec = (long long)(nk * tb * 11 / sizeof(float));
+  hipLaunchKernelGGL(k_clear_inst, dim3(std::min(2048u, std::max(1u, div_up(nvec, kBlock)))), dim3(kBlock), 0,
+                     b->stream, h.d_u, h.d_v, h.d_a, h.d_x, h.d_b, nk, (float*)h.d_vec, nvec, (int*)info);
+  FEM_HIP(hipGetLastError());
   h.dirty = true;
   return 0;
 }
@@ -414,10 +425,10 @@ void fill_dev(fem_batch* b, InstHost& h) {
 }
 
 void free_plan(fem_batch* b) {
-  void* ptrs[] = {b->d_insts, b->d_teams, b->d_wg_team, b->d_team_inst, b->d_slots, b->d_halo,
-                  b->d_halo_mem};
+  void* ptrs[] = {b->d_plan, b->d_slots, b->d_halo_mem};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  b->d_plan = nullptr;
   b->d_insts = nullptr;
   b->d_teams = nullptr;
   b->d_wg_team = nullptr;
@@ -703,15 +714,27 @@ int build_plan(fem_batch* b) {
     ht[t].inst_end = (int)team_inst.size();
     for (int q = 0; q < sizes[t]; q++) wg_team[wg++] = t;
   }
-  b->d_insts = dalloc<Inst>(ninst, &rc);
-  b->d_teams = dalloc<Team>(nteams, &rc);
-  b->d_wg_team = dalloc<int>(grid, &rc);
-  b->d_team_inst = dalloc<int>(team_inst.size(), &rc);
+  // the plan's tables in one block, sent in one copy
+  size_t plan_bytes = 0;
+  auto place = [&](size_t bytes) {
+    const size_t at = plan_bytes;
+    plan_bytes += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t nlist = team_inst.size();
+  const size_t o_insts = place(sizeof(Inst) * ninst), o_teams = place(sizeof(Team) * nteams);
+  const size_t o_wg = place(sizeof(int) * grid), o_list = place(sizeof(int) * nlist);
+  const size_t o_halo = place(sizeof(HaloRef) * nlist);
+  b->d_plan = dalloc<char>(plan_bytes, &rc);
   b->d_slots = dalloc<double>(slot_bytes(grid, k) / sizeof(double), &rc);
   if (rc) return rc;
+  b->d_insts = (Inst*)(b->d_plan + o_insts);
+  b->d_teams = (Team*)(b->d_plan + o_teams);
+  b->d_wg_team = (int*)(b->d_plan + o_wg);
+  b->d_team_inst = (int*)(b->d_plan + o_list);
   // halos of the teams whose workgroups keep their rows in LDS
-  std::vector<HaloRef> halo(team_inst.size());
-  std::vector<HaloShape> shape(team_inst.size());
+  std::vector<HaloRef> halo(nlist);
+  std::vector<HaloShape> shape(nlist);
   size_t halo_bytes = 0;
   for (int t = 0; t < nteams; t++)
     for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++)
@@ -720,25 +743,41 @@ int build_plan(fem_batch* b) {
       else
         shape[q].cap = 0;
   if (halo_bytes > 0) {
-    b->d_halo = dalloc<HaloRef>(halo.size(), &rc);
+    b->d_halo = (HaloRef*)(b->d_plan + o_halo);
     b->d_halo_mem = dalloc<char>(halo_bytes, &rc);
     if (rc) return rc;
     size_t at = 0;
-    for (size_t q = 0; q < halo.size(); q++) {
+    for (size_t q = 0; q < nlist; q++) {
       if (shape[q].cap == 0) continue;
       halo[q] = halo_ref(shape[q], b->d_halo_mem + at);
       at += shape[q].n_bytes + shape[q].list_bytes + shape[q].place_bytes;
     }
-    const size_t bytes = sizeof(HaloRef) * halo.size();
-    FEM_HIP(hipMemcpyAsync(b->d_halo, halo.data(), bytes, hipMemcpyHostToDevice, b->stream));
+  }
+  for (int t = 0; t < nteams; t++) {
+    ht[t].halo = b->d_halo;
+    team_slots(&ht[t], b->d_slots, grid, k);
+    ht[t].abort_flag = b->d_abort;
+    ht[t].wait_ticks = b->wait_ticks;
+    ht[t].allpoll = b->poll_override == 1 ? 1 : b->poll_override == 2 ? 0 : flat_reduction(sizes[t], k);
+  }
+  std::vector<Inst> hi(ninst);
+  for (int i = 0; i < ninst; i++) hi[i] = persistent_desc(b->insts[i].dev);
+  std::vector<char> host(plan_bytes);
+  std::memcpy(&host[o_insts], hi.data(), sizeof(Inst) * ninst);
+  std::memcpy(&host[o_teams], ht.data(), sizeof(Team) * nteams);
+  std::memcpy(&host[o_wg], wg_team.data(), sizeof(int) * grid);
+  std::memcpy(&host[o_list], team_inst.data(), sizeof(int) * nlist);
+  std::memcpy(&host[o_halo], halo.data(), sizeof(HaloRef) * nlist);
+  FEM_HIP(hipMemcpyAsync(b->d_plan, host.data(), plan_bytes, hipMemcpyHostToDevice, b->stream));
+  if (b->d_halo) {  // built on the device, which says which fit
     for (int t = 0; t < nteams; t++)
       for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++)
         if (shape[q].cap > 0 &&
             (rc = launch_halo(b->insts[team_inst[q]].ctx, k, sizes[t], shape[q], halo[q], b->d_halo + q, b->stream)))
           return rc;
-    FEM_HIP(hipMemcpyAsync(halo.data(), b->d_halo, bytes, hipMemcpyDeviceToHost, b->stream));
-    FEM_HIP(hipStreamSynchronize(b->stream));
+    FEM_HIP(hipMemcpyAsync(halo.data(), b->d_halo, sizeof(HaloRef) * nlist, hipMemcpyDeviceToHost, b->stream));
   }
+  FEM_HIP(hipStreamSynchronize(b->stream));
   // Whether any instance keeps its rows in LDS (the kernel variant), and the
   // exchange mode: teams of several workgroups with more rows than the row
   // cache holds stream their phases: fenced barriers.  Plans of one-workgroup teams run the plain
@@ -755,22 +794,7 @@ int build_plan(fem_batch* b) {
     set_error("team plan exceeds the co-resident grid");
     return FEM_ERR_INVALID;
   }
-  for (int t = 0; t < nteams; t++) {
-    ht[t].halo = b->d_halo;
-    team_slots(&ht[t], b->d_slots, grid, k);
-    ht[t].abort_flag = b->d_abort;
-    ht[t].wait_ticks = b->wait_ticks;
-    ht[t].allpoll = b->poll_override == 1 ? 1 : b->poll_override == 2 ? 0 : flat_reduction(sizes[t], k);
-  }
-  std::vector<Inst> hi(ninst);
-  for (int i = 0; i < ninst; i++) hi[i] = persistent_desc(b->insts[i].dev);
-  FEM_HIP(hipMemcpyAsync(b->d_insts, hi.data(), sizeof(Inst) * ninst, hipMemcpyHostToDevice, b->stream));
   b->uploaded = hi;
-  FEM_HIP(hipMemcpyAsync(b->d_teams, ht.data(), sizeof(Team) * nteams, hipMemcpyHostToDevice, b->stream));
-  FEM_HIP(hipMemcpyAsync(b->d_wg_team, wg_team.data(), sizeof(int) * grid, hipMemcpyHostToDevice, b->stream));
-  FEM_HIP(hipMemcpyAsync(b->d_team_inst, team_inst.data(), sizeof(int) * team_inst.size(), hipMemcpyHostToDevice,
-                         b->stream));
-  FEM_HIP(hipStreamSynchronize(b->stream));
   b->launch.teams = b->d_teams;
   b->launch.wg_team = b->d_wg_team;
   b->launch.insts = b->d_insts;
@@ -803,12 +827,19 @@ void batch_free(fem_batch* b) {
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->d_info) (void)hipFree(b->d_info);
-  if (b->h_info) (void)hipHostFree(b->h_info);
-  if (b->stream) (void)hipStreamDestroy(b->stream);
+  if (b->once) {
+    delete[] b->h_info;
+  } else {
+    if (b->h_info) (void)hipHostFree(b->h_info);
+    if (b->stream) (void)hipStreamDestroy(b->stream);
+  }
   delete b;
 }
 
-int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, fem_batch** out) {
+// once: the batch serves one call and is then freed.  It runs on its (only)
+// context's stream and reads its outcome into pageable memory: making and
+// freeing a stream and pinned memory took 200 us of a one-off solve.
+int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, fem_batch** out, bool once) {
   if (count <= 0 || !ctxs) {
     set_error("batch_create: no contexts");
     return FEM_ERR_INVALID;
@@ -835,7 +866,10 @@ int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, f
     return FEM_ERR_INVALID;
   }
   b->nrhs = nr;
-  hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
+  b->once = once && ctxs[0];
+  hipError_t e = hipSuccess;
+  if (b->once) b->stream = ctxs[0]->stream;
+  else e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&b->ev0);
   if (e == hipSuccess) e = hipEventCreate(&b->ev1);
   if (e != hipSuccess) {
@@ -849,7 +883,9 @@ int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, f
   {
     int rc = 0;
     b->d_info = dalloc<char>(b->info_bytes, &rc);
-    if (!rc) {
+    if (!rc && b->once) {
+      b->h_info = new char[b->info_bytes];
+    } else if (!rc) {
       e = hipHostMalloc((void**)&b->h_info, b->info_bytes, hipHostMallocDefault);
       if (e != hipSuccess) rc = hip_fail(e, "batch_create: hipHostMalloc");
     }
@@ -1008,17 +1044,15 @@ int batch_set_linear(fem_batch* b, int inst, const double coef[3]) {
 int linear_solve(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
                  fem_step_stats* stats) {
   fem_batch* b = nullptr;
-  int rc = batch_create(&c, 1, opts, &b);
+  int rc = batch_create(&c, 1, opts, &b, true);
   if (rc) return rc;
   rc = batch_set_linear(b, 0, coef);
   InstHost& h = b->insts[0];
   const size_t bytes = sizeof(double) * (size_t)c->n * b->nrhs;
   if (!rc && c->n > 0) {
     hipError_t e = hipMemcpyAsync(h.d_b, bh, bytes, hipMemcpyHostToDevice, b->stream);
-    if (e == hipSuccess)
-      e = b->opts.warm_start ? hipMemcpyAsync(h.d_x, xh, bytes, hipMemcpyHostToDevice, b->stream)
-                             : hipMemsetAsync(h.d_x, 0, bytes, b->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+    if (e == hipSuccess && b->opts.warm_start)  // else x is zero from its allocation
+      e = hipMemcpyAsync(h.d_x, xh, bytes, hipMemcpyHostToDevice, b->stream);
     if (e != hipSuccess) rc = hip_fail(e, "linear_solve: upload");
   }
   int out = rc;
@@ -1185,6 +1219,8 @@ int batch_set_surface(fem_batch* b, int inst, int field, const float* values_nv)
   InstHost& h = b->insts[inst];
   fem_ctx* c = h.ctx;
   if (c->nv == 0) return 0;
+  rc = alloc_surface(h);
+  if (rc) return rc;
   // the values go through pinned staging, so the call returns without waiting
   // for the device: the previous upload from the staging must have completed
   FEM_HIP(hipEventSynchronize(h.surf_done));
@@ -1205,6 +1241,8 @@ int batch_get_surface(fem_batch* b, int inst, int field, float* values_nv) {
   InstHost& h = b->insts[inst];
   fem_ctx* c = h.ctx;
   if (c->nv == 0) return 0;
+  rc = alloc_surface(h);
+  if (rc) return rc;
   hipLaunchKernelGGL(k_surface_scatter, dim3(div_up(c->nv, kBlock)), dim3(kBlock), 0, b->stream, c->d_idx, c->nv,
                      d, h.k, col, nc, h.d_surf);
   FEM_HIP(hipGetLastError());

@@ -25,8 +25,9 @@ struct fem_ctx {
   double* d_M = nullptr;
   double* d_A = nullptr;
   double* d_lumped = nullptr; // row sums of M
-  double* d_kappa_e = nullptr;
+  double* d_kappa_e = nullptr;  // coefficients of the last assembly that had any, kept for the next
   double* d_vel_e = nullptr;
+  char* d_slabs[2] = {nullptr, nullptr};  // all of the above but these two: mesh and rows, entries
   std::vector<int> h_rp;
 };
 

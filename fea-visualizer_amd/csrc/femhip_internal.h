@@ -215,6 +215,7 @@ inline T* dalloc(size_t count, int* rc) {
 inline unsigned int div_up(long long a, long long b) { return (unsigned int)((a + b - 1) / b); }
 
 // Device exclusive scan (int32 -> int32 offsets, total returned), scan.hip.
-int exclusive_scan_i32(const int* in, int* out, int n, int* total, hipStream_t st);
+int scan_scratch(int n);
+int exclusive_scan_i32(const int* in, int* out, int n, int* scratch, hipStream_t st);
 
 }  // namespace femhip

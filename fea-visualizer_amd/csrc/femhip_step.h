@@ -118,9 +118,10 @@ struct InstHost {
   long long* d_counters = nullptr;
   double* d_last_res = nullptr;
   int* d_hist = nullptr;     // predictor history levels held (Inst::hist_dev), in the info block
-  float* d_surf = nullptr;   // surface-space staging of set_state / get_state [nv][k]
+  float* d_surf = nullptr;   // surface-space staging of set_state / get_state [nv][k], made when first used
   float* h_surf = nullptr;   // pinned host staging of set_state's values [nv][k]
   hipEvent_t surf_done = nullptr;  // the last upload from h_surf has completed
+  float* d_normals = nullptr;      // smooth_normals: normals, values, output [7 nv], made when first used
   Inst dev{};                // mirror of the device descriptor
 };
 
@@ -139,9 +140,11 @@ struct fem_batch {
   fem_solver_opts opts{};
   int nrhs = 1;
   hipStream_t stream = nullptr;
+  bool once = false;  // serves one call: its context's stream, pageable h_info
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // launch plan (device arrays)
+  // launch plan: device arrays in d_plan, except the barrier records and the halo tables
   bool plan_ready = false;
+  char* d_plan = nullptr;
   femhip::StepLaunch launch;
   femhip::Inst* d_insts = nullptr;
   femhip::Team* d_teams = nullptr;
@@ -153,7 +156,7 @@ struct fem_batch {
   int grid = 0;
   int* d_abort = nullptr;       // in the info block
   char* d_info = nullptr;       // [ninst][kInfoBytes] + abort flag
-  char* h_info = nullptr;       // pinned host copy
+  char* h_info = nullptr;       // host copy, pinned unless once
   size_t info_bytes = 0;
   std::vector<femhip::Inst> uploaded;  // descriptors last copied to the plan's d_insts
   int nteams = 0;
@@ -197,7 +200,7 @@ struct fem_solver {
 };
 
 namespace femhip {
-int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, fem_batch** out);
+int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, fem_batch** out, bool once = false);
 void batch_free(fem_batch* b);
 int batch_set_equation(fem_batch* b, int inst, int equation, const void* params, size_t size);
 int batch_set_state_unknowns(fem_batch* b, int inst, int field, const double* x);

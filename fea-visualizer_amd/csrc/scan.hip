@@ -76,22 +76,17 @@ __global__ void __launch_bounds__(kBlock) k_tile_scan(const int* in, int n, cons
 
 }  // namespace
 
-// out[i] = sum_{j<i} in[i]; out may alias in.  *total receives the grand
-// total (host value, synchronous on `st`).
-int exclusive_scan_i32(const int* in, int* out, int n, int* total, hipStream_t st) {
-  int rc = 0;
-  int tiles = (int)div_up(n > 0 ? n : 1, kTile);
-  int* sums = dalloc<int>((size_t)tiles + 1, &rc);
-  if (!sums) return rc;
-  int* dtot = sums + tiles;
-  hipLaunchKernelGGL(k_tile_sums, dim3(tiles), dim3(kBlock), 0, st, in, n, sums);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kBlock), 0, st, sums, tiles, dtot);
-  hipLaunchKernelGGL(k_tile_scan, dim3(tiles), dim3(kBlock), 0, st, in, n, sums, out);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(total, dtot, sizeof(int), hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  (void)hipFree(sums);
-  if (e != hipSuccess) return hip_fail(e, "exclusive_scan_i32");
+// Ints of scratch a scan of n values needs.
+int scan_scratch(int n) { return (int)div_up(n > 0 ? n : 1, kTile) + 1; }
+
+// out[i] = sum_{j<i} in[i] on `st`; out may alias in.  scratch: device memory
+// of scan_scratch(n) ints, free again once the stream has passed the scan.
+int exclusive_scan_i32(const int* in, int* out, int n, int* scratch, hipStream_t st) {
+  const int tiles = scan_scratch(n) - 1;
+  hipLaunchKernelGGL(k_tile_sums, dim3(tiles), dim3(kBlock), 0, st, in, n, scratch);
+  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kBlock), 0, st, scratch, tiles, scratch + tiles);
+  hipLaunchKernelGGL(k_tile_scan, dim3(tiles), dim3(kBlock), 0, st, in, n, scratch, out);
+  FEM_HIP(hipGetLastError());
   return 0;
 }
 

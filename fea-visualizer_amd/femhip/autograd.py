@@ -6,9 +6,8 @@ checkpoint-and-recompute, fem_adjoint_* in include/femhip.h).  The forward is
 the backward-Euler heat / advection-diffusion step of the reference
 (CPUSolver.cpp:72-102) with the stiffness assembled per element as
 K = sum_e kappa_e K_e.  GPU tensors stay on the device: their pointers cross
-the C ABI (fem_adjoint_forward_device / _backward_device); only a changed
-kappa_e comes to the host, once, for the re-assembly.  CPU tensors cross as
-host float64 arrays.  The arithmetic runs in the HIP library either way.
+the C ABI (fem_adjoint_forward_device / _backward_device, fem_ctx_assemble).
+CPU tensors cross as host float64 arrays.  The arithmetic runs in the HIP library either way.
 """
 from __future__ import annotations
 
@@ -69,9 +68,15 @@ class Rollout:
     def _assemble(self, kappa_e: torch.Tensor):
         k = kappa_e.detach()
         if self._kappa is None or self._kappa.device != k.device or not torch.equal(self._kappa, k):
-            self.ctx.assemble_matrices(self.velocity, self.velocity_e, self.normalize,
-                                       k.to(device="cpu", dtype=torch.float64).numpy())
-            self._kappa = k.clone()
+            own = k.clone()
+            if k.is_cuda and k.numel() == self.ntri and len(L.hip_runtimes()) == 1:  # read where it is
+                d = own.to(torch.float64).contiguous()
+                torch.cuda.current_stream(d.device).synchronize()  # the library reads on its own stream
+                self.ctx._assemble(self.velocity, self.velocity_e, self.normalize, kappa_ptr=d.data_ptr())
+            else:
+                self.ctx.assemble_matrices(self.velocity, self.velocity_e, self.normalize,
+                                           k.to(device="cpu", dtype=torch.float64).numpy())
+            self._kappa = own
 
     @staticmethod
     def _check_one_runtime():

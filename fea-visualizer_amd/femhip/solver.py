@@ -182,6 +182,10 @@ class FEMContext:
 
     def assemble_matrices(self, velocity=None, velocity_e=None, normalize_velocity=True, kappa_e=None):
         """FEMContext::assemble_matrices (FEMContext.cpp:57-64) on the GPU."""
+        self._assemble(velocity, velocity_e, normalize_velocity, kappa_e)
+
+    def _assemble(self, velocity, velocity_e, normalize_velocity, kappa_e=None, kappa_ptr=0):
+        """kappa_ptr: the diffusivities in device memory (float64, one per triangle) instead of kappa_e."""
         if velocity is None:
             velocity = self.parameters[Equation.Advection_Diffusion].velocity
         p = L.fem_assembly_params()
@@ -196,6 +200,8 @@ class FEMContext:
             ke = np.ascontiguousarray(kappa_e, dtype=np.float64).reshape(-1)
             self._keep["ke"] = ke
             p.kappa_e = L.ptr(ke, C.c_double)
+        if kappa_ptr:
+            p.kappa_e = C.cast(C.c_void_p(kappa_ptr), C.POINTER(C.c_double))
         L.check(self._lib.fem_ctx_assemble(self.handle, C.byref(p)))
 
     def info(self):

@@ -93,7 +93,8 @@ typedef struct fem_assembly_params {
   double velocity[3];          /* constant velocity */
   const double* velocity_e;    /* optional: 3 per triangle (overrides velocity) */
   int32_t normalize_velocity;  /* 1 = reference (unit tangential velocity, FEMContext.cpp:180) */
-  const double* kappa_e;       /* optional: per-triangle diffusivity multiplying K */
+  const double* kappa_e;       /* optional: per-triangle diffusivity multiplying K, in
+                                * host or device memory */
 } fem_assembly_params;
 
 /* Equation parameters: EquationParameters.hpp:4-49 (widened to double). */
