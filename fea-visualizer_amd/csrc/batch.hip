@@ -258,7 +258,7 @@ int alloc_inst(fem_batch* b, InstHost& h, int k, int kv) {
   h.d_a = dalloc<double>((size_t)n * k, &rc);
   h.d_x = dalloc<double>((size_t)n * k, &rc);
   h.d_b = dalloc<double>((size_t)n * k, &rc);
-  h.d_vec = (void*)dalloc<char>((size_t)n * k * tb * 11, &rc);
+  h.d_vec = (void*)dalloc<char>((size_t)n * k * tb * 11 + 16, &rc);  // 16: packed_rows' alignment
   if (rc) return rc;
   char* info = b->d_info + (size_t)(&h - b->insts.data()) * kInfoBytes;
   h.d_counters = (long long*)info;

@@ -249,6 +249,10 @@ __device__ void run_vector(const Inst& I, const SArgs& a, Shared& sh, int b, int
       vphase_res<K, V, TI, true>(I, row_lo, row_hi, sh, acc, rs);
     else
       vphase_res<K, V, TI>(I, row_lo, row_hi, sh, acc);
+  } else if constexpr (PH == PH_PCG_INIT && K == 1) {
+    vphase_pcg_init_packed<TI>(I, row_lo, row_hi, g, packed_rows<TI>(I, 0), acc);
+  } else if constexpr (PH == PH_PCG_ITER && K == 1) {
+    vphase_pcg_iter_packed<TI>(I, row_lo, row_hi, g, packed_rows<TI>(I, par), packed_rows<TI>(I, par ^ 1), sh, acc);
   } else if constexpr (PH == PH_PCG_INIT) {
     vphase_pcg_init<K, V, TI>(I, row_lo, row_hi, g, (TI*)I.r, (TI*)I.q, acc);
   } else if constexpr (PH == PH_PCG_ITER) {
@@ -337,20 +341,16 @@ __global__ void __launch_bounds__(kBlock) k_sphase(SArgs a) {
         phase_update<K, TI, kPlain>(I, row_lo, row_hi, sh, I.status, a.step, lvn);
     } else if constexpr (vec_layout<K>() && staged_phase<PH>()) {
       // stage the block's pattern: row pointers, columns, S D^-1 (phase A of classic CG: S)
-      extern __shared__ int dyn[];
+      extern __shared__ __attribute__((aligned(16))) int dyn[];
       const int GA* rp = gp(I.rp);
-      const int s_lo = rp[row_lo], s_hi = rp[row_hi];
-      const int nrow = row_hi - row_lo, nnz = s_hi - s_lo;  // within the stage (plan)
+      const int base = rp[row_lo] & ~3, s_hi = rp[row_hi];
+      const int nrow = row_hi - row_lo;  // rows and entries are within the stage (plan)
       int LA* lrp = (int LA*)dyn;
       int LA* lci = lrp + ((a.stage_rows + 4) & ~3);
-      TI LA* lw = (TI LA*)(lci + ((a.stage_nnz + 3) & ~3));
-      const int GA* ci = gp(I.ci);
-      const TI GA* w = gp((const TI*)(PH == PH_CG_A ? I.Si : I.SDi));
-      for (int t = threadIdx.x; t <= nrow; t += kBlock) lrp[t] = rp[row_lo + t] - s_lo;
-      for (int t = threadIdx.x; t < nnz; t += kBlock) {
-        lci[t] = ci[s_lo + t];
-        lw[t] = w[s_lo + t];
-      }
+      TI LA* lw = (TI LA*)(lci + a.stage_nnz);
+      for (int t = threadIdx.x; t <= nrow; t += kBlock) lrp[t] = rp[row_lo + t] - base;
+      stage_entries<TI, false>(gp(I.ci), gp((const TI*)(PH == PH_CG_A ? I.Si : I.SDi)), nullptr, base, s_hi, I.nnz, lci,
+                               lw, nullptr);
       __syncthreads();
       run_vector<K, V, TI, PH>(I, a, sh, b, row_lo, row_hi, Stage<TI>{lrp, lci, lw, row_lo});
     } else if constexpr (vec_layout<K>() && (PH == PH_RHS || PH == PH_RES)) {
@@ -361,21 +361,18 @@ __global__ void __launch_bounds__(kBlock) k_sphase(SArgs a) {
       if (rcase) {
         extern __shared__ __attribute__((aligned(16))) int dyn[];
         const int GA* rp = gp(I.rp);
-        const int s_lo = rp[row_lo], s_hi = rp[row_hi];
-        const int nrow = row_hi - row_lo, nnz = s_hi - s_lo;  // within the stage (plan)
+        const int base = rp[row_lo] & ~3, s_hi = rp[row_hi];
+        const int nrow = row_hi - row_lo;  // rows and entries are within the stage (plan)
         int LA* lrp = (int LA*)dyn;
         int LA* lci = lrp + ((a.stage_rows + 4) & ~3);
-        double LA* la = (double LA*)(lci + ((a.stage_nnz + 3) & ~3));
+        double LA* la = (double LA*)(lci + a.stage_nnz);
         double LA* ls = la + a.stage_nnz;
-        const int GA* ci = gp(I.ci);
-        const double GA* wa = gp(rcase == 1 ? I.K64 : rcase == 2 ? I.M64 : I.S64);
-        const double GA* ws = gp(I.S64);
-        for (int t = threadIdx.x; t <= nrow; t += kBlock) lrp[t] = rp[row_lo + t] - s_lo;
-        for (int t = threadIdx.x; t < nnz; t += kBlock) {
-          lci[t] = ci[s_lo + t];
-          la[t] = wa[s_lo + t];
-          if (rcase != 3) ls[t] = ws[s_lo + t];
-        }
+        for (int t = threadIdx.x; t <= nrow; t += kBlock) lrp[t] = rp[row_lo + t] - base;
+        if constexpr (PH == PH_RES)
+          stage_entries<double, false>(gp(I.ci), gp(I.S64), nullptr, base, s_hi, I.nnz, lci, la, nullptr);
+        else
+          stage_entries<double, true>(gp(I.ci), gp(rcase == 1 ? I.K64 : I.M64), gp(I.S64), base, s_hi, I.nnz, lci, la,
+                                      ls);
         __syncthreads();
         run_vector<K, V, TI, PH>(I, a, sh, b, row_lo, row_hi, Stage<TI>{}, rcase, RhsStage{lrp, lci, la, ls});
       } else {
@@ -1021,7 +1018,6 @@ int stream_plan_build(const std::vector<InstHost>& insts, const Inst* d_insts, i
   p->kr = kr;
   p->rows = rows;
   std::vector<int> bi, br, be, ib(p->ninst + 1, 0);
-  double s_bytes = 0.0;  // FP64 S rows of all instances
   for (int i = 0; i < p->ninst; i++) {
     ib[i] = (int)bi.size();
     const fem_ctx* c = insts[i].ctx;
@@ -1042,25 +1038,30 @@ int stream_plan_build(const std::vector<InstHost>& insts, const Inst* d_insts, i
       p->stage_nnz = std::max(p->stage_nnz, rp[e] - rp[r]);
       r = e;
     }
-    s_bytes += 8.0 * rp[n];
   }
   ib[p->ninst] = (int)bi.size();
   p->nblocks = (int)bi.size();
+  // dynamic LDS of a stage that holds `nnz` entries of `bytes` bytes of values
+  // each; the limits are on the entries, the launches carry the slack of the
+  // aligned start (stage_entries) on top
+  auto stage = [&](int nnz, size_t bytes) {
+    return 4 * (size_t)((p->stage_rows + 4) & ~3) + 4 * (size_t)((nnz + 3) & ~3) + bytes * nnz;
+  };
   const size_t tb = fp32 ? 4 : 8;
-  p->lds = 4 * (size_t)((p->stage_rows + 4) & ~3) + 4 * (size_t)((p->stage_nnz + 3) & ~3) + tb * p->stage_nnz;
-  if (stream_vec_layout(k) && p->lds > kMaxLds) {
+  if (stream_vec_layout(k) && stage(p->stage_nnz, tb) > kMaxLds) {
     delete p;
     set_error("stream engine: a matrix row has too many nonzeros for the LDS stage; use the persistent engine");
     return FEM_ERR_INVALID;
   }
   // the right-hand side's stage: pattern and two FP64 value rows, where it fits
-  const size_t lds_rhs =
-      4 * (size_t)((p->stage_rows + 4) & ~3) + 4 * (size_t)((p->stage_nnz + 3) & ~3) + 16 * (size_t)p->stage_nnz;
-  p->lds_rhs = stream_vec_layout(k) && lds_rhs <= kMaxLds ? lds_rhs : 0;
-  // the residual's S rows: staged when they exceed half of the 256 MB
-  // Infinity Cache (they then come from HBM); below that they stay cached
-  // between sweeps and one lane per row reads them faster than a staged copy
-  p->lds_res = p->lds_rhs && s_bytes > 128.0 * (1 << 20) ? lds_rhs - 8 * (size_t)p->stage_nnz : 0;
+  const bool rhs = stream_vec_layout(k) && stage(p->stage_nnz, 16) <= kMaxLds;
+  // and the residual's, S alone: one lane per row reading its row from memory
+  // touches many lines per load (16 columns, uneven batches: 95 us a pass
+  // against 80 staged; one column, 1.05M rows: 34 against 32.6)
+  p->stage_nnz = (p->stage_nnz + 6) & ~3;
+  p->lds = stage(p->stage_nnz, tb);
+  p->lds_rhs = rhs ? stage(p->stage_nnz, 16) : 0;
+  p->lds_res = rhs ? stage(p->stage_nnz, 8) : 0;
   int rc = 0;
   p->d_ss = dalloc<SState>(p->ninst, &rc);
   p->d_blk_inst = dalloc<int>(std::max(1, p->nblocks), &rc);

@@ -142,6 +142,45 @@ struct Stage {
   int row_lo;
 };
 
+// Copy the entries [base, s_hi) of the columns and of one or two value rows
+// to LDS: base is a multiple of 4, so all but the arrays' last chunk go in
+// 16-byte loads, two chunks of 4 entries per lane in flight at once.  Element
+// loads, one wave-wide entry after the other, made every block wait for
+// memory 4 to 8 times before its gathers (16 FP32 columns, BiCGSTAB's phase S
+// over uneven batches: 43.0 us, now 41.0; one column's right-hand side over
+// 1.05M rows 71, now 64).
+template <typename T, bool TWO>
+__device__ inline void stage_entries(const int GA* ci, const T GA* a, const T GA* b, int base, int s_hi, int nnz,
+                                     int LA* lci, T LA* la, T LA* lb) {
+  constexpr int U = 2;
+  const int nch = (s_hi - base + 3) >> 2, whole = min(nch, (nnz - base) >> 2);
+  for (int q0 = threadIdx.x; q0 < whole; q0 += U * kBlock) {
+    vec<int, 4> c[U];
+    vec<T, 4> x[U], y[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int e = base + 4 * min(q0 + u * kBlock, whole - 1);
+      c[u] = *(const vec<int, 4> GA*)(ci + e);
+      x[u] = *(const vec<T, 4> GA*)(a + e);
+      if (TWO) y[u] = *(const vec<T, 4> GA*)(b + e);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int q = q0 + u * kBlock;
+      if (q >= whole) break;
+      *(vec<int, 4> LA*)(lci + 4 * q) = c[u];
+      *(vec<T, 4> LA*)(la + 4 * q) = x[u];
+      if (TWO) *(vec<T, 4> LA*)(lb + 4 * q) = y[u];
+    }
+  }
+  const int e = 4 * whole + (int)threadIdx.x;  // the arrays' last, incomplete chunk
+  if (whole < nch && threadIdx.x < 4 && base + e < nnz) {
+    lci[e] = ci[base + e];
+    la[e] = a[base + e];
+    if (TWO) lb[e] = b[base + e];
+  }
+}
+
 // The right-hand side's steady cases after a launch's first step, where the
 // previous update formed what the rows gather (vphase_rhs's nm and pre): 1
 // Newmark (K and S rows, gathering hvec and the guess in x), 2 heat or
@@ -463,6 +502,102 @@ __device__ void vphase_pcg_iter(const Inst& I, int row_lo, int row_hi, const Sta
     acc[0] += to_d<V>(rr) * to_d<V>(un);
     acc[1] += to_d<V>(un) * to_d<V>(wa);
     acc[2] += to_d<V>(rr) * to_d<V>(rr);
+  }
+}
+
+// One column: an iteration's residual, product, direction and search direction
+// of a row lie together, {r, w, s, p}, so that a neighbour's three values are
+// one load and a row is stored in one.  Rows of uneven length put a wave's
+// neighbours on several lattice rows: its 21 scalar gathers made 12.9M cache
+// accesses an iteration at 1.05M rows, 50K per CU, and bound the phase at
+// 28 us (FP32); packed it makes 6.6M and takes 21.5, near
+// what the 130 MB that it moves take within the caches (6 TB/s).
+//
+// Two buffers of the packed rows in the vector slab behind xi and r, from the
+// next 16 bytes on (alloc_inst leaves room).
+template <typename TI>
+__device__ inline TI* packed_rows(const Inst& I, int which) {
+  return (TI*)(((uintptr_t)I.z + 15) & ~(uintptr_t)15) + (size_t)which * 4 * I.n;
+}
+template <typename TI>
+__device__ inline void put_row(TI* q, int row, TI r, TI w, TI s, TI p) {
+  if constexpr (sizeof(TI) == 4) {
+    *(vec<TI, 4> GA*)(q + 4 * (size_t)row) = vec<TI, 4>{r, w, s, p};
+  } else {
+    *(vec<TI, 2> GA*)(q + 4 * (size_t)row) = vec<TI, 2>{r, w};
+    *(vec<TI, 2> GA*)(q + 4 * (size_t)row + 2) = vec<TI, 2>{s, p};
+  }
+}
+template <typename TI>
+struct Packed {
+  TI r, w, s, p;
+};
+// whole: with p, which only the row itself needs
+template <bool whole, typename TI>
+__device__ inline Packed<TI> get_row(const TI* q, int row) {
+  const TI* at = q + 4 * (size_t)row;
+  if constexpr (sizeof(TI) == 4) {
+    const vec<TI, 4> v = *(const vec<TI, 4> GA*)at;
+    return {v.x, v.y, v.z, v.w};
+  } else {
+    const vec<TI, 2> v = *(const vec<TI, 2> GA*)at;
+    if constexpr (whole) {
+      const vec<TI, 2> u = *(const vec<TI, 2> GA*)(at + 2);
+      return {v.x, v.y, u.x, u.y};
+    } else {
+      return {v.x, v.y, gp(at)[2], (TI)0};
+    }
+  }
+}
+
+template <typename TI>
+__device__ void vphase_pcg_init_packed(const Inst& I, int row_lo, int row_hi, const Stage<TI>& g, TI* q,
+                                       vec<double, 1> (&acc)[2]) {
+  constexpr int U = vunroll<1>();
+  const TI GA* r = gp((const TI*)I.r);
+  TI GA* xi = gp((TI*)I.xi);
+  const TI GA* dinv = gp((const TI*)I.dinvi);
+  for (int row = row_lo + (int)threadIdx.x; row < row_hi; row += kBlock) {
+    const TI ro = r[row];
+    const int lr = row - g.row_lo;
+    const TI wa = vgather<U>(g.rp[lr], g.rp[lr + 1], (TI)0, [&](int s) { return g.w[s] * r[g.ci[s]]; });
+    gp(I.x)[row] = gp(I.x)[row] + (double)xi[row];
+    xi[row] = (TI)0;
+    put_row<TI>(q, row, ro, wa, (TI)0, (TI)0);
+    const TI uo = dinv[row] * ro;
+    acc[0] += (double)ro * (double)uo;
+    acc[1] += (double)uo * (double)wa;
+  }
+}
+
+// One Chronopoulos-Gear iteration from qc to qn (vphase_pcg_iter's
+// arithmetic; s and p are zero and beta is zero before the first).
+template <typename TI>
+__device__ void vphase_pcg_iter_packed(const Inst& I, int row_lo, int row_hi, const Stage<TI>& g, const TI* qc, TI* qn,
+                                       const Shared& sh, vec<double, 1> (&acc)[3]) {
+  constexpr int U = 5;  // 62 registers and 8 waves per SIMD; 8 entries at a time: 83 and 5, 10% slower
+  TI GA* xi = gp((TI*)I.xi);
+  const TI GA* dinv = gp((const TI*)I.dinvi);
+  const TI al = to_ti<TI>(sh.alpha[0]), be = to_ti<TI>(sh.beta[0]);
+  for (int row = row_lo + (int)threadIdx.x; row < row_hi; row += kBlock) {
+    const Packed<TI> o = get_row<true>(qc, row);
+    const TI xio = xi[row];
+    const TI d = dinv[row];
+    const int lr = row - g.row_lo;
+    const TI wa = vgather<U>(g.rp[lr], g.rp[lr + 1], (TI)0, [&](int s) {
+      const Packed<TI> c = get_row<false>(qc, g.ci[s]);
+      return g.w[s] * cg_r<TI>(c.r, cg_s<TI>(c.w, c.s, be, false), al);
+    });
+    const TI uo = d * o.r;
+    const TI pn = uo + be * o.p;
+    const TI sv = cg_s<TI>(o.w, o.s, be, false);
+    const TI rr = cg_r<TI>(o.r, sv, al);
+    xi[row] = xio + al * pn;
+    put_row<TI>(qn, row, rr, wa, sv, pn);
+    const TI un = d * rr;
+    acc[0] += (double)rr * (double)un;
+    acc[1] += (double)un * (double)wa;
+    acc[2] += (double)rr * (double)rr;
   }
 }
 

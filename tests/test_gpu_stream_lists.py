@@ -39,3 +39,63 @@ def test_lists_and_reductions(gpu, count, cells, k, advdiff, precision):
         b.close()
     for i, (x, y) in enumerate(zip(*got)):
         assert np.linalg.norm(x - y) <= TOL * np.linalg.norm(y), i
+
+
+def two_engines(m, bc, prm, k, n, **opts):
+    """The state after two steps, on the streaming and on the persistent engine."""
+    ctx = FEMContext(m, bc, velocity=(0.5, 0.3, 0.0), normalize_velocity=False)
+    f = np.random.default_rng(10).standard_normal((n, k))
+    got = []
+    for eng in (_lib.FEM_ENGINE_STREAM, _lib.FEM_ENGINE_PERSISTENT):
+        b = Batch([ctx], SolverOptions(nrhs=k, engine=eng, tol=1e-12, max_iters=1000, **opts))
+        b.set_equation(0, prm)
+        b.set_state_unknowns(0, _lib.FEM_FIELD_U, f)
+        assert b.advance(2) == _lib.FEM_OK
+        got.append(b.get_state_unknowns(0).reshape(-1, k))
+        b.close()
+    ctx.close()
+    return got
+
+
+@pytest.mark.parametrize("k,krylov", [(1, 1), (1, 2), (1, 3), (4, 1), (16, 2), (16, 3)])
+@pytest.mark.parametrize("precision", [_lib.FEM_PREC_FP32_IR, _lib.FEM_PREC_FP64])
+def test_stage_edges(gpu, k, krylov, precision):
+    """Row blocks staged in 16-byte pieces from an aligned start: entry counts
+    of every remainder by 4, one block and several."""
+    rest = set()
+    for cells, held in ((4, 0), (5, 0), (5, 1), (6, 2), (7, 1), (8, 3), (20, 1), (21, 0), (34, 2), (35, 1)):
+        print("case stream stage", k, krylov, precision, cells, held, flush=True)
+        m = meshes.jittered_square(cells, seed=cells)
+        m["on_boundary"][np.flatnonzero(m["on_boundary"] == 0)[:held]] = 1  # held vertices change the remainder
+        ctx = FEMContext(m, 0)
+        n = ctx.info().num_unknowns
+        rest.add(ctx.info().nnz % 4)
+        ctx.close()
+        c = 1.5 / (1e-3 * cells * cells)
+        prm = AdvectionDiffusionParameters(1e-3, c) if krylov == _lib.FEM_KRYLOV_BICGSTAB else HeatParameters(1e-3, c)
+        x, y = two_engines(m, 0, prm, k, n, krylov=krylov, precision=precision)
+        assert np.linalg.norm(x - y) <= TOL * np.linalg.norm(y), cells
+    assert rest == {0, 1, 2, 3}
+
+
+def test_longest_row_that_fits(gpu):
+    """A hub whose FP64 row of 5,074 entries fills the stage's limit (61,936
+    bytes: 12 an entry and 1,040 for the block's rows) from an unaligned start,
+    so the aligned one's slack comes on top; one entry more is refused."""
+    def fan(d):
+        t = 2 * np.pi * np.arange(d) / d
+        xyz = np.concatenate([[[3, 0, 0], [4, 0, 0], [3, 1, 0], [0, 0, 0.5]],
+                              np.stack([np.cos(t), np.sin(t), 0 * t], 1)]).astype(np.float32)
+        tri = np.concatenate([[[0, 1, 2]], np.stack([np.full(d, 3), 4 + np.arange(d), 4 + (np.arange(d) + 1) % d], 1)])
+        return {"xyz": xyz, "tri": tri.astype(np.uint32), "on_boundary": np.zeros(d + 4, np.uint8)}
+
+    print("case stream longest row", flush=True)
+    prm = HeatParameters(1e-3, 1e-3)
+    x, y = two_engines(fan(5073), 1, prm, 1, 5077, precision=_lib.FEM_PREC_FP64)
+    assert np.linalg.norm(x - y) <= TOL * np.linalg.norm(y)
+    print("case stream row refused", flush=True)
+    b = Batch([FEMContext(fan(5074), 1)], SolverOptions(engine=_lib.FEM_ENGINE_STREAM, precision=_lib.FEM_PREC_FP64))
+    b.set_equation(0, prm)
+    with pytest.raises(_lib.FemError, match="too many nonzeros"):
+        b.advance(1)
+    b.close()
