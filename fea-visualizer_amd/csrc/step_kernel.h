@@ -1435,11 +1435,13 @@ FEM_INLINE void phase_res_rows(const Inst& I, const Team& T, int row_lo, int row
   auto load = [&](int row, Row& w) {
     if (row >= row_hi) return;
     const int lo = rp[row], hi = rp[row + 1];
+    if (hi > lo) {  // a vertex without triangles has no entries
 #pragma unroll
-    for (int e = 0; e < kCacheE; e++) {
-      const int s = min(lo + e, hi - 1);  // past the row's end: its weights are 0 below
-      w.s[e] = S64[(size_t)s * kv + vj];
-      w.m[e] = hpre ? M64[s] : 0.0;
+      for (int e = 0; e < kCacheE; e++) {
+        const int s = min(lo + e, hi - 1);  // past the row's end: its weights are 0 below
+        w.s[e] = S64[(size_t)s * kv + vj];
+        w.m[e] = hpre ? M64[s] : 0.0;
+      }
     }
 #pragma unroll
     for (int e = 0; e < kCacheE; e++)

@@ -101,3 +101,32 @@ def test_launch_plan_kept_over_new_matrices(gpu, precision):
     assert np.array_equal(seen[0], seen[2])
     b.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("precision", [_lib.FEM_PREC_FP32_IR, _lib.FEM_PREC_FP64])
+@pytest.mark.parametrize("advdiff", [False, True])
+@pytest.mark.parametrize("k,team", [(1, 0), (1, 3), (4, 20)])
+def test_vertices_without_triangles(gpu, k, team, advdiff, precision):
+    """Rows without entries, the first and the last of the pattern among them:
+    the phases that read a row's entries all at once leave them out.  The
+    streaming engine, whose gathers take them one by one, is the reference."""
+    print("case empty rows", k, team, advdiff, precision, flush=True)
+    m = meshes.jittered_square(24, seed=5)
+    alone = np.zeros((3, 3), np.float32)
+    m = {"xyz": np.ascontiguousarray(np.concatenate([alone + 2, m["xyz"], alone + 3])),
+         "tri": np.ascontiguousarray(m["tri"] + 3).astype(np.uint32),
+         "on_boundary": np.concatenate([np.zeros(3, np.uint8), m["on_boundary"], np.zeros(3, np.uint8)])}
+    ctx = FEMContext(m, 1, velocity=VEL, normalize_velocity=False)
+    rp, _ = ctx.pattern()
+    assert rp[3] == 0 and rp[-1] == rp[-4]
+    f = np.random.default_rng(6).standard_normal((len(rp) - 1, k))
+    got = []
+    for opts in ({"team_size": team}, {"engine": _lib.FEM_ENGINE_STREAM}):
+        b = Batch([ctx], SolverOptions(nrhs=k, precision=precision, tol=1e-12, **opts))
+        b.set_equation(0, AdvectionDiffusionParameters(1e-3, 0.05) if advdiff else HeatParameters(1e-3, 0.05))
+        b.set_state_unknowns(0, _lib.FEM_FIELD_U, f)
+        assert b.advance(3) == _lib.FEM_OK
+        got.append(b.get_state_unknowns(0).reshape(-1, k))
+        b.close()
+    assert rel(got[0], got[1]) <= TOL
+    ctx.close()
