@@ -109,15 +109,20 @@ __device__ inline A vgather(int lo, int hi, A zero, F f) {
   return acc;
 }
 
+// One column: 5 of a row's ~7 entries at a time leaves 8 waves per SIMD (CG
+// iteration over packed rows: 62 registers, against 83 and 5 waves with 8, 10%
+// slower; FP64 residual, 1.05M rows: 28.4 us against 33.7; right-hand side 5%).
 template <int V>
 constexpr int vunroll() {
-  return V >= 4 ? 2 : V == 2 ? 4 : 8;
+  return V >= 4 ? 2 : V == 2 ? 4 : 5;
 }
 // BiCGSTAB's gathers (one and two vectors per neighbour): twice the entries
-// in flight at four columns per lane measured faster on 7-point rows.
+// in flight at four columns per lane measured faster on 7-point rows; phase S
+// takes 5 (1.2M rows x 16 columns: 112 us against 117 with 4, 114 with 3).  One
+// column, 490K rows, FP64, phase S: 16.5 us with 5, 19.1 with 8.
 template <int V>
-constexpr int vunroll_bi() {
-  return V >= 4 ? 4 : V == 2 ? 4 : 8;
+constexpr int vunroll_bi(bool two = false) {
+  return V >= 4 ? (two ? 5 : 4) : V == 2 ? 4 : 5;
 }
 
 // Lane layout: G = K / V lanes per row; lane columns j0 .. j0 + V - 1 with
@@ -575,7 +580,7 @@ __device__ void vphase_pcg_init_packed(const Inst& I, int row_lo, int row_hi, co
 template <typename TI>
 __device__ void vphase_pcg_iter_packed(const Inst& I, int row_lo, int row_hi, const Stage<TI>& g, const TI* qc, TI* qn,
                                        const Shared& sh, vec<double, 1> (&acc)[3]) {
-  constexpr int U = 5;  // 62 registers and 8 waves per SIMD; 8 entries at a time: 83 and 5, 10% slower
+  constexpr int U = vunroll<1>();
   TI GA* xi = gp((TI*)I.xi);
   const TI GA* dinv = gp((const TI*)I.dinvi);
   const TI al = to_ti<TI>(sh.alpha[0]), be = to_ti<TI>(sh.beta[0]);
@@ -719,7 +724,7 @@ __device__ void vphase_bi_s(const Inst& I, int row_lo, int row_hi, const Stage<T
   using TV = vec<TI, V>;
   using DV = vec<double, V>;
   using L = VLay<K, V>;
-  constexpr int U = vunroll_bi<V>();
+  constexpr int U = vunroll_bi<V>(true);
   const int j0 = ((int)threadIdx.x % L::G) * V;
   TI* tv = (TI*)I.t;  // own rows only
   const TI* rh = (const TI*)I.rh;
