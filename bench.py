@@ -44,9 +44,9 @@ import numpy as np  # noqa: E402
 HBM_PEAK_GBS = 8000.0
 # Bytes of the dominant kernel's dispatch measured with rocprofv3
 # FETCH_SIZE / WRITE_SIZE (calibrated against a plain copy kernel) for the
-# exact command given; the summaries with their commands are in profiles/.
+# arguments given; the summaries with their commands are in profiles/.
 PROFILED_TRAFFIC = {
-    "grayscott": {"steps": 20, "warmup": 5, "predictor": "sextic", "bytes_per_launch": 1.5290e9,
+    "grayscott": {"steps": 20, "warmup": 5, "predictor": "sextic", "bytes_per_launch": 1.3856e9,
                   "source": "profiles/k_step_grayscott_icosphere6.md"},
     "spmv": {"bytes_per_launch": 1.2087e9, "source": "profiles/k_spmv_stream_jittered4096.md"},
 }

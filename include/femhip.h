@@ -91,7 +91,8 @@ typedef struct fem_mesh {
  * (EquationParameters.hpp:17-26, read at FEMContext.cpp:58) plus extensions. */
 typedef struct fem_assembly_params {
   double velocity[3];          /* constant velocity */
-  const double* velocity_e;    /* optional: 3 per triangle (overrides velocity) */
+  const double* velocity_e;    /* optional: 3 per triangle (overrides velocity), in host
+                                * or device memory */
   int32_t normalize_velocity;  /* 1 = reference (unit tangential velocity, FEMContext.cpp:180) */
   const double* kappa_e;       /* optional: per-triangle diffusivity multiplying K, in
                                 * host or device memory */
