@@ -398,6 +398,18 @@ FEM_INLINE void collect(const Team& T, int rank, unsigned e, TeamShared& sh) {
   if (to) sh.tmo = 1;
 }
 
+// Run scalars() in the control wave on the sums its lanes have stored to
+// sh.red.  Lane j reads what other lanes of the wave wrote: the fence keeps
+// the compiler from moving those loads before the stores (the wave's LDS
+// accesses complete in program order).
+template <typename F>
+FEM_INLINE void run_scalars(F scalars) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  scalars();
+}
+
 // Reduction + barrier: acc -> team sums in sh.red[q*K + j], handed to
 // scalars(), which the control wave (whose lanes wrote them) runs; every wave
 // returns once all ranks have arrived and the scalars are in LDS.  Returns
@@ -408,7 +420,7 @@ FEM_INLINE bool team_reduce(const double (&acc)[NS], const Team& T, int rank, un
   // a one-workgroup team (also inside a multi-workgroup launch) reduces in LDS
   if (C == kPlain || T.size == 1) {
     block_partials<K, NS, kPlain>(acc, sh, sh.red, e);
-    if (ctl() >= 0) scalars();
+    if (ctl() >= 0) run_scalars(scalars);
     __syncthreads();
     return true;
   }
@@ -417,7 +429,7 @@ FEM_INLINE bool team_reduce(const double (&acc)[NS], const Team& T, int rank, un
     collect<K, NS * K>(T, rank, e, sh);
     // acquire: drop cached copies of data other workgroups wrote this phase
     if constexpr (C == kFenced) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    scalars();
+    run_scalars(scalars);
   }
   __syncthreads();
   if (sh.tmo) {
@@ -439,14 +451,14 @@ FEM_INLINE bool rows_reduce(const double (&acc)[NS], const Team& T, int rank, un
   e++;
   if (C == kPlain || T.size == 1) {
     block_partials<K, NS, kPlain>(acc, sh, sh.red, e);
-    if (ctl() >= 0) scalars();
+    if (ctl() >= 0) run_scalars(scalars);
     __syncthreads();
     return true;
   }
   block_partials<K, NS, C, false>(acc, sh, team_record(T, e & 3, rank), e);
   if (ctl() >= 0) {
     collect<K, NS * K>(T, rank, e, sh);
-    scalars();
+    run_scalars(scalars);
   } else {
     int to = 0;
     halo.take(T, e, &to);
