@@ -15,7 +15,6 @@
 #include "femhip_ctx.h"
 
 #include <algorithm>
-#include <cstdint>
 
 namespace femhip {
 
@@ -120,7 +119,7 @@ __global__ void __launch_bounds__(kBlock) k_spmv_stream(int n, long long nnz, co
   using SS = StreamShape<T, K>;
   constexpr int V = SS::V, LPR = SS::LPR, R = SS::R;
   constexpr int CAP = R * kCapRow;  // multiple of 4
-  typedef T vec __attribute__((ext_vector_type(V)));
+  typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));  // x and y: aligned to the type alone
   __shared__ int s_ci[CAP];
   __shared__ T s_val[CAP];
   const int row0 = dealt_block() * R;
@@ -210,7 +209,7 @@ __global__ void __launch_bounds__(kBlock) k_spmv_pipe(int n, long long nnz, int 
   constexpr int V = SS::V, LPR = SS::LPR, R = SS::R;
   constexpr int CAP = R * kCapRow;                       // multiple of 4
   constexpr int NCH = (CAP / 4 + kBlock - 1) / kBlock;   // 4-entry chunks per thread
-  typedef T vec __attribute__((ext_vector_type(V)));
+  typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));  // x and y: aligned to the type alone
   typedef T v4t __attribute__((ext_vector_type(4)));
   __shared__ int s_ci[2][CAP];
   __shared__ T s_val[2][CAP];
@@ -380,15 +379,12 @@ int stream_rows(int k) {
 // stream with non-temporal matrix loads.  16 lanes per row with 16 columns is
 // one column per lane, 4 bytes a gather where the stream has 16: 1000 x 1100
 // nodes, FP32, 120 us a product against 61; 700 x 700 FP64 116 against 56;
-// 64 x 64 FP32 3.3 against 2.7.  It takes x and y at any alignment of their
-// type, and keeps those that the stream's 16-byte accesses cannot.  Below 256
-// x 256 nodes and one column 4 lanes per row take 2.2 us against 2.8, both
-// under the launch's own cost; the other stream variants lie within 10% of
-// this one either way.
-int default_schedule(int k, const void* x, const void* y) {
-  if (k >= 16 && (((uintptr_t)x | (uintptr_t)y) & 15)) return 16;
-  return FEM_SPMV_STREAM_NT;
-}
+// 64 x 64 FP32 3.3 against 2.7.  Callers hand x and y over at any alignment of
+// their type; the stream's vector accesses to them assume no more (the code is
+// the same as for aligned vectors).  Below 256 x 256 nodes and one column 4
+// lanes per row take 2.2 us against 2.8, both under the launch's own cost; the
+// other stream variants lie within 10% of this one either way.
+constexpr int kDefaultSchedule = FEM_SPMV_STREAM_NT;
 
 template <typename T>
 int pipe_grid_k(int k, bool nt, int nblk, int* grid) {
@@ -500,7 +496,7 @@ int operator_apply_device(fem_operator* op, int k, const void* x, void* y) {
     set_error("operator: nrhs must be 1, 2, 4 or 16");
     return FEM_ERR_INVALID;
   }
-  const int g = op->lanes[k] ? op->lanes[k] : default_schedule(k, x, y);
+  const int g = op->lanes[k] ? op->lanes[k] : kDefaultSchedule;
   return launch(op, k, g, x, y);
 }
 
@@ -567,7 +563,7 @@ int operator_time(fem_operator* op, int k, const void* x, void* y, int reps, dou
     set_error("operator_time: nrhs must be 1, 2, 4 or 16 and reps >= 1");
     return FEM_ERR_INVALID;
   }
-  const int g = op->lanes[k] ? op->lanes[k] : default_schedule(k, x, y);
+  const int g = op->lanes[k] ? op->lanes[k] : kDefaultSchedule;
   return time_lanes(op, k, g, x, y, reps, ms);
 }
 
@@ -586,7 +582,7 @@ int operator_autotune(fem_operator* op, int k, const void* x, void* y, int reps,
     return FEM_ERR_INVALID;
   }
   double best = 1e300;
-  int bg = default_schedule(k, x, y);
+  int bg = kDefaultSchedule;
   for (int g : {1, 2, 4, 8, 16, (int)FEM_SPMV_STREAM, (int)FEM_SPMV_STREAM_NT, (int)FEM_SPMV_PIPE,
                 (int)FEM_SPMV_PIPE_NT}) {
     if (g < k) continue;
