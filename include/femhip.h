@@ -88,7 +88,10 @@ typedef struct fem_mesh {
 } fem_mesh;
 
 /* Assembly inputs: AdvectionDiffusionParameters::velocity
- * (EquationParameters.hpp:17-26, read at FEMContext.cpp:58) plus extensions. */
+ * (EquationParameters.hpp:17-26, read at FEMContext.cpp:58) plus extensions.
+ * Coefficients in device memory must be complete when the call is made: it
+ * reads them on the context's own stream, which waits for no other stream, the
+ * null stream included.  They are read before the call returns. */
 typedef struct fem_assembly_params {
   double velocity[3];          /* constant velocity */
   const double* velocity_e;    /* optional: 3 per triangle (overrides velocity), in host
