@@ -760,6 +760,21 @@ int build_plan(fem_batch* b) {
     ht[t].wait_ticks = b->wait_ticks;
     ht[t].allpoll = b->poll_override == 1 ? 1 : b->poll_override == 2 ? 0 : flat_reduction(sizes[t], k);
   }
+  // exchange words of the instances whose teams may keep their rows in LDS (at
+  // most kCacheP per lane of the grid); the others do without
+  std::vector<char> wants(ninst, 0);
+  for (size_t q = 0; q < nlist; q++) wants[team_inst[q]] |= shape[q].cap > 0;
+  for (int i = 0; i < ninst; i++) {
+    InstHost& h = b->insts[i];
+    if (wants[i] && !h.d_xch) {
+      h.d_xch = dalloc<unsigned long long>((size_t)h.ctx->n * k * xch_words(inner_fp32 ? 4 : 8), &rc);
+      if (rc) return rc;
+    } else if (!wants[i] && h.d_xch) {
+      (void)hipFree(h.d_xch);
+      h.d_xch = nullptr;
+    }
+    h.dev.xch = h.d_xch;
+  }
   std::vector<Inst> hi(ninst);
   for (int i = 0; i < ninst; i++) hi[i] = persistent_desc(b->insts[i].dev);
   std::vector<char> host(plan_bytes);
@@ -1296,12 +1311,6 @@ int batch_prepare(fem_batch* b, bool need_plan) {
       if (!h.d_xnext) h.d_xnext = dalloc<double>((size_t)h.ctx->n * h.k, &rc);
       if (!rc && need_plan && !h.d_hpre) h.d_hpre = dalloc<double>((size_t)h.ctx->n * h.k, &rc);
       if (!rc && need_plan && !h.d_hvec) h.d_hvec = dalloc<double>((size_t)h.ctx->n * h.k, &rc);
-      if (rc) return rc;
-    }
-    // exchange words of the persistent plans
-    if (need_plan && !h.d_xch) {
-      int rc = 0;
-      h.d_xch = dalloc<unsigned long long>((size_t)h.ctx->n * h.k * xch_words((int)inner_bytes(b)), &rc);
       if (rc) return rc;
     }
     // Newmark on the streaming engine: each update forms the next step's
