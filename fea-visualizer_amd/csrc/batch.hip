@@ -443,9 +443,14 @@ void free_plan(fem_batch* b) {
 }  // namespace
 
 // Workgroups of the team of a lone instance, within maxb co-resident
-// workgroups: team_size when given and it fits, else one per 128 rows x
-// columns, up to one per CU.  Few rows per workgroup leave most of its waves
-// to the halo and the control wave.  Where that would leave the flat reduction
+// workgroups: team_size when given and it fits.  Else one up to kCacheP rows x
+// columns per lane: its barriers stay on the CU (us a step, one workgroup and
+// the fastest team of several: 162 rows of a sphere 16 and 34, 484 lattice rows
+// 38 and 58, 256 rows of 2 columns 41 and 65; classic CG, which has no rows in
+// LDS, 256 rows 75 and 144, 484 rows 134 and 144; a workgroup past its rows in
+// LDS takes twice as long as two).  Else one per 128 rows x columns, up to one
+// per CU.  Few rows per workgroup leave most of its waves to the halo and the
+// control wave.  Where that would leave the flat reduction
 // (flat_reduction), its largest team is kept while its workgroups stay short:
 // the second level costs an iteration more than the longer gathers do (one
 // column, us per iteration: 9,801 rows 4.7 at 64 workgroups, 5.3 at 128;
@@ -455,7 +460,8 @@ void free_plan(fem_batch* b) {
 int single_team_size(long long n, int k, int team_size, int maxb) {
   if (team_size > 0 && team_size <= maxb) return team_size;
   const long long lanes = n * k;
-  int g = (int)std::min<long long>(1024, std::max(1LL, (lanes + 127) / 128));
+  if (lanes <= kCacheP * kBlock) return 1;
+  int g = (int)std::min<long long>(1024, (lanes + 127) / 128);
   const int flat = std::max(kGroup, 256 / (4 * k));
   if (g > flat && lanes <= (long long)flat * (k == 1 ? 640 : 320)) g = flat;
   return std::min(g, maxb);
