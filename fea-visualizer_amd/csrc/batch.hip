@@ -451,19 +451,23 @@ void free_plan(fem_batch* b) {
 // LDS takes twice as long as two).  Else one per 128 rows x columns, up to one
 // per CU.  Few rows per workgroup leave most of its waves to the halo and the
 // control wave.  Where that would leave the flat reduction
-// (flat_reduction), its largest team is kept while its workgroups stay short:
-// the second level costs an iteration more than the longer gathers do (one
+// (flat_reduction), its largest team is kept (flat) while its workgroups stay
+// short: the second level costs an iteration more than the longer gathers do (one
 // column, us per iteration: 9,801 rows 4.7 at 64 workgroups, 5.3 at 128;
 // 39,601 rows 4.3 and 4.5; 89,401 rows take two-level teams; two columns:
 // 2,562 rows 5.4 at 20 workgroups and 6.3 at 40, 10,242 rows 9.1 at 40 and
-// 7.6 at 160).
-int single_team_size(long long n, int k, int team_size, int maxb) {
+// 7.6 at 160).  That holds for gathers from LDS alone: from memory they are most
+// of an iteration, and more workgroups have more of them in flight (us per
+// iteration at 64 and 256 workgroups: 16,000 rows of a Delaunay mesh, up to 12
+// entries a row, 11.3 and 8.5; 40,000 rows 23.8 and 11.6; classic CG on 39,601
+// scattered rows 27.7 and 16.0).
+int single_team_size(long long n, int k, int team_size, int maxb, bool flat) {
   if (team_size > 0 && team_size <= maxb) return team_size;
   const long long lanes = n * k;
   if (lanes <= kCacheP * kBlock) return 1;
   int g = (int)std::min<long long>(1024, (lanes + 127) / 128);
-  const int flat = std::max(kGroup, 256 / (4 * k));
-  if (g > flat && lanes <= (long long)flat * (k == 1 ? 640 : 320)) g = flat;
+  const int f = std::max(kGroup, 256 / (4 * k));
+  if (flat && g > f && lanes <= (long long)f * (k == 1 ? 640 : 320)) g = f;
   return std::min(g, maxb);
 }
 
@@ -490,13 +494,16 @@ bool team_streams(long long n, int k, int size) {
   return rows * k > (long long)kCacheP * kTeamBlock;
 }
 
-// Whether the workgroups of a team can keep the instance's rows in LDS, but
-// for the halo (HaloRef::ok): at most kCacheP rows per lane, rows of at most
-// kCacheE entries, and not classic CG.
+// Whether any team can keep the instance's rows in LDS: rows of at most kCacheE
+// entries, and not classic CG.
+bool rows_possible(const fem_ctx* c, int kr) { return kr != 2 && c->max_row <= kCacheE; }
+
+// Whether the workgroups of a team of `size` can, but for the halo
+// (HaloRef::ok): at most kCacheP rows per lane.
 bool rows_fit(const fem_ctx* c, int k, int size, int kr) {
   const long long rows = (c->n + size - 1) / size;
   const int block = size == 1 ? kBlock : kTeamBlock;
-  return kr != 2 && c->max_row <= kCacheE && rows * k <= (long long)kCacheP * block;
+  return rows_possible(c, kr) && rows * k <= (long long)kCacheP * block;
 }
 
 // Co-resident workgroups that both variants of an exchange mode (rows in LDS
@@ -601,7 +608,9 @@ static Inst persistent_desc(const Inst& d) {
   return I;
 }
 
-int build_plan(fem_batch* b) {
+// flat: a lone instance's team may be kept at the flat reduction's largest, if
+// its rows may stay in LDS there.
+int build_plan(fem_batch* b, bool flat = true) {
   free_plan(b);
   const int ninst = (int)b->insts.size();
   const int k = b->insts[0].k;
@@ -617,6 +626,7 @@ int build_plan(fem_batch* b) {
       return FEM_ERR_INVALID;
     }
   const int inner_fp32 = inner_bytes(b) == 4;
+  flat = flat && ninst == 1 && rows_possible(b->insts[0].ctx, kr);
   // co-resident workgroups of each variant: plain (one-workgroup teams),
   // coherent and fenced exchange; they differ in registers
   int maxv[3] = {0, 0, 0};
@@ -641,7 +651,7 @@ int build_plan(fem_batch* b) {
     sizes.clear();
     if (ninst == 1) {
       teams.push_back({0});
-      sizes.push_back(single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, maxb));
+      sizes.push_back(single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, maxb, flat));
     } else if (b->opts.team_size > 0 && (long long)b->opts.team_size * ninst <= maxb) {
       for (int i = 0; i < ninst; i++) {
         teams.push_back({i});
@@ -810,6 +820,11 @@ int build_plan(fem_batch* b) {
       rows |= fits;
       streaming |= sizes[t] > 1 && team_streams(b->insts[team_inst[q]].ctx->n, k, sizes[t]);
     }
+  // a team sized for rows in LDS, but the halo of a scattered numbering does not fit
+  if (flat && multi && !rows) {
+    const int maxb = std::min(maxv[kExchangeCoherent], maxv[kExchangeFenced]);
+    if (single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, maxb, false) != grid) return build_plan(b, false);
+  }
   const int mode = exchange_mode(multi, streaming, forced, b->mode_override);
   if (grid > maxv[mode]) {
     set_error("team plan exceeds the co-resident grid");

@@ -27,11 +27,12 @@ constexpr int kExchangeCoherent = 1, kExchangeFenced = 2;
 int launch_step(const StepLaunch& L, int nsteps, hipStream_t st);
 
 // Plan rules shared by the batch plans and the allocation-free solve (batch.hip).
-int single_team_size(long long n, int k, int team_size, int maxb);
+int single_team_size(long long n, int k, int team_size, int maxb, bool flat);
 int flat_reduction(int size, int k);
 size_t slot_bytes(int grid, int k);
 void team_slots(Team* T, double* slots, int grid, int k);
 bool team_streams(long long n, int k, int size);
+bool rows_possible(const fem_ctx* c, int kr);
 bool rows_fit(const fem_ctx* c, int k, int size, int kr);
 int variant_coresident(int k, int inner_fp32, int kr, int coh, int* blocks);
 int exchange_mode(bool multi, bool streaming, int forced, int tuned);

@@ -89,10 +89,9 @@ __global__ void k_noalloc_setup(Team team, Inst inst, HaloRef halo, int grid, Te
   for (long long q = i; q < nzero; q += (long long)gridDim.x * blockDim.x) zero[q] = 0.0;
 }
 
-}  // namespace
-
-int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
-                         fem_step_stats* stats) {
+// flat as in build_plan: the same plan, so the same results bit for bit.
+int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
+                  fem_step_stats* stats, bool flat) {
   fem_solver_opts o;
   fem_opts_default(&o);
   if (opts) o = *opts;
@@ -117,6 +116,7 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   int kr = o.krylov;
   if (kr == FEM_KRYLOV_AUTO) kr = coef[2] != 0.0 ? FEM_KRYLOV_BICGSTAB : FEM_KRYLOV_CG;
   const int kri = (kr == FEM_KRYLOV_BICGSTAB) ? 1 : (kr == FEM_KRYLOV_CG_CLASSIC) ? 2 : 0;
+  flat = flat && rows_possible(c, kri);
 
   // plan: one team, sized and moded as a one-instance batch plan
   int maxv[3] = {0, 0, 0};
@@ -125,10 +125,10 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
     if (rc) return rc;
   }
   const int forced = (o.exchange == FEM_EXCHANGE_COHERENT || o.exchange == FEM_EXCHANGE_FENCED) ? o.exchange : 0;
-  int grid = single_team_size(n, k, o.team_size, maxv[kExchangeCoherent]);
+  int grid = single_team_size(n, k, o.team_size, maxv[kExchangeCoherent], flat);
   int mode = exchange_mode(grid > 1, team_streams(n, k, grid), forced, 0);
   if (grid > maxv[mode]) {
-    grid = single_team_size(n, k, o.team_size, std::min(maxv[0], std::min(maxv[1], maxv[2])));
+    grid = single_team_size(n, k, o.team_size, std::min(maxv[0], std::min(maxv[1], maxv[2])), flat);
     mode = exchange_mode(grid > 1, team_streams(n, k, grid), forced, 0);
   }
   if (grid <= 0 || grid > maxv[mode]) {
@@ -261,6 +261,15 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   if (rc) return rc;
   rc = launch_slot_reset(slots, grid, slot_vals(k), abort_flag, d_inst, 1, st);
   if (rc) return rc;
+  // which variant runs, and at which size, takes the answer whether the halo fits
+  HaloRef built{};
+  if (halos) {
+    FEM_HIP(hipMemcpyAsync(&built, d_halo, sizeof(built), hipMemcpyDeviceToHost, st));
+    FEM_HIP(hipStreamSynchronize(st));
+  }
+  const bool rows = grid == 1 ? rows_fit(c, k, 1, kri) : built.ok != 0;
+  if (flat && grid > 1 && !rows && single_team_size(n, k, o.team_size, maxv[mode], false) != grid)
+    return solve_noalloc(c, coef, opts, bh, xh, stats, false);
   StepLaunch SL;
   SL.teams = d_team;
   SL.wg_team = d_wg_team;
@@ -271,7 +280,7 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   SL.inner_fp32 = fp32;
   SL.kr = kri;
   SL.coh = mode;
-  SL.rows = grid == 1 ? rows_fit(c, k, 1, kri) : halos;
+  SL.rows = rows;
   rc = launch_step(SL, 1, st);
   if (rc) return rc;
   alignas(8) char rec[kInfoBytes + sizeof(int)];
@@ -300,6 +309,13 @@ int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts
   if (status & (ST_UNSTABLE | ST_NONFINITE)) return FEM_DIVERGED;
   if (status & ST_NOT_CONVERGED) return FEM_NOT_CONVERGED;
   return FEM_OK;
+}
+
+}  // namespace
+
+int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
+                         fem_step_stats* stats) {
+  return solve_noalloc(c, coef, opts, bh, xh, stats, true);
 }
 
 }  // namespace femhip

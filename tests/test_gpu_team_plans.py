@@ -1,11 +1,14 @@
 """The plan rules of the persistent engine at the sizes where they change.
 
-Tolerances as in test_gpu_team_rows (solves to 1e-12 of systems with condition
-numbers below 10, 3 steps, against the oracle)."""
+Tolerances as in test_gpu_team_rows: solves to 1e-12 of Jacobi-scaled systems,
+here with condition numbers up to 16, and 3 steps, so the states are within 5e-11
+of the oracle's."""
+import numpy as np
 import pytest
 
-from femhip import _lib, meshes
-from test_gpu_team_rows import check
+from femhip import FEMContext, SolverOptions, _lib, meshes
+from test_gpu_team_rows import check, scattered
+from test_zz_no_alloc import solve
 
 pytestmark = pytest.mark.gpu
 
@@ -19,3 +22,46 @@ def test_one_workgroup_up_to_two_rows_per_lane(gpu, cells, k, grid, krylov):
     print("case one workgroup", cells, k, krylov, flush=True)
     info = check(meshes.jittered_square(cells, seed=6), False, k, _lib.FEM_PREC_FP32_IR, krylov=krylov, max_iters=1000)
     assert info.grid == grid and (info.exchange == 0) == (grid == 1)
+
+
+def fan_square(cells, seed):
+    """A jittered square whose vertex in the middle is joined to all vertices
+    within four cells, which leaves rows past the 10 entries that stay in LDS."""
+    m = meshes.jittered_square(cells, seed=seed)
+    side, c, r = cells + 1, cells // 2, 4
+    idx = np.arange(side * side).reshape(side, side)
+    drop = idx[c - r + 1:c + r, c - r + 1:c + r].ravel()
+    hub = idx[c, c]
+    keep = m["tri"][~np.isin(m["tri"], drop).any(1)]
+    ring = np.concatenate([idx[c - r, c - r:c + r], idx[c - r:c + r, c + r], idx[c + r, c + r:c - r:-1],
+                           idx[c + r:c - r:-1, c - r]])
+    tri = np.concatenate([keep, np.stack([np.full(len(ring), hub), ring, np.roll(ring, -1)], 1)])
+    used = np.zeros(side * side, bool)
+    used[tri] = True
+    to = np.cumsum(used) - 1
+    return {"xyz": np.ascontiguousarray(m["xyz"][used]), "tri": to[tri].astype(np.uint32),
+            "on_boundary": np.ascontiguousarray(m["on_boundary"][used])}
+
+
+@pytest.mark.parametrize("mesh,precision,krylov,grid", [
+    ("lattice", _lib.FEM_PREC_FP32_IR, _lib.FEM_KRYLOV_CG, 64), ("lattice", _lib.FEM_PREC_FP64, _lib.FEM_KRYLOV_CG, 64),
+    ("lattice", _lib.FEM_PREC_FP32_IR, _lib.FEM_KRYLOV_CG_CLASSIC, 256),
+    ("long rows", _lib.FEM_PREC_FP32_IR, _lib.FEM_KRYLOV_CG, 256), ("long rows", _lib.FEM_PREC_FP64, _lib.FEM_KRYLOV_BICGSTAB, 256),
+    ("scattered", _lib.FEM_PREC_FP32_IR, _lib.FEM_KRYLOV_CG, 64), ("scattered", _lib.FEM_PREC_FP64, _lib.FEM_KRYLOV_CG, 256)])
+def test_team_of_rows_not_in_lds(gpu, mesh, precision, krylov, grid):
+    """About 39,000 unknowns: a team of 64 keeps 620 rows a workgroup in LDS, but
+    not with classic CG, rows of more than 10 entries, or, in FP64, the halo of a
+    scattered numbering (about 3,500 rows, where 1,141 fit).  Such teams get one
+    workgroup per 128 rows, and the solves without allocation the same plan."""
+    print("case rows not in LDS", mesh, precision, krylov, flush=True)
+    m = fan_square(200, 3) if mesh == "long rows" else meshes.jittered_square(198, seed=3)
+    m = scattered(m, 5) if mesh == "scattered" else m
+    info = check(m, False, 1, precision, krylov=krylov)
+    assert (info.grid, info.exchange) == (grid, _lib.FEM_EXCHANGE_COHERENT)
+    ctx = FEMContext(m, 0)
+    b = np.random.default_rng(16).standard_normal(ctx.num_unknowns())
+    got = [solve(gpu, ctx, fn, (1000.0, 0.05, 0.0), b, SolverOptions(precision=precision, krylov=krylov))
+           for fn in ("fem_ctx_solve", "fem_ctx_solve_noalloc")]
+    assert got[0][0] == got[1][0] == _lib.FEM_OK
+    assert np.array_equal(got[0][1], got[1][1])
+    ctx.close()
