@@ -813,12 +813,13 @@ int build_plan(fem_batch* b, bool flat = true) {
   // exchange mode: teams of several workgroups with more rows than the row
   // cache holds stream their phases: fenced barriers.  Plans of one-workgroup teams run the plain
   // variant.
-  bool rows = false, streaming = false;
+  bool rows = false, streaming = false, scattered = false;
   for (int t = 0; t < nteams; t++)
     for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++) {
       const bool fits = sizes[t] == 1 ? rows_fit(b->insts[team_inst[q]].ctx, k, 1, kr) : halo[q].ok != 0;
       rows |= fits;
       streaming |= sizes[t] > 1 && team_streams(b->insts[team_inst[q]].ctx->n, k, sizes[t]);
+      scattered |= sizes[t] > 1 && !fits && rows_fit(b->insts[team_inst[q]].ctx, k, sizes[t], kr);
     }
   // a team sized for rows in LDS, but the halo of a scattered numbering does not fit
   if (flat && multi && !rows) {
@@ -830,6 +831,13 @@ int build_plan(fem_batch* b, bool flat = true) {
     set_error("team plan exceeds the co-resident grid");
     return FEM_ERR_INVALID;
   }
+  // A scattered numbering whose halo does not fit gathers through the row cache,
+  // which the variant with rows in LDS has no registers for.  Its gathers, each
+  // from a line of its own, make it the plan's longest instance, so the plan
+  // takes the variant without (ms of 5 steps with it and without: 201 x 201
+  // lattice nodes beside 451 x 451 scattered ones 42.0 and 24.8; 101 x 101 and
+  // 221 x 221, 4 columns, 11.0 and 7.0).
+  if (mode == kExchangeCoherent && scattered) rows = false;
   b->uploaded = hi;
   b->launch.teams = b->d_teams;
   b->launch.wg_team = b->d_wg_team;

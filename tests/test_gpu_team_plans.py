@@ -6,8 +6,9 @@ of the oracle's."""
 import numpy as np
 import pytest
 
-from femhip import FEMContext, SolverOptions, _lib, meshes
-from test_gpu_team_rows import check, scattered
+import oracle
+from femhip import AdvectionDiffusionParameters, Batch, FEMContext, HeatParameters, SolverOptions, _lib, meshes
+from test_gpu_team_rows import TOL, VEL, check, rel, scattered
 from test_zz_no_alloc import solve
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +66,31 @@ def test_team_of_rows_not_in_lds(gpu, mesh, precision, krylov, grid):
     assert got[0][0] == got[1][0] == _lib.FEM_OK
     assert np.array_equal(got[0][1], got[1][1])
     ctx.close()
+
+
+@pytest.mark.parametrize("precision", [_lib.FEM_PREC_FP32_IR, _lib.FEM_PREC_FP64])
+@pytest.mark.parametrize("advdiff", [False, True])
+@pytest.mark.parametrize("order", [(0, 1, 2), (1, 2, 0)])
+def test_batch_of_fitting_and_other_halos(gpu, order, advdiff, precision):
+    """A lattice, a scattered numbering whose halo fits in FP32 and not in FP64
+    (about 1,000 rows per workgroup), and a mesh with a long row, in one plan."""
+    print("case mixed halos", order, advdiff, precision, flush=True)
+    mesh = [(meshes.jittered_square(30, seed=4)), scattered(meshes.jittered_square(78, seed=4), 7), fan_square(30, 4)]
+    mesh = [mesh[i] for i in order]
+    ctxs = [FEMContext(m, 0, velocity=VEL, normalize_velocity=False) for m in mesh]
+    b = Batch(ctxs, SolverOptions(precision=precision, tol=1e-12, team_size=6))
+    refs = []
+    for i, m in enumerate(mesh):
+        s = oracle.System(m, bc=0, velocity=VEL, normalize=False)
+        f = np.random.default_rng(17 + i).standard_normal(s.n)
+        b.set_equation(i, AdvectionDiffusionParameters(1e-3, 0.05) if advdiff else HeatParameters(1e-3, 0.05))
+        b.set_state_unknowns(i, _lib.FEM_FIELD_U, f)
+        kw = {"krylov": oracle.BICGSTAB} if advdiff else {}
+        refs.append(s.run(oracle.ADVDIFF if advdiff else oracle.HEAT, [1e-3, 0.05], 3, f.copy(), tol=1e-14, **kw)[1])
+    assert b.plan_info().grid == 18
+    assert b.advance(3) == _lib.FEM_OK
+    for i, ref in enumerate(refs):
+        assert rel(b.get_state_unknowns(i), ref) <= TOL, i
+    b.close()
+    for c in ctxs:
+        c.close()
