@@ -645,14 +645,15 @@ int build_plan(fem_batch* b, bool flat = true) {
   }
   std::vector<std::vector<int>> teams;  // instance lists
   std::vector<int> sizes;
-  // Plan within `maxb` co-resident workgroups.
-  auto make_plan = [&](int maxb) {
+  // Plan within `maxb` co-resident workgroups; alone: every instance in a
+  // one-workgroup team.
+  auto make_plan = [&](int maxb, bool alone = false) {
     teams.clear();
     sizes.clear();
     if (ninst == 1) {
       teams.push_back({0});
       sizes.push_back(single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, maxb, flat));
-    } else if (b->opts.team_size > 0 && (long long)b->opts.team_size * ninst <= maxb) {
+    } else if (!alone && b->opts.team_size > 0 && (long long)b->opts.team_size * ninst <= maxb) {
       for (int i = 0; i < ninst; i++) {
         teams.push_back({i});
         sizes.push_back(b->opts.team_size);
@@ -666,7 +667,7 @@ int build_plan(fem_batch* b, bool flat = true) {
       std::vector<int> small;
       double wsmall = 0.0;
       for (int i = 0; i < ninst; i++)
-        if (work[i] < share) {
+        if (alone || work[i] < share) {
           small.push_back(i);
           wsmall += work[i];
         } else {
@@ -674,8 +675,8 @@ int build_plan(fem_batch* b, bool flat = true) {
           sizes.push_back(1);
         }
       const int big = (int)teams.size();
-      int bins = std::max(1, std::min((int)small.size(), std::max(1, std::min((int)std::lround(wsmall / share),
-                                                                            budget - big))));
+      const int room = alone ? budget : std::min((int)std::lround(wsmall / share), budget - big);
+      const int bins = std::max(1, std::min((int)small.size(), room));
       int left = budget - big - (small.empty() ? 0 : bins);
       using Load = std::pair<double, int>;  // work per workgroup, team
       std::priority_queue<Load> heaviest;
@@ -714,6 +715,8 @@ int build_plan(fem_batch* b, bool flat = true) {
   if (multi) {
     make_plan(std::min(maxv[kExchangeCoherent], maxv[kExchangeFenced]));
     multi = any_multi();
+    // more instances than one workgroup per CU: the plain variant holds twice as many
+    if (!multi) make_plan(maxv[0], true);
   }
   const int forced = (b->opts.exchange == FEM_EXCHANGE_COHERENT || b->opts.exchange == FEM_EXCHANGE_FENCED)
                          ? b->opts.exchange : 0;

@@ -94,3 +94,27 @@ def test_batch_of_fitting_and_other_halos(gpu, order, advdiff, precision):
     b.close()
     for c in ctxs:
         c.close()
+
+
+@pytest.mark.parametrize("count,grid", [(256, 256), (257, 257), (300, 300), (512, 512), (513, 512)])
+@pytest.mark.parametrize("advdiff", [False, True])
+def test_more_instances_than_cus(gpu, advdiff, count, grid):
+    """Equal instances, past one per CU: one-workgroup teams, two of which fit a CU."""
+    print("case many instances", count, advdiff, flush=True)
+    m = meshes.jittered_square(17, seed=4)
+    ctx = FEMContext(m, 0, velocity=VEL, normalize_velocity=False)
+    s = oracle.System(m, bc=0, velocity=VEL, normalize=False)
+    b = Batch([ctx] * count, SolverOptions(tol=1e-12))
+    f = np.random.default_rng(18).standard_normal((count, s.n))
+    for i in range(count):
+        b.set_equation(i, AdvectionDiffusionParameters(1e-3, 0.05) if advdiff else HeatParameters(1e-3, 0.05))
+        b.set_state_unknowns(i, _lib.FEM_FIELD_U, f[i])
+    info = b.plan_info()
+    assert (info.grid, info.exchange) == (grid, 0)
+    assert b.advance(3) == _lib.FEM_OK
+    for i in (0, 255, count - 1):
+        kw = {"krylov": oracle.BICGSTAB} if advdiff else {}
+        ref = s.run(oracle.ADVDIFF if advdiff else oracle.HEAT, [1e-3, 0.05], 3, f[i].copy(), tol=1e-14, **kw)[1]
+        assert rel(b.get_state_unknowns(i), ref) <= TOL, i
+    b.close()
+    ctx.close()
