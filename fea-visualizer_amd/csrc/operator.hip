@@ -385,13 +385,15 @@ int stream_rows(int k) {
 // Schedule of a column count that was neither tuned nor set: the row-block
 // stream with non-temporal matrix loads.  16 lanes per row with 16 columns is
 // one column per lane, 4 bytes a gather where the stream has 16: 1000 x 1100
-// nodes, FP32, 120 us a product against 61; 700 x 700 FP64 116 against 56;
-// 64 x 64 FP32 3.3 against 2.7.  Callers hand x and y over at any alignment of
-// their type; the stream's vector accesses to them assume no more (the code is
-// the same as for aligned vectors).  Below 256 x 256 nodes and one column 4
-// lanes per row take 2.2 us against 2.8, both under the launch's own cost; the
-// other stream variants lie within 10% of this one either way.
-constexpr int kDefaultSchedule = FEM_SPMV_STREAM_NT;
+// nodes, FP32, 120 us a product against 61; 700 x 700 FP64 76 against 41; 15,600
+// rows FP64 4.6 against 3.2.  Below some 8,000 rows its 16 times as many
+// workgroups are the faster ones (3,969 rows, FP32, 2.2 us against 2.5; 7,921
+// rows 2.5 against 2.7, FP64 3.0 against 2.9).  Callers hand x and y over at any
+// alignment of their type; the stream's vector accesses to them assume no more
+// (the code is the same as for aligned vectors).  Below 256 x 256 nodes and one
+// column 4 lanes per row take 2.2 us against 2.8, both under the launch's own
+// cost; the other stream variants lie within 10% of this one either way.
+int default_schedule(const fem_operator* op, int k) { return k == 16 && op->n < 8192 ? 16 : FEM_SPMV_STREAM_NT; }
 
 template <typename T>
 int pipe_grid_k(int k, bool nt, int nblk, int* grid) {
@@ -503,7 +505,7 @@ int operator_apply_device(fem_operator* op, int k, const void* x, void* y) {
     set_error("operator: nrhs must be 1, 2, 4 or 16");
     return FEM_ERR_INVALID;
   }
-  const int g = op->lanes[k] ? op->lanes[k] : kDefaultSchedule;
+  const int g = op->lanes[k] ? op->lanes[k] : default_schedule(op, k);
   return launch(op, k, g, x, y);
 }
 
@@ -570,7 +572,7 @@ int operator_time(fem_operator* op, int k, const void* x, void* y, int reps, dou
     set_error("operator_time: nrhs must be 1, 2, 4 or 16 and reps >= 1");
     return FEM_ERR_INVALID;
   }
-  const int g = op->lanes[k] ? op->lanes[k] : kDefaultSchedule;
+  const int g = op->lanes[k] ? op->lanes[k] : default_schedule(op, k);
   return time_lanes(op, k, g, x, y, reps, ms);
 }
 
@@ -589,7 +591,7 @@ int operator_autotune(fem_operator* op, int k, const void* x, void* y, int reps,
     return FEM_ERR_INVALID;
   }
   double best = 1e300;
-  int bg = kDefaultSchedule;
+  int bg = default_schedule(op, k);
   for (int g : {1, 2, 4, 8, 16, (int)FEM_SPMV_STREAM, (int)FEM_SPMV_STREAM_NT, (int)FEM_SPMV_PIPE,
                 (int)FEM_SPMV_PIPE_NT}) {
     if (g < k) continue;
