@@ -95,93 +95,139 @@ unsigned reset_grid(int nrec, int rec_vals, int ninst) {
   return div_up(std::max(2LL * kSlotBufs * nrec * rec_vals, (long long)ninst), kBlock);
 }
 
-// Halos of one team-instance whose workgroups keep their rows in LDS
-// (HaloRef): workgroup `rank` collects the distinct columns outside its rows
-// in a hash table (at most rows x kCacheE of them, under two thirds of the
-// table), sorts them, and writes for every lane and entry the place of its
+// Halos of the team-instances whose workgroups may keep their rows in LDS
+// (HaloRef::cap > 0), one launch per plan: workgroup `rank` of a team marks the
+// columns outside its rows that they read in a bitmap of the unknowns (between
+// the first and the last of them), counts the bits before each word, and writes
+// the columns in ascending order and, for every lane and entry, the place of its
 // value in the staging area.  A halo beyond the capacity clears ref->ok: the
-// team then reads its neighbours from memory.  Run once per plan.
-constexpr int kHaloHash = 16384;
-__global__ void __launch_bounds__(kTeamBlock) k_halo(HaloRef* ref, int n, const int* rp, const int* ci,
-                                                     int rows_per_wg, int passes, int K, int* cnt_out, int* list,
-                                                     unsigned short* place) {
-  __shared__ int hash[kHaloHash], keys[kHaloHash];
-  __shared__ int cnt;
-  const int rank = blockIdx.x, tid = threadIdx.x;
-  const int lo = min(n, rank * rows_per_wg), hi = min(n, lo + rows_per_wg);
-  for (int i = tid; i < kHaloHash; i += kTeamBlock) hash[i] = -1;
-  if (tid == 0) cnt = 0;
-  __syncthreads();
-  for (int row = lo + tid; row < hi; row += kTeamBlock)
-    for (int s = rp[row]; s < rp[row + 1]; s++) {
-      const int c = ci[s];
-      if (c >= lo && c < hi) continue;
-      unsigned h = ((unsigned)c * 2654435761u) >> 18;
-      while (true) {
-        const int was = atomicCAS(&hash[h], -1, c);
-        if (was == -1) keys[atomicAdd(&cnt, 1)] = c;
-        if (was == -1 || was == c) break;
-        h = (h + 1) & (kHaloHash - 1);
-      }
-    }
-  __syncthreads();
-  const int total = cnt;
-  int m = 1;
-  while (m < total) m <<= 1;
-  for (int i = total + tid; i < m; i += kTeamBlock) keys[i] = INT32_MAX;
-  for (int k = 2; k <= m; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      __syncthreads();
-      for (int i = tid; i < m; i += kTeamBlock) {
-        const int p = i ^ j;
-        if (p > i) {
-          const int a = keys[i], b = keys[p];
-          if ((a > b) == ((i & k) == 0)) {
-            keys[i] = b;
-            keys[p] = a;
-          }
-        }
-      }
-    }
-  __syncthreads();
-  const int cap = ref->cap;
-  if (total > cap) {
-    if (tid == 0) {
-      ref->ok = 0;
-      cnt_out[rank] = 0;
-    }
-    return;
-  }
-  if (tid == 0) {
-    cnt_out[rank] = total;
-    atomicMax(&ref->max_n, total);
-  }
-  for (int i = tid; i < total; i += kTeamBlock) list[(size_t)rank * cap + i] = keys[i];
-  const int rpp = kTeamBlock / K;
-  for (int q = 0; q < passes; q++) {
-    const int row = lo + tid / K + q * rpp;
-    int s0 = 0, s1 = 0;
-    if (row < hi) {
-      s0 = rp[row];
-      s1 = rp[row + 1];
-    }
-    for (int e = 0; e < kCacheE; e++) {
-      int at = 0;
-      if (s0 + e < s1) {
-        const int c = ci[s0 + e];
-        if (c >= lo && c < hi) {
-          at = c - lo;
+// team then reads its neighbours from memory.
+//
+// Bound by latency: plan -> rows -> entries, and the launch (9 to 18 us).  A
+// launch per instance, each with a hash table for the largest team and a sort by
+// barriers, took 49 us: of the first advance of 60 meshes of 3,969 rows 1.9 ms,
+// 0.74 with this; of one with 99,225 rows 0.21 ms, 0.16.
+__global__ void __launch_bounds__(kTeamBlock) k_halo(const Team* teams, const int* wg_team, const Inst* insts,
+                                                     const int* team_inst) {
+  constexpr int kWords = kHaloRows / 32, W = kTeamBlock / kWave;
+  __shared__ unsigned bits[kWords];
+  __shared__ int before[kWords];
+  __shared__ int wsum[W], wmin[W], wmax[W];
+  const Team T = teams[wg_team[blockIdx.x]];
+  if (T.size <= 1 || !T.halo) return;
+  const int rank = (int)blockIdx.x - T.first_wg, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  for (int inst = T.inst_begin; inst < T.inst_end; inst++) {
+    HaloRef* ref = const_cast<HaloRef*>(T.halo) + inst;
+    const HaloRef R = *ref;
+    if (R.cap == 0) continue;
+    const Inst& I = insts[team_inst[inst]];
+    const int n = I.n, K = I.k;  // n <= kHaloRows (halo_shape)
+    const int *rp = I.rp, *ci = I.ci;
+    const int rows = (n + T.size - 1) / T.size;  // at most kCacheP per thread
+    const int lo = min(n, rank * rows), hi = min(n, lo + rows);
+    int c[kCacheP][kCacheE];  // columns of others' rows, else -1
+    int first = INT32_MAX, last = -1;
+#pragma unroll
+    for (int q = 0; q < kCacheP; q++) {
+      const int row = lo + tid + q * kTeamBlock;
+      const int s0 = row < hi ? rp[row] : 0, s1 = row < hi ? rp[row + 1] : 0;
+#pragma unroll
+      for (int e = 0; e < kCacheE; e++) c[q][e] = s0 < s1 ? ci[min(s0 + e, s1 - 1)] : lo;
+#pragma unroll
+      for (int e = 0; e < kCacheE; e++) {
+        if (s0 == s1 || (c[q][e] >= lo && c[q][e] < hi)) {
+          c[q][e] = -1;
         } else {
-          int a = 0, b = total;
-          while (a < b) {
-            const int mid = (a + b) >> 1;
-            if (keys[mid] < c) a = mid + 1;
-            else b = mid;
-          }
-          at = hi - lo + a;
+          first = min(first, c[q][e]);
+          last = max(last, c[q][e]);
         }
       }
-      place[(size_t)rank * ref->place_n + (q * kCacheE + e) * kTeamBlock + tid] = (unsigned short)at;
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+      first = min(first, __shfl_xor(first, d));
+      last = max(last, __shfl_xor(last, d));
+    }
+    __syncthreads();  // the previous instance's readers are done
+    if (lane == 0) {
+      wmin[wave] = first;
+      wmax[wave] = last;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+      first = min(first, wmin[w]);
+      last = max(last, wmax[w]);
+    }
+    // the bitmap's words between the first and the last of them
+    const int base = last < 0 ? 0 : first >> 5, words = last < 0 ? 0 : (last >> 5) - base + 1;
+    for (int w = tid; w < words; w += kTeamBlock) bits[w] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kCacheP; q++)
+#pragma unroll
+      for (int e = 0; e < kCacheE; e++)
+        if (c[q][e] >= 0) atomicOr(&bits[(c[q][e] >> 5) - base], 1u << (c[q][e] & 31));
+    __syncthreads();
+    // every thread counts a stretch of words, and the workgroup those before it
+    const int per = (words + kTeamBlock - 1) / kTeamBlock, w0 = min(words, tid * per), w1 = min(words, w0 + per);
+    int mine = 0;
+    for (int w = w0; w < w1; w++) mine += __popc(bits[w]);
+    int upto = mine;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int v = __shfl_up(upto, d);
+      if (lane >= d) upto += v;
+    }
+    if (lane == kWave - 1) wsum[wave] = upto;
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+      if (w < wave) upto += wsum[w];
+      total += wsum[w];
+    }
+    int* cnt_out = const_cast<int*>(R.n) + rank;
+    if (total > R.cap) {
+      if (tid == 0) {
+        ref->ok = 0;
+        *cnt_out = 0;
+      }
+      continue;
+    }
+    if (tid == 0) {
+      *cnt_out = total;
+      atomicMax(&ref->max_n, total);
+    }
+    int* list = const_cast<int*>(R.list) + (size_t)rank * R.cap;
+    int r = upto - mine;
+    for (int w = w0; w < w1; w++) {
+      before[w] = r;
+      for (unsigned b = bits[w]; b; b &= b - 1) list[r++] = 32 * (base + w) + __ffs(b) - 1;
+    }
+    __syncthreads();
+    unsigned short* place = const_cast<unsigned short*>(R.place) + (size_t)rank * R.place_n;
+    const int rpp = kTeamBlock / K;
+    for (int q = 0; q * kCacheE * kTeamBlock < R.place_n; q++) {
+      const int row = lo + tid / K + q * rpp;
+      int s0 = 0, s1 = 0;
+      if (row < hi) {
+        s0 = rp[row];
+        s1 = rp[row + 1];
+      }
+      int col[kCacheE];
+#pragma unroll
+      for (int e = 0; e < kCacheE; e++) col[e] = s0 < s1 ? ci[min(s0 + e, s1 - 1)] : 0;
+#pragma unroll
+      for (int e = 0; e < kCacheE; e++) {
+        int at = 0;
+        if (s0 + e < s1) {
+          const int w = (col[e] >> 5) - base;
+          at = col[e] >= lo && col[e] < hi ? col[e] - lo
+                                           : hi - lo + before[w] + __popc(bits[w] & ((1u << (col[e] & 31)) - 1));
+        }
+        place[(q * kCacheE + e) * kTeamBlock + tid] = (unsigned short)at;
+      }
     }
   }
 }
@@ -215,7 +261,7 @@ __global__ void __launch_bounds__(kBlock) k_clear_inst(double* u, double* v, dou
 void free_inst(InstHost& h) {
   void* ptrs[] = {h.d_S64, h.d_Si,    h.d_dinv64, h.d_dinvi, h.d_SDi, h.d_u, h.d_v,   h.d_a,
                   h.d_h3,  h.d_h4,    h.d_xnext,  h.d_hpre,  h.d_hvec, h.d_x, h.d_b, h.d_vec,
-                  h.d_surf, h.d_h5, h.d_h6, h.d_xch, h.d_normals};
+                  h.d_surf, h.d_h5, h.d_h6, h.d_normals};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (h.surf_done) (void)hipEventSynchronize(h.surf_done);
@@ -388,7 +434,7 @@ void fill_dev(fem_batch* b, InstHost& h) {
   I.h4 = h.d_h4;
   I.h5 = h.d_h5;
   I.h6 = h.d_h6;
-  I.xch = h.d_xch;
+  I.xch = h.xch;
   I.xnext = h.d_xnext;
   I.hpre = h.d_hpre;
   I.hvec = h.d_hvec;
@@ -425,9 +471,7 @@ void fill_dev(fem_batch* b, InstHost& h) {
 }
 
 void free_plan(fem_batch* b) {
-  void* ptrs[] = {b->d_plan, b->d_slots, b->d_halo_mem};
-  for (void* p : ptrs)
-    if (p) (void)hipFree(p);
+  if (b->d_plan) (void)hipFree(b->d_plan);
   b->d_plan = nullptr;
   b->d_insts = nullptr;
   b->d_teams = nullptr;
@@ -435,7 +479,7 @@ void free_plan(fem_batch* b) {
   b->d_team_inst = nullptr;
   b->d_slots = nullptr;
   b->d_halo = nullptr;
-  b->d_halo_mem = nullptr;
+  for (auto& h : b->insts) h.xch = nullptr;
   b->uploaded.clear();
   b->plan_ready = false;
 }
@@ -524,11 +568,11 @@ int exchange_mode(bool multi, bool streaming, int forced, int tuned) {
 }
 
 // The halos of one team-instance: whether its workgroups can keep their rows
-// in LDS at all, how many halo rows fit beside them (4 bytes of list and four
+// in LDS at all (kCacheP per lane of 256 CUs are kHaloRows), how many halo rows fit beside them (4 bytes of list and four
 // values of ti bytes per column each: the staged one and three Krylov
 // vectors), and the bytes its tables take.
 bool halo_shape(const fem_ctx* c, int k, int size, int ti, int kr, HaloShape* h) {
-  if (size <= 1 || c->n == 0 || !rows_fit(c, k, size, kr)) return false;
+  if (size <= 1 || c->n == 0 || c->n > kHaloRows || !rows_fit(c, k, size, kr)) return false;
   h->rows = (c->n + size - 1) / size;
   h->passes = (int)div_up((long long)h->rows * k, kTeamBlock);
   const int room = kTeamPool - rows_cells_bytes(h->passes, kTeamBlock, ti) - ti * h->rows * k;
@@ -553,11 +597,10 @@ HaloRef halo_ref(const HaloShape& h, void* mem) {
   return r;
 }
 
-// Fill the tables of `ref` (already at d_ref).
-int launch_halo(const fem_ctx* c, int k, int size, const HaloShape& h, const HaloRef& ref, HaloRef* d_ref,
+// Fill the halo tables of a plan of `grid` workgroups whose records are on the device.
+int launch_halo(const Team* teams, const int* wg_team, const Inst* insts, const int* team_inst, int grid,
                 hipStream_t st) {
-  hipLaunchKernelGGL(k_halo, dim3(size), dim3(kTeamBlock), 0, st, d_ref, c->n, c->d_rp, c->d_ci, h.rows, h.passes, k,
-                     const_cast<int*>(ref.n), const_cast<int*>(ref.list), const_cast<unsigned short*>(ref.place));
+  hipLaunchKernelGGL(k_halo, dim3(grid), dim3(kTeamBlock), 0, st, teams, wg_team, insts, team_inst);
   FEM_HIP(hipGetLastError());
   return 0;
 }
@@ -733,7 +776,8 @@ int build_plan(fem_batch* b, bool flat = true) {
     ht[t].inst_end = (int)team_inst.size();
     for (int q = 0; q < sizes[t]; q++) wg_team[wg++] = t;
   }
-  // the plan's tables in one block, sent in one copy
+  // the plan in one block: its tables, sent in one copy, then the barrier
+  // records, the halo tables and the exchange words
   size_t plan_bytes = 0;
   auto place = [&](size_t bytes) {
     const size_t at = plan_bytes;
@@ -744,33 +788,41 @@ int build_plan(fem_batch* b, bool flat = true) {
   const size_t o_insts = place(sizeof(Inst) * ninst), o_teams = place(sizeof(Team) * nteams);
   const size_t o_wg = place(sizeof(int) * grid), o_list = place(sizeof(int) * nlist);
   const size_t o_halo = place(sizeof(HaloRef) * nlist);
+  const size_t table_bytes = plan_bytes, o_slots = place(slot_bytes(grid, k));
+  // Halos of the teams whose workgroups may keep their rows in LDS, and the
+  // exchange words of their instances (each in one such team; at most kCacheP
+  // rows x columns per lane of the grid).  The other instances do without.
+  std::vector<HaloRef> halo(nlist);
+  std::vector<HaloShape> shape(nlist);
+  std::vector<size_t> o_tables(nlist), o_xch(nlist);
+  bool halos = false;
+  for (int t = 0; t < nteams; t++)
+    for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++) {
+      const fem_ctx* c = b->insts[team_inst[q]].ctx;
+      HaloShape& hs = shape[q];
+      if (!halo_shape(c, k, sizes[t], inner_fp32 ? 4 : 8, kr, &hs)) {
+        hs.cap = 0;
+        continue;
+      }
+      halos = true;
+      o_tables[q] = place(hs.n_bytes + hs.list_bytes + hs.place_bytes);
+      o_xch[q] = place(sizeof(unsigned long long) * xch_words(inner_fp32 ? 4 : 8) * (size_t)c->n * k);
+    }
   b->d_plan = dalloc<char>(plan_bytes, &rc);
-  b->d_slots = dalloc<double>(slot_bytes(grid, k) / sizeof(double), &rc);
   if (rc) return rc;
   b->d_insts = (Inst*)(b->d_plan + o_insts);
   b->d_teams = (Team*)(b->d_plan + o_teams);
   b->d_wg_team = (int*)(b->d_plan + o_wg);
   b->d_team_inst = (int*)(b->d_plan + o_list);
-  // halos of the teams whose workgroups keep their rows in LDS
-  std::vector<HaloRef> halo(nlist);
-  std::vector<HaloShape> shape(nlist);
-  size_t halo_bytes = 0;
-  for (int t = 0; t < nteams; t++)
-    for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++)
-      if (halo_shape(b->insts[team_inst[q]].ctx, k, sizes[t], inner_fp32 ? 4 : 8, kr, &shape[q]))
-        halo_bytes += shape[q].n_bytes + shape[q].list_bytes + shape[q].place_bytes;
-      else
-        shape[q].cap = 0;
-  if (halo_bytes > 0) {
-    b->d_halo = (HaloRef*)(b->d_plan + o_halo);
-    b->d_halo_mem = dalloc<char>(halo_bytes, &rc);
-    if (rc) return rc;
-    size_t at = 0;
-    for (size_t q = 0; q < nlist; q++) {
-      if (shape[q].cap == 0) continue;
-      halo[q] = halo_ref(shape[q], b->d_halo_mem + at);
-      at += shape[q].n_bytes + shape[q].list_bytes + shape[q].place_bytes;
+  b->d_slots = (double*)(b->d_plan + o_slots);
+  if (halos) b->d_halo = (HaloRef*)(b->d_plan + o_halo);
+  for (size_t q = 0; q < nlist; q++) {
+    InstHost& h = b->insts[team_inst[q]];
+    if (shape[q].cap > 0) {
+      halo[q] = halo_ref(shape[q], b->d_plan + o_tables[q]);
+      h.xch = (unsigned long long*)(b->d_plan + o_xch[q]);
     }
+    h.dev.xch = h.xch;
   }
   for (int t = 0; t < nteams; t++) {
     ht[t].halo = b->d_halo;
@@ -779,39 +831,22 @@ int build_plan(fem_batch* b, bool flat = true) {
     ht[t].wait_ticks = b->wait_ticks;
     ht[t].allpoll = b->poll_override == 1 ? 1 : b->poll_override == 2 ? 0 : flat_reduction(sizes[t], k);
   }
-  // exchange words of the instances whose teams may keep their rows in LDS (at
-  // most kCacheP per lane of the grid); the others do without
-  std::vector<char> wants(ninst, 0);
-  for (size_t q = 0; q < nlist; q++) wants[team_inst[q]] |= shape[q].cap > 0;
-  for (int i = 0; i < ninst; i++) {
-    InstHost& h = b->insts[i];
-    if (wants[i] && !h.d_xch) {
-      h.d_xch = dalloc<unsigned long long>((size_t)h.ctx->n * k * xch_words(inner_fp32 ? 4 : 8), &rc);
-      if (rc) return rc;
-    } else if (!wants[i] && h.d_xch) {
-      (void)hipFree(h.d_xch);
-      h.d_xch = nullptr;
-    }
-    h.dev.xch = h.d_xch;
-  }
   std::vector<Inst> hi(ninst);
   for (int i = 0; i < ninst; i++) hi[i] = persistent_desc(b->insts[i].dev);
-  std::vector<char> host(plan_bytes);
+  std::vector<char> host(table_bytes);
   std::memcpy(&host[o_insts], hi.data(), sizeof(Inst) * ninst);
   std::memcpy(&host[o_teams], ht.data(), sizeof(Team) * nteams);
   std::memcpy(&host[o_wg], wg_team.data(), sizeof(int) * grid);
   std::memcpy(&host[o_list], team_inst.data(), sizeof(int) * nlist);
   std::memcpy(&host[o_halo], halo.data(), sizeof(HaloRef) * nlist);
-  FEM_HIP(hipMemcpyAsync(b->d_plan, host.data(), plan_bytes, hipMemcpyHostToDevice, b->stream));
+  FEM_HIP(hipMemcpyAsync(b->d_plan, host.data(), table_bytes, hipMemcpyHostToDevice, b->stream));
   if (b->d_halo) {  // built on the device, which says which fit
-    for (int t = 0; t < nteams; t++)
-      for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++)
-        if (shape[q].cap > 0 &&
-            (rc = launch_halo(b->insts[team_inst[q]].ctx, k, sizes[t], shape[q], halo[q], b->d_halo + q, b->stream)))
-          return rc;
-    FEM_HIP(hipMemcpyAsync(halo.data(), b->d_halo, sizeof(HaloRef) * nlist, hipMemcpyDeviceToHost, b->stream));
+    rc = launch_halo(b->d_teams, b->d_wg_team, b->d_insts, b->d_team_inst, grid, b->stream);
+    if (rc) return rc;
+    FEM_HIP(hipMemcpyAsync(b->h_halo, b->d_halo, sizeof(HaloRef) * nlist, hipMemcpyDeviceToHost, b->stream));
   }
   FEM_HIP(hipStreamSynchronize(b->stream));
+  if (b->d_halo) halo.assign(b->h_halo, b->h_halo + nlist);
   // Whether any instance keeps its rows in LDS (the kernel variant), and the
   // exchange mode: teams of several workgroups with more rows than the row
   // cache holds stream their phases: fenced barriers.  Plans of one-workgroup teams run the plain
@@ -929,11 +964,13 @@ int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, f
   b->info_bytes = (size_t)count * kInfoBytes + sizeof(int);
   {
     int rc = 0;
+    // the host's copy, and behind it the halo records of a launch plan
+    const size_t halo_at = ((size_t)count + 1) * kInfoBytes, host_bytes = halo_at + sizeof(HaloRef) * (size_t)count;
     b->d_info = dalloc<char>(b->info_bytes, &rc);
     if (!rc && b->once) {
-      b->h_info = new char[b->info_bytes];
+      b->h_info = new char[host_bytes];
     } else if (!rc) {
-      e = hipHostMalloc((void**)&b->h_info, b->info_bytes, hipHostMallocDefault);
+      e = hipHostMalloc((void**)&b->h_info, host_bytes, hipHostMallocDefault);
       if (e != hipSuccess) rc = hip_fail(e, "batch_create: hipHostMalloc");
     }
     if (!rc) {
@@ -945,6 +982,7 @@ int batch_create(fem_ctx* const* ctxs, int count, const fem_solver_opts* opts, f
       return rc;
     }
     b->d_abort = (int*)(b->d_info + (size_t)count * kInfoBytes);
+    b->h_halo = (HaloRef*)(b->h_info + halo_at);
   }
   for (int i = 0; i < count; i++) {
     if (!ctxs[i]) {

@@ -149,6 +149,8 @@ __host__ __device__ constexpr int rows_pool_bytes(int block, int ti) {
   return rows_cells_bytes(kCacheP, block, ti) + 16 * kCacheP * block;
 }
 constexpr int kTeamPool = 145 * 1024;
+// Most rows of an instance whose workgroups keep them there (the bitmap of k_halo).
+constexpr int kHaloRows = 256 * kCacheP * kTeamBlock;
 
 // The halos of one team-instance (k_halo): per rank the rows of other
 // workgroups that its rows read, ascending, and per lane and entry the place

@@ -46,7 +46,7 @@ struct HaloShape {
 };
 bool halo_shape(const fem_ctx* c, int k, int size, int ti, int kr, HaloShape* h);
 HaloRef halo_ref(const HaloShape& h, void* mem);
-int launch_halo(const fem_ctx* c, int k, int size, const HaloShape& h, const HaloRef& ref, HaloRef* d_ref,
+int launch_halo(const Team* teams, const int* wg_team, const Inst* insts, const int* team_inst, int grid,
                 hipStream_t st);
 
 // Streaming engine (stream.hip): row-block table and per-instance scalars.
@@ -103,7 +103,7 @@ struct InstHost {
   double* d_xnext = nullptr; // Inst::xnext, Inst::hpre
   double* d_hpre = nullptr;
   double* d_hvec = nullptr;  // Inst::hvec
-  unsigned long long* d_xch = nullptr;  // Inst::xch
+  unsigned long long* xch = nullptr;  // Inst::xch, in the launch plan's block
   double* d_S64 = nullptr;
   void* d_Si = nullptr;
   double* d_dinv64 = nullptr;
@@ -143,7 +143,7 @@ struct fem_batch {
   hipStream_t stream = nullptr;
   bool once = false;  // serves one call: its context's stream, pageable h_info
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // launch plan: device arrays in d_plan, except the barrier records and the halo tables
+  // launch plan: device arrays in d_plan
   bool plan_ready = false;
   char* d_plan = nullptr;
   femhip::StepLaunch launch;
@@ -152,12 +152,12 @@ struct fem_batch {
   int* d_wg_team = nullptr;
   int* d_team_inst = nullptr;
   double* d_slots = nullptr;    // barrier records of the workgroups, then of the groups: 2 x [kSlotBufs][grid][slot_vals]
-  femhip::HaloRef* d_halo = nullptr;  // by position in the team-instance list; tables in d_halo_mem
-  char* d_halo_mem = nullptr;
+  femhip::HaloRef* d_halo = nullptr;  // by position in the team-instance list (null: no team may keep its rows)
   int grid = 0;
   int* d_abort = nullptr;       // in the info block
   char* d_info = nullptr;       // [ninst][kInfoBytes] + abort flag
   char* h_info = nullptr;       // host copy, pinned unless once
+  femhip::HaloRef* h_halo = nullptr;  // behind it: d_halo as k_halo left it
   size_t info_bytes = 0;
   std::vector<femhip::Inst> uploaded;  // descriptors last copied to the plan's d_insts
   int nteams = 0;

@@ -254,7 +254,7 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
                      dim3(kBlock), 0, st, T, I, halo, grid, d_team, d_wg_team, d_team_inst, d_inst, d_halo, I.u, nzero);
   FEM_HIP(hipGetLastError());
   if (halos) {
-    rc = launch_halo(c, k, grid, hs, halo, d_halo, st);
+    rc = launch_halo(d_team, d_wg_team, d_inst, d_team_inst, grid, st);
     if (rc) return rc;
   }
   rc = form_system(c, coef, fp32, (double*)I.S64, (void*)I.Si, (double*)I.dinv64, (void*)I.dinvi, st);

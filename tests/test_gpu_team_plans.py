@@ -118,3 +118,27 @@ def test_more_instances_than_cus(gpu, advdiff, count, grid):
         assert rel(b.get_state_unknowns(i), ref) <= TOL, i
     b.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("precision", [_lib.FEM_PREC_FP32_IR, _lib.FEM_PREC_FP64])
+@pytest.mark.parametrize("advdiff", [False, True])
+@pytest.mark.parametrize("cells,exchange", [(513, _lib.FEM_EXCHANGE_COHERENT), (514, _lib.FEM_EXCHANGE_FENCED)])
+def test_largest_mesh_in_lds_and_one_past_it(gpu, cells, exchange, advdiff, precision):
+    """262,144 unknowns are two rows per lane of every CU, the most that stay in
+    LDS; one lattice row more streams its phases.  Against the streaming engine:
+    solves to 1e-12, condition numbers below 15, two steps of two engines."""
+    print("case largest in LDS", cells, advdiff, precision, flush=True)
+    ctx = FEMContext(meshes.jittered_square(cells, seed=7), 0, velocity=VEL, normalize_velocity=False)
+    f = np.random.default_rng(19).standard_normal(ctx.num_unknowns())
+    got = []
+    for engine in (_lib.FEM_ENGINE_PERSISTENT, _lib.FEM_ENGINE_STREAM):
+        b = Batch([ctx], SolverOptions(precision=precision, tol=1e-12, engine=engine))
+        b.set_equation(0, AdvectionDiffusionParameters(1e-4, 0.05) if advdiff else HeatParameters(1e-4, 0.05))
+        b.set_state_unknowns(0, _lib.FEM_FIELD_U, f)
+        if engine == _lib.FEM_ENGINE_PERSISTENT:
+            assert (b.plan_info().grid, b.plan_info().exchange) == (256, exchange)
+        assert b.advance(2) == _lib.FEM_OK
+        got.append(b.get_state_unknowns(0))
+        b.close()
+    assert rel(got[0], got[1]) <= TOL
+    ctx.close()
