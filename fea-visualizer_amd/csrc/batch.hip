@@ -1818,14 +1818,15 @@ static int stream_graph_launch(fem_batch* b, fem_step_stats* stats) {
 
 // Autotuner: run `probe` steps under a few launch plans from the same state
 // (snapshotted and restored around every probe) and keep the fastest by
-// kernel time.  One instance: the team size around the one-row-per-lane
-// default; several: the number of workgroups the plan spreads the batch over.
+// kernel time.  One instance: team sizes around the untuned one; several: the
+// number of workgroups the plan spreads the batch over.
 int batch_autotune(fem_batch* b, int probe, int* chosen, double* best_ms) {
   if (b->opts.engine != FEM_ENGINE_PERSISTENT || probe <= 0) return 0;
   int rc = batch_prepare(b, true);
   if (rc) return rc;
-  int maxb = 0;
+  int maxb = 0, alone = 0;  // workgroups of teams of several, and of one-workgroup teams
   rc = variant_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, kExchangeCoherent, &maxb);
+  if (!rc) rc = variant_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, 0, &alone);
   if (rc) return rc;
   const bool single = b->insts.size() == 1;
   // Rows x columns per lane of the whole co-resident grid: beyond ~64 every
@@ -1844,15 +1845,13 @@ int batch_autotune(fem_batch* b, int probe, int* chosen, double* best_ms) {
       const int g = std::max(1, std::min(maxb, (int)std::lround(g0 * f)));
       if (std::find(cands.begin(), cands.end(), g) == cands.end()) cands.push_back(g);
     }
-    // one and two workgroups per CU: no CU hosts one workgroup more than
-    // another, so no straggler holds up the barriers
-    int dev = 0, cus = 0;
-    FEM_HIP(hipGetDevice(&dev));
-    FEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    for (int g : {cus / 2, cus, 2 * cus})
-      if (g >= 1 && g <= maxb && std::find(cands.begin(), cands.end(), g) == cands.end()) cands.push_back(g);
+    // one workgroup per CU, and on every second
+    for (int g : {maxb / 2, maxb})
+      if (g >= 1 && std::find(cands.begin(), cands.end(), g) == cands.end()) cands.push_back(g);
   } else {
     for (double f : {0.25, 0.5, 0.75, 1.0}) cands.push_back(std::max(1, (int)(maxb * f)));
+    // more instances than teams of several: the untuned plan's one-workgroup teams
+    if ((int)b->insts.size() > maxb && alone > maxb) cands.push_back(alone);
   }
   // snapshot the state
   std::vector<double*> snap;

@@ -142,3 +142,26 @@ def test_largest_mesh_in_lds_and_one_past_it(gpu, cells, exchange, advdiff, prec
         b.close()
     assert rel(got[0], got[1]) <= TOL
     ctx.close()
+
+
+def test_autotuner_tries_the_untuned_plan(gpu):
+    """300 small instances: the plan of 300 one-workgroup teams is among the
+    candidates.  Within one workgroup per CU a quarter of the teams walks two
+    instances, twice the time; the limit leaves half of that for the clock."""
+    print("case autotune many", flush=True)
+    ctx = FEMContext(meshes.jittered_square(20, seed=4), 0)
+    b = Batch([ctx] * 300, SolverOptions())
+    f = np.random.default_rng(20).standard_normal(ctx.num_unknowns())
+    ms = []
+    for rep in range(4):
+        for i in range(300):
+            b.set_equation(i, HeatParameters(1e-3, 0.05))
+            b.set_state_unknowns(i, _lib.FEM_FIELD_U, f)
+        assert b.advance(10) == _lib.FEM_OK
+        ms.append(b.last_stats.ms)
+    for i in range(300):
+        b.set_state_unknowns(i, _lib.FEM_FIELD_U, f)
+    _, best = b.autotune(10)
+    assert best <= 1.5 * min(ms), (best, ms)
+    b.close()
+    ctx.close()
