@@ -486,6 +486,25 @@ void free_plan(fem_batch* b) {
 
 }  // namespace
 
+// Whether every workgroup of a team sums all records: one group's worth, or up
+// to 256 values, four per lane of the control wave; beyond, two levels.  The
+// flat form is one publish and poll, but every workgroup reads every record
+// (pipelined CG on 39,601 rows: 4.3 us an iteration flat at 64 workgroups, 5.3
+// at 128 and 6.8 at 256; in two levels 4.5 and 4.7).  16 columns have a lane per
+// value, and more than eight of a lane's loads in flight spill: flat up to 24
+// workgroups (10 steps on 529 rows, ms: 16 workgroups 1.03, 24 1.10 flat and 1.18 in
+// two levels, 46 1.43 and 1.20).
+constexpr int kFlat16 = 24;
+int flat_reduction(int size, int k) {
+  return size <= kGroup || (long long)size * 4 * k <= 256 || (k == 16 && size <= kFlat16);
+}
+
+// The team sizes with a flat reduction that a lone instance's team may be kept
+// at, best first: attempt 0, 1, ...; 0 when there are no more.
+int flat_team(int k, int attempt) {
+  return attempt == 0 ? std::max(kGroup, 256 / (4 * k)) : attempt == 1 && k == 16 ? kFlat16 : 0;
+}
+
 // Workgroups of the team of a lone instance, within maxb co-resident
 // workgroups: team_size when given and it fits.  Else one up to kCacheP rows x
 // columns per lane: its barriers stay on the CU (us a step, one workgroup and
@@ -494,33 +513,27 @@ void free_plan(fem_batch* b) {
 // LDS, 256 rows 75 and 144, 484 rows 134 and 144; a workgroup past its rows in
 // LDS takes twice as long as two).  Else one per 128 rows x columns, up to one
 // per CU.  Few rows per workgroup leave most of its waves to the halo and the
-// control wave.  Where that would leave the flat reduction
-// (flat_reduction), its largest team is kept (flat) while its workgroups stay
-// short: the second level costs an iteration more than the longer gathers do (one
-// column, us per iteration: 9,801 rows 4.7 at 64 workgroups, 5.3 at 128;
-// 39,601 rows 4.3 and 4.5; 89,401 rows take two-level teams; two columns:
-// 2,562 rows 5.4 at 20 workgroups and 6.3 at 40, 10,242 rows 9.1 at 40 and
-// 7.6 at 160).  That holds for gathers from LDS alone: from memory they are most
-// of an iteration, and more workgroups have more of them in flight (us per
-// iteration at 64 and 256 workgroups: 16,000 rows of a Delaunay mesh, up to 12
-// entries a row, 11.3 and 8.5; 40,000 rows 23.8 and 11.6; classic CG on 39,601
-// scattered rows 27.7 and 16.0).
-int single_team_size(long long n, int k, int team_size, int maxb, bool flat) {
+// control wave.
+//
+// Where that would leave the flat reduction, a team of `flat` workgroups
+// (flat_team) is kept while they stay short: the second level costs an iteration
+// more than the longer gathers do (one column, us per iteration: 9,801 rows 4.7
+// at 64 workgroups, 5.3 at 128; 39,601 rows 4.3 and 4.5; 89,401 rows take
+// two-level teams; two columns: 2,562 rows 5.4 at 20 workgroups and 6.3 at 40,
+// 10,242 rows 9.1 at 40 and 7.6 at 160; 16 columns, ms a run: 361 rows 0.92 at 16
+// and 1.12 at 46, 1,024 rows 1.08 at 16 and 1.33 at 128).  That holds for gathers
+// from LDS alone: from memory they are most of an iteration, and more workgroups
+// have more of them in flight (us per iteration at 64 and 256 workgroups: 16,000
+// rows of a Delaunay mesh, up to 12 entries a row, 11.3 and 8.5; 40,000 rows 23.8
+// and 11.6; classic CG on 39,601 scattered rows 27.7 and 16.0).
+int single_team_size(long long n, int k, int team_size, int maxb, int flat) {
   if (team_size > 0 && team_size <= maxb) return team_size;
   const long long lanes = n * k;
   if (lanes <= kCacheP * kBlock) return 1;
   int g = (int)std::min<long long>(1024, (lanes + 127) / 128);
-  const int f = std::max(kGroup, 256 / (4 * k));
-  if (flat && g > f && lanes <= (long long)f * (k == 1 ? 640 : 320)) g = f;
+  if (g > flat && lanes <= (long long)flat * (k == 1 ? 640 : k == 16 ? kCacheP * kTeamBlock : 320)) g = flat;
   return std::min(g, maxb);
 }
-
-// Whether every workgroup of a team sums all records: one group's worth, or up
-// to 256 values, four per lane of the control wave; beyond, two levels.  The
-// flat form is one publish and poll, but every workgroup reads every record
-// (pipelined CG on 39,601 rows: 4.3 us an iteration flat at 64 workgroups, 5.3
-// at 128 and 6.8 at 256; in two levels 4.5 and 4.7).
-int flat_reduction(int size, int k) { return size <= kGroup || (long long)size * 4 * k <= 256 ? 1 : 0; }
 
 // Barrier records of a launch of `grid` workgroups, and a team's among them.
 size_t slot_bytes(int grid, int k) { return sizeof(double) * 2 * kSlotBufs * (size_t)grid * slot_vals(k); }
@@ -651,9 +664,9 @@ static Inst persistent_desc(const Inst& d) {
   return I;
 }
 
-// flat: a lone instance's team may be kept at the flat reduction's largest, if
-// its rows may stay in LDS there.
-int build_plan(fem_batch* b, bool flat = true) {
+// attempt: which of the flat reduction's teams (flat_team) a lone instance may be
+// kept at, if its rows may stay in LDS there.
+int build_plan(fem_batch* b, int attempt = 0) {
   free_plan(b);
   const int ninst = (int)b->insts.size();
   const int k = b->insts[0].k;
@@ -669,7 +682,7 @@ int build_plan(fem_batch* b, bool flat = true) {
       return FEM_ERR_INVALID;
     }
   const int inner_fp32 = inner_bytes(b) == 4;
-  flat = flat && ninst == 1 && rows_possible(b->insts[0].ctx, kr);
+  const int flat = ninst == 1 && rows_possible(b->insts[0].ctx, kr) ? flat_team(k, attempt) : 0;
   // co-resident workgroups of each variant: plain (one-workgroup teams),
   // coherent and fenced exchange; they differ in registers
   int maxv[3] = {0, 0, 0};
@@ -860,9 +873,9 @@ int build_plan(fem_batch* b, bool flat = true) {
       scattered |= sizes[t] > 1 && !fits && rows_fit(b->insts[team_inst[q]].ctx, k, sizes[t], kr);
     }
   // a team sized for rows in LDS, but the halo of a scattered numbering does not fit
-  if (flat && multi && !rows) {
+  if (flat > 0 && multi && !rows) {
     const int maxb = std::min(maxv[kExchangeCoherent], maxv[kExchangeFenced]);
-    if (single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, maxb, false) != grid) return build_plan(b, false);
+    if (single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, maxb, 0) != grid) return build_plan(b, attempt + 1);
   }
   const int mode = exchange_mode(multi, streaming, forced, b->mode_override);
   if (grid > maxv[mode]) {

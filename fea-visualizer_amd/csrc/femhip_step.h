@@ -27,7 +27,8 @@ constexpr int kExchangeCoherent = 1, kExchangeFenced = 2;
 int launch_step(const StepLaunch& L, int nsteps, hipStream_t st);
 
 // Plan rules shared by the batch plans and the allocation-free solve (batch.hip).
-int single_team_size(long long n, int k, int team_size, int maxb, bool flat);
+int single_team_size(long long n, int k, int team_size, int maxb, int flat);
+int flat_team(int k, int attempt);
 int flat_reduction(int size, int k);
 size_t slot_bytes(int grid, int k);
 void team_slots(Team* T, double* slots, int grid, int k);

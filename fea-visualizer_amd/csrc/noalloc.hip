@@ -89,9 +89,9 @@ __global__ void k_noalloc_setup(Team team, Inst inst, HaloRef halo, int grid, Te
   for (long long q = i; q < nzero; q += (long long)gridDim.x * blockDim.x) zero[q] = 0.0;
 }
 
-// flat as in build_plan: the same plan, so the same results bit for bit.
+// attempt as in build_plan: the same plan, so the same results bit for bit.
 int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
-                  fem_step_stats* stats, bool flat) {
+                  fem_step_stats* stats, int attempt) {
   fem_solver_opts o;
   fem_opts_default(&o);
   if (opts) o = *opts;
@@ -116,7 +116,7 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
   int kr = o.krylov;
   if (kr == FEM_KRYLOV_AUTO) kr = coef[2] != 0.0 ? FEM_KRYLOV_BICGSTAB : FEM_KRYLOV_CG;
   const int kri = (kr == FEM_KRYLOV_BICGSTAB) ? 1 : (kr == FEM_KRYLOV_CG_CLASSIC) ? 2 : 0;
-  flat = flat && rows_possible(c, kri);
+  const int flat = rows_possible(c, kri) ? flat_team(k, attempt) : 0;
 
   // plan: one team, sized and moded as a one-instance batch plan
   int maxv[3] = {0, 0, 0};
@@ -268,8 +268,8 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
     FEM_HIP(hipStreamSynchronize(st));
   }
   const bool rows = grid == 1 ? rows_fit(c, k, 1, kri) : built.ok != 0;
-  if (flat && grid > 1 && !rows && single_team_size(n, k, o.team_size, maxv[mode], false) != grid)
-    return solve_noalloc(c, coef, opts, bh, xh, stats, false);
+  if (flat > 0 && grid > 1 && !rows && single_team_size(n, k, o.team_size, maxv[mode], 0) != grid)
+    return solve_noalloc(c, coef, opts, bh, xh, stats, attempt + 1);
   StepLaunch SL;
   SL.teams = d_team;
   SL.wg_team = d_wg_team;
@@ -315,7 +315,7 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
 
 int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
                          fem_step_stats* stats) {
-  return solve_noalloc(c, coef, opts, bh, xh, stats, true);
+  return solve_noalloc(c, coef, opts, bh, xh, stats, 0);
 }
 
 }  // namespace femhip

@@ -165,3 +165,27 @@ def test_autotuner_tries_the_untuned_plan(gpu):
     assert best <= 1.5 * min(ms), (best, ms)
     b.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("mesh,precision,krylov,grid", [
+    ((20, False), _lib.FEM_PREC_FP32_IR, _lib.FEM_KRYLOV_CG, 16), ((20, False), _lib.FEM_PREC_FP64, _lib.FEM_KRYLOV_BICGSTAB, 16),
+    ((33, False), _lib.FEM_PREC_FP64, _lib.FEM_KRYLOV_CG, 16), ((34, False), _lib.FEM_PREC_FP32_IR, _lib.FEM_KRYLOV_CG, 137),
+    ((24, True), _lib.FEM_PREC_FP32_IR, _lib.FEM_KRYLOV_CG, 16), ((24, True), _lib.FEM_PREC_FP64, _lib.FEM_KRYLOV_CG, 24),
+    ((33, True), _lib.FEM_PREC_FP64, _lib.FEM_KRYLOV_BICGSTAB, 128)])
+def test_sixteen_column_teams(gpu, mesh, precision, krylov, grid):
+    """(cells - 1)^2 unknowns x 16, scattered or not: 16 workgroups while two
+    rows x columns per lane suffice, 24 (also summed in one level) where the halo
+    does not fit those 16 in FP64, one per 128 rows x columns beyond."""
+    cells, shuffled = mesh
+    print("case sixteen columns", cells, shuffled, precision, krylov, flush=True)
+    m = meshes.jittered_square(cells, seed=8)
+    m = scattered(m, 6) if shuffled else m
+    info = check(m, False, 16, precision, krylov=krylov)
+    assert (info.grid, info.exchange) == (grid, _lib.FEM_EXCHANGE_COHERENT)
+    ctx = FEMContext(m, 0)
+    b = np.random.default_rng(21).standard_normal((ctx.num_unknowns(), 16))
+    got = [solve(gpu, ctx, fn, (1000.0, 0.05, 0.0), b, SolverOptions(precision=precision, krylov=krylov))
+           for fn in ("fem_ctx_solve", "fem_ctx_solve_noalloc")]
+    assert got[0][0] == got[1][0] == _lib.FEM_OK
+    assert np.array_equal(got[0][1], got[1][1])
+    ctx.close()
