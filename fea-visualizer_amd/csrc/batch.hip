@@ -298,7 +298,6 @@ int alloc_inst(fem_batch* b, InstHost& h, int k, int kv) {
   h.d_Si = (void*)dalloc<char>((size_t)nnz * kv * tb, &rc);
   h.d_dinv64 = dalloc<double>((size_t)n * kv, &rc);
   h.d_dinvi = (void*)dalloc<char>((size_t)n * kv * tb, &rc);
-  if (kv == 1 && stream_vec_layout(k)) h.d_SDi = (void*)dalloc<char>((size_t)nnz * tb, &rc);
   h.d_u = dalloc<double>((size_t)n * k, &rc);
   h.d_v = dalloc<double>((size_t)n * k, &rc);
   h.d_a = dalloc<double>((size_t)n * k, &rc);
@@ -320,6 +319,20 @@ int alloc_inst(fem_batch* b, InstHost& h, int k, int kv) {
                      b->stream, h.d_u, h.d_v, h.d_a, h.d_x, h.d_b, nk, (float*)h.d_vec, nvec, (int*)info);
   FEM_HIP(hipGetLastError());
   h.dirty = true;
+  return 0;
+}
+
+// Inst::SDi from the formed matrix.
+int form_scaled(fem_batch* b, InstHost& h) {
+  fem_ctx* c = h.ctx;
+  if (c->nnz == 0) return 0;
+  if (inner_bytes(b) == 4)
+    hipLaunchKernelGGL(k_colscale<float>, dim3(div_up(c->nnz, kBlock)), dim3(kBlock), 0, b->stream, (int)c->nnz, c->d_ci,
+                       (const float*)h.d_Si, (const float*)h.d_dinvi, (float*)h.d_SDi);
+  else
+    hipLaunchKernelGGL(k_colscale<double>, dim3(div_up(c->nnz, kBlock)), dim3(kBlock), 0, b->stream, (int)c->nnz, c->d_ci,
+                       (const double*)h.d_Si, (const double*)h.d_dinvi, (double*)h.d_SDi);
+  FEM_HIP(hipGetLastError());
   return 0;
 }
 
@@ -372,14 +385,9 @@ int form_inst(fem_batch* b, InstHost& h) {
                          c->d_diag, tp, c->d_M, c->d_K, c->d_A, h.kv, cf, h.d_S64, (double*)h.d_Si, h.d_dinv64,
                          (double*)h.d_dinvi);
     FEM_HIP(hipGetLastError());
-    if (h.d_SDi && c->nnz > 0) {
-      if (inner_bytes(b) == 4)
-        hipLaunchKernelGGL(k_colscale<float>, dim3(div_up(c->nnz, kBlock)), dim3(kBlock), 0, b->stream, (int)c->nnz,
-                           c->d_ci, (const float*)h.d_Si, (const float*)h.d_dinvi, (float*)h.d_SDi);
-      else
-        hipLaunchKernelGGL(k_colscale<double>, dim3(div_up(c->nnz, kBlock)), dim3(kBlock), 0, b->stream, (int)c->nnz,
-                           c->d_ci, (const double*)h.d_Si, (const double*)h.d_dinvi, (double*)h.d_SDi);
-      FEM_HIP(hipGetLastError());
+    if (h.d_SDi) {
+      const int rc = form_scaled(b, h);
+      if (rc) return rc;
     }
   }
   h.formed_version = c->version;
@@ -1408,6 +1416,16 @@ int batch_prepare(fem_batch* b, bool need_plan) {
       if (rc) return rc;
       b->plan_gen++;  // the plan stays (no value enters it), a recorded advance goes stale
     }
+    // Inst::SDi is the streaming engine's alone.  Held by every solver it put
+    // the solvers of 200,000 rows and more past the 64 MB of freed blocks that
+    // HIP keeps for the next allocation, where each hipFree takes 0.3-0.8 ms:
+    // create, one advance and close of 254,016 rows 1.72 ms, 1.30 without it.
+    if (b->opts.engine == FEM_ENGINE_STREAM && h.kv == 1 && stream_vec_layout(h.k) && !h.d_SDi) {
+      int rc = 0;
+      h.d_SDi = (void*)dalloc<char>((size_t)h.ctx->nnz * inner_bytes(b), &rc);
+      if (!rc) rc = form_scaled(b, h);
+      if (rc) return rc;
+    }
     fill_dev(b, h);
   }
   if (!need_plan) return 0;
@@ -1974,6 +1992,12 @@ int batch_autotune(fem_batch* b, int probe, int* chosen, double* best_ms) {
   if (!rc && stream_best) {
     b->opts.engine = FEM_ENGINE_STREAM;
     b->opts.team_size = 0;
+  } else {
+    for (auto& h : b->insts) {  // the probes' matrix: the persistent kernel has no use for it
+      (void)hipFree(h.d_SDi);
+      h.d_SDi = nullptr;
+      h.dev.SDi = nullptr;
+    }
   }
   b->plan_ready = false;
   if (chosen) *chosen = (!rc && stream_best) ? 0 : best_c;
