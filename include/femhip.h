@@ -125,7 +125,10 @@ typedef struct fem_solver_opts {
   int32_t max_inner;     /* FP32 iterations per refinement sweep; 0 = 200 */
   int32_t max_sweeps;    /* refinement sweeps per solve; 0 = 30 */
   int32_t team_size;     /* persistent engine: workgroups per instance; stream engine: rows per
-                            workgroup; 0 = autotuned / by column count */
+                            workgroup; 0 = autotuned / by column count.  A request that does not
+                            fit the device at once (team_size x instances beyond
+                            fem_plan_info.coresident of a plan with teams of several workgroups:
+                            one per CU, 256) is as 0 */
   double tol;            /* relative residual |b - Ax| <= tol |b| in FP64; 0 = 1e-10 */
   double inner_tol;      /* FP32 sweep reduction; 0 = 1e-4 */
   int32_t exchange;      /* multi-workgroup teams: FEM_EXCHANGE_AUTO (row-cache rule or

@@ -189,3 +189,31 @@ def test_sixteen_column_teams(gpu, mesh, precision, krylov, grid):
     assert got[0][0] == got[1][0] == _lib.FEM_OK
     assert np.array_equal(got[0][1], got[1][1])
     ctx.close()
+
+
+@pytest.mark.parametrize("instances,team_size,grid", [(1, 256, 256), (1, 257, 64), (2, 128, 256), (2, 129, 256)])
+def test_team_size_beyond_the_device_is_the_plans_own(gpu, instances, team_size, grid):
+    """128 x 128 unknowns: a request that fits is taken; beyond one workgroup per
+    CU the plan is that of team_size 0 (alone the 64 workgroups of the flat
+    reduction, two share all by their work) and so are the results, bit for bit."""
+    print("case team size", instances, team_size, flush=True)
+    ctx = FEMContext(meshes.jittered_square(129, seed=2), 0)
+    f = np.random.default_rng(21).standard_normal(ctx.num_unknowns())
+    got = []
+    for size in (team_size, 0):
+        b = Batch([ctx] * instances, SolverOptions(team_size=size, tol=1e-12))
+        for i in range(instances):
+            b.set_equation(i, HeatParameters(1e-3, 0.05))
+            b.set_state_unknowns(i, _lib.FEM_FIELD_U, f)
+        info = b.plan_info()
+        if size:
+            assert (info.grid, info.coresident) == (grid, 256)
+        elif team_size * instances > 256:
+            assert info.grid == grid
+        assert b.advance(2) == _lib.FEM_OK
+        got.append(b.get_state_unknowns(instances - 1))
+        b.close()
+    assert rel(got[0], got[1]) <= TOL
+    if team_size * instances > 256:
+        assert np.array_equal(got[0], got[1])
+    ctx.close()
