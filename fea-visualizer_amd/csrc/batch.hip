@@ -572,7 +572,9 @@ bool rows_fit(const fem_ctx* c, int k, int size, int kr) {
 }
 
 // Co-resident workgroups that both variants of an exchange mode (rows in LDS
-// or not) hold.
+// or not) hold.  Teams of several workgroups: one workgroup of 512 threads per
+// CU in either, the pool of kTeamPool bytes in the one and more than 128
+// registers a lane in the other allow no second.
 int variant_coresident(int k, int inner_fp32, int kr, int coh, int* blocks) {
   int rc = step_max_coresident(k, inner_fp32, kr, coh, 0, blocks);
   int with_rows = *blocks;
@@ -589,9 +591,9 @@ int exchange_mode(bool multi, bool streaming, int forced, int tuned) {
 }
 
 // The halos of one team-instance: whether its workgroups can keep their rows
-// in LDS at all (kCacheP per lane of 256 CUs are kHaloRows), how many halo rows fit beside them (4 bytes of list and four
-// values of ti bytes per column each: the staged one and three Krylov
-// vectors), and the bytes its tables take.
+// in LDS at all (kCacheP per lane of 256 CUs are kHaloRows), how many halo rows
+// fit beside them (4 bytes of list and four values of ti bytes per column each:
+// the staged one and three Krylov vectors), and the bytes its tables take.
 bool halo_shape(const fem_ctx* c, int k, int size, int ti, int kr, HaloShape* h) {
   if (size <= 1 || c->n == 0 || c->n > kHaloRows || !rows_fit(c, k, size, kr)) return false;
   h->rows = (c->n + size - 1) / size;
@@ -658,12 +660,6 @@ int launch_slot_reset(double* slots, int nrec, int rec_vals, int* abort_flag, In
 
 namespace {
 
-// Team plan.  Work of an instance ~ (nnz + n) * k per Krylov iteration.  With
-// one instance the team takes ~4 rows per lane, capped by the co-resident
-// grid.  With many, instances heavier than the per-workgroup share get teams
-// proportional to their work; the rest are packed longest-first onto
-// single-workgroup teams (each walks its instances in turn).
-
 // The persistent kernel's copy of a descriptor: its predictor is quartic at
 // most (the history levels beyond h4 belong to the streaming engine).
 static Inst persistent_desc(const Inst& d) {
@@ -672,6 +668,11 @@ static Inst persistent_desc(const Inst& d) {
   return I;
 }
 
+// Team plan.  Work of an instance ~ (nnz + n) * k per Krylov iteration.  One
+// instance takes a team of single_team_size.  Of many, instances heavier than
+// the per-workgroup share get teams of their own, one workgroup more at a time
+// where the work per workgroup is largest; the rest are packed longest-first
+// onto single-workgroup teams (each walks its instances in turn).
 // attempt: which of the flat reduction's teams (flat_team) a lone instance may be
 // kept at, if its rows may stay in LDS there.
 int build_plan(fem_batch* b, int attempt = 0) {
@@ -870,8 +871,8 @@ int build_plan(fem_batch* b, int attempt = 0) {
   if (b->d_halo) halo.assign(b->h_halo, b->h_halo + nlist);
   // Whether any instance keeps its rows in LDS (the kernel variant), and the
   // exchange mode: teams of several workgroups with more rows than the row
-  // cache holds stream their phases: fenced barriers.  Plans of one-workgroup teams run the plain
-  // variant.
+  // cache holds stream their phases: fenced barriers.  Plans of one-workgroup
+  // teams run the plain variant.
   bool rows = false, streaming = false, scattered = false;
   for (int t = 0; t < nteams; t++)
     for (int q = ht[t].inst_begin; q < ht[t].inst_end; q++) {

@@ -30,9 +30,10 @@ static __device__ __align__(256) unsigned char scratch[size_t(32) << 20];
 namespace {
 
 // Largest footprint a call may lay out: 32 MiB per GPU.  One right-hand side
-// of an FP32 + refinement solve uses about 12 nnz + 80 N bytes plus 0.5 KiB
-// per workgroup of barrier records, so meshes up to roughly 180,000 unknowns
-// fit at one column (about 25,000 at sixteen).
+// of an FP32 + refinement solve uses about 12 nnz + 80 N bytes plus the barrier
+// records (slot_bytes: 1 KiB per workgroup up to four columns, 4 KiB at
+// sixteen), so meshes up to roughly 180,000 unknowns fit at one column (about
+// 25,000 at sixteen).
 constexpr size_t kScratchBytes = size_t(32) << 20;
 
 constexpr int kMaxDevices = 64;

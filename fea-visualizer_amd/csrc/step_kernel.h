@@ -1,6 +1,7 @@
 // step_kernel.h -- persistent, cooperative time-stepping kernel (included by
-// one translation unit per exchange mode: step_plain.hip, step_coherent.hip,
-// step_fenced.hip).
+// two translation units per exchange mode, without and with rows in LDS:
+// step_plain.hip, step_coherent.hip, step_fenced.hip and step_plain_rows.hip,
+// step_coherent_rows.hip, step_fenced_rows.hip).
 //
 // One launch advances every instance of a batch by `nsteps` implicit time
 // steps.  The grid is split into teams (contiguous workgroup ranges); a team
@@ -1897,9 +1898,11 @@ FEM_INLINE bool krylov_pcg(const Inst& I, const Team& T, int rank, unsigned& e, 
 // started: the update phase already formed w = S D^-1 r and the start
 // scalars (x holds the initial guess, xi = 0).
 // Latency-bound: publishing the sums, polling them and the words (~1.5 us), the
-// scalars, and the LDS gather.  us per iteration, three coherent loads per
-// entry from memory and now: 3,969 FP64 rows 6.3 -> 3.2; 39,601 rows 7.3 ->
-// 4.3; 259,000 rows 12.2 -> 5.1; BiCGSTAB on 261,000 rows 48 -> 15.
+// scalars, and the LDS gather.  Device time of a run over its iterations, the
+// residuals and right-hand sides included (us; three coherent loads per entry
+// from memory, and now): 3,969 FP64 rows 6.3 -> 3.1; 39,601 rows 7.3 -> 4.3;
+// 259,000 rows 12.2 -> 5.1; BiCGSTAB on 261,000 rows 48 -> 16.  An iteration of
+// the loop alone (140 against 40 in one sweep): 2.7, 3.0, 4.1 and 10.4.
 template <int K, typename TI, int C>
 FEM_INLINE bool krylov_pcg_rows(const Inst& I, const Team& T, int rank, unsigned& e, TeamShared& sh, int row_lo,
                                 int row_hi, int& its, const Rows<TI>& R, bool started) {
