@@ -9,6 +9,7 @@
 #include "femhip_step.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -571,18 +572,6 @@ bool rows_fit(const fem_ctx* c, int k, int size, int kr) {
   return rows_possible(c, kr) && rows * k <= (long long)kCacheP * block;
 }
 
-// Co-resident workgroups that both variants of an exchange mode (rows in LDS
-// or not) hold.  Teams of several workgroups: one workgroup of 512 threads per
-// CU in either, the pool of kTeamPool bytes in the one and more than 128
-// registers a lane in the other allow no second.
-int variant_coresident(int k, int inner_fp32, int kr, int coh, int* blocks) {
-  int rc = step_max_coresident(k, inner_fp32, kr, coh, 0, blocks);
-  int with_rows = *blocks;
-  if (!rc && kr != 2) rc = step_max_coresident(k, inner_fp32, kr, coh, 1, &with_rows);
-  *blocks = std::min(*blocks, with_rows);
-  return rc;
-}
-
 // Exchange mode of a plan: plain for one-workgroup teams only; else forced,
 // then the autotuner's choice, then fenced for teams that stream their phases
 // (more rows than the row cache holds), coherent otherwise.
@@ -674,8 +663,8 @@ static Inst persistent_desc(const Inst& d) {
 // where the work per workgroup is largest; the rest are packed longest-first
 // onto single-workgroup teams (each walks its instances in turn).
 // attempt: which of the flat reduction's teams (flat_team) a lone instance may be
-// kept at, if its rows may stay in LDS there.
-int build_plan(fem_batch* b, int attempt = 0) {
+// kept at, if its rows may stay in LDS there.  cap: at most so many workgroups.
+int build_plan(fem_batch* b, int attempt = 0, int cap = INT_MAX) {
   free_plan(b);
   const int ninst = (int)b->insts.size();
   const int k = b->insts[0].k;
@@ -692,16 +681,12 @@ int build_plan(fem_batch* b, int attempt = 0) {
     }
   const int inner_fp32 = inner_bytes(b) == 4;
   const int flat = ninst == 1 && rows_possible(b->insts[0].ctx, kr) ? flat_team(k, attempt) : 0;
-  // co-resident workgroups of each variant: plain (one-workgroup teams),
-  // coherent and fenced exchange; they differ in registers
-  int maxv[3] = {0, 0, 0};
-  int rc = 0;
-  for (int m = 0; m < 3 && !rc; m++) rc = variant_coresident(k, inner_fp32, kr, m, &maxv[m]);
+  // co-resident workgroups with teams of several, and of one-workgroup teams
+  int teamed = 0, lone = 0;
+  int rc = step_plan_blocks(k, inner_fp32, kr, &teamed, &lone);
   if (rc) return rc;
-  if (std::min(maxv[0], std::min(maxv[1], maxv[2])) <= 0) {
-    set_error("persistent kernel cannot be resident on this device");
-    return FEM_ERR_HIP;
-  }
+  teamed = std::min(teamed, cap);
+  lone = std::min(lone, cap);
   std::vector<double> work(ninst);
   double W = 0;
   for (int i = 0; i < ninst; i++) {
@@ -774,14 +759,14 @@ int build_plan(fem_batch* b, int attempt = 0) {
   };
   auto any_multi = [&]() { return std::any_of(sizes.begin(), sizes.end(), [](int g) { return g > 1; }); };
   // One-workgroup teams only: the plain variant (smaller workgroups, more of
-  // them); else within what both exchange modes hold.
-  make_plan(maxv[0]);
+  // them).
+  make_plan(lone);
   bool multi = any_multi();
   if (multi) {
-    make_plan(std::min(maxv[kExchangeCoherent], maxv[kExchangeFenced]));
+    make_plan(teamed);
     multi = any_multi();
     // more instances than one workgroup per CU: the plain variant holds twice as many
-    if (!multi) make_plan(maxv[0], true);
+    if (!multi) make_plan(lone, true);
   }
   const int forced = (b->opts.exchange == FEM_EXCHANGE_COHERENT || b->opts.exchange == FEM_EXCHANGE_FENCED)
                          ? b->opts.exchange : 0;
@@ -882,15 +867,9 @@ int build_plan(fem_batch* b, int attempt = 0) {
       scattered |= sizes[t] > 1 && !fits && rows_fit(b->insts[team_inst[q]].ctx, k, sizes[t], kr);
     }
   // a team sized for rows in LDS, but the halo of a scattered numbering does not fit
-  if (flat > 0 && multi && !rows) {
-    const int maxb = std::min(maxv[kExchangeCoherent], maxv[kExchangeFenced]);
-    if (single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, maxb, 0) != grid) return build_plan(b, attempt + 1);
-  }
+  if (flat > 0 && multi && !rows && single_team_size(b->insts[0].ctx->n, k, b->opts.team_size, teamed, 0) != grid)
+    return build_plan(b, attempt + 1, cap);
   const int mode = exchange_mode(multi, streaming, forced, b->mode_override);
-  if (grid > maxv[mode]) {
-    set_error("team plan exceeds the co-resident grid");
-    return FEM_ERR_INVALID;
-  }
   // A scattered numbering whose halo does not fit gathers through the row cache,
   // which the variant with rows in LDS has no registers for.  Its gathers, each
   // from a line of its own, make it the plan's longest instance, so the plan
@@ -898,6 +877,14 @@ int build_plan(fem_batch* b, int attempt = 0) {
   // lattice nodes beside 451 x 451 scattered ones 42.0 and 24.8; 101 x 101 and
   // 221 x 221, 4 columns, 11.0 and 7.0).
   if (mode == kExchangeCoherent && scattered) rows = false;
+  int held = 0;
+  rc = step_max_coresident(k, inner_fp32, kr, mode, rows, &held);
+  if (rc) return rc;
+  if (held <= 0) {
+    set_error("persistent kernel cannot be resident on this device");
+    return FEM_ERR_HIP;
+  }
+  if (grid > held) return build_plan(b, attempt, held);
   b->uploaded = hi;
   b->launch.teams = b->d_teams;
   b->launch.wg_team = b->d_wg_team;
@@ -1857,8 +1844,7 @@ int batch_autotune(fem_batch* b, int probe, int* chosen, double* best_ms) {
   int rc = batch_prepare(b, true);
   if (rc) return rc;
   int maxb = 0, alone = 0;  // workgroups of teams of several, and of one-workgroup teams
-  rc = variant_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, kExchangeCoherent, &maxb);
-  if (!rc) rc = variant_coresident(b->launch.k, b->launch.inner_fp32, b->launch.kr, 0, &alone);
+  rc = step_plan_blocks(b->launch.k, b->launch.inner_fp32, b->launch.kr, &maxb, &alone);
   if (rc) return rc;
   const bool single = b->insts.size() == 1;
   // Rows x columns per lane of the whole co-resident grid: beyond ~64 every

@@ -35,7 +35,6 @@ void team_slots(Team* T, double* slots, int grid, int k);
 bool team_streams(long long n, int k, int size);
 bool rows_possible(const fem_ctx* c, int kr);
 bool rows_fit(const fem_ctx* c, int k, int size, int kr);
-int variant_coresident(int k, int inner_fp32, int kr, int coh, int* blocks);
 int exchange_mode(bool multi, bool streaming, int forced, int tuned);
 int launch_slot_reset(double* slots, int nrec, int rec_vals, int* abort_flag, Inst* insts, int ninst,
                       hipStream_t st);
@@ -80,6 +79,7 @@ int stream_run(const StreamPlan* p, const Inst* d_insts, int max_sweeps, int max
 // Column counts whose stream phases use the multi-column layout with the
 // staged pattern (one value column, Inst::SDi present).
 bool stream_vec_layout(int k);
+int step_plan_blocks(int k, int inner_fp32, int kr, int* teamed, int* alone);
 int step_max_coresident(int k, int inner_fp32, int kr, int coh, int rows, int* blocks);
 int step_graph_node(const StepLaunch& L, int nsteps, hipGraph_t g, hipGraphNode_t dep, hipGraphNode_t* out);
 

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -90,9 +91,9 @@ __global__ void k_noalloc_setup(Team team, Inst inst, HaloRef halo, int grid, Te
   for (long long q = i; q < nzero; q += (long long)gridDim.x * blockDim.x) zero[q] = 0.0;
 }
 
-// attempt as in build_plan: the same plan, so the same results bit for bit.
+// attempt and cap as in build_plan: the same plan, so the same results bit for bit.
 int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
-                  fem_step_stats* stats, int attempt) {
+                  fem_step_stats* stats, int attempt, int cap) {
   fem_solver_opts o;
   fem_opts_default(&o);
   if (opts) o = *opts;
@@ -120,22 +121,13 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
   const int flat = rows_possible(c, kri) ? flat_team(k, attempt) : 0;
 
   // plan: one team, sized and moded as a one-instance batch plan
-  int maxv[3] = {0, 0, 0};
-  for (int m = 0; m < 3; m++) {
-    const int rc = variant_coresident(k, fp32, kri, m, &maxv[m]);
-    if (rc) return rc;
-  }
+  int maxb = 0, lone = 0;
+  int rc = step_plan_blocks(k, fp32, kri, &maxb, &lone);
+  if (rc) return rc;
+  maxb = std::min(maxb, cap);
   const int forced = (o.exchange == FEM_EXCHANGE_COHERENT || o.exchange == FEM_EXCHANGE_FENCED) ? o.exchange : 0;
-  int grid = single_team_size(n, k, o.team_size, maxv[kExchangeCoherent], flat);
-  int mode = exchange_mode(grid > 1, team_streams(n, k, grid), forced, 0);
-  if (grid > maxv[mode]) {
-    grid = single_team_size(n, k, o.team_size, std::min(maxv[0], std::min(maxv[1], maxv[2])), flat);
-    mode = exchange_mode(grid > 1, team_streams(n, k, grid), forced, 0);
-  }
-  if (grid <= 0 || grid > maxv[mode]) {
-    set_error("persistent kernel cannot be resident on this device");
-    return FEM_ERR_HIP;
-  }
+  const int grid = single_team_size(n, k, o.team_size, maxb, flat);
+  const int mode = exchange_mode(grid > 1, team_streams(n, k, grid), forced, 0);
 
   // footprint
   Layout L;
@@ -173,7 +165,7 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
     return FEM_ERR_INVALID;
   }
   unsigned char* base = nullptr;
-  int rc = scratch_ptr(&base);
+  rc = scratch_ptr(&base);
   if (rc) return rc;
 
   double* slots = (double*)(base + o_slots);
@@ -269,8 +261,16 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
     FEM_HIP(hipStreamSynchronize(st));
   }
   const bool rows = grid == 1 ? rows_fit(c, k, 1, kri) : built.ok != 0;
-  if (flat > 0 && grid > 1 && !rows && single_team_size(n, k, o.team_size, maxv[mode], 0) != grid)
-    return solve_noalloc(c, coef, opts, bh, xh, stats, attempt + 1);
+  if (flat > 0 && grid > 1 && !rows && single_team_size(n, k, o.team_size, maxb, 0) != grid)
+    return solve_noalloc(c, coef, opts, bh, xh, stats, attempt + 1, cap);
+  int held = 0;
+  rc = step_max_coresident(k, fp32, kri, mode, rows, &held);
+  if (rc) return rc;
+  if (held <= 0) {
+    set_error("persistent kernel cannot be resident on this device");
+    return FEM_ERR_HIP;
+  }
+  if (grid > held) return solve_noalloc(c, coef, opts, bh, xh, stats, attempt, held);
   StepLaunch SL;
   SL.teams = d_team;
   SL.wg_team = d_wg_team;
@@ -316,7 +316,7 @@ int solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts,
 
 int linear_solve_noalloc(fem_ctx* c, const double coef[3], const fem_solver_opts* opts, const double* bh, double* xh,
                          fem_step_stats* stats) {
-  return solve_noalloc(c, coef, opts, bh, xh, stats, 0);
+  return solve_noalloc(c, coef, opts, bh, xh, stats, 0, INT_MAX);
 }
 
 }  // namespace femhip

@@ -115,6 +115,27 @@ int step_graph_node(const StepLaunch& L, int nsteps, hipGraph_t g, hipGraphNode_
   return 0;
 }
 
+// Workgroups that a plan is sized within: one per CU with teams of several, two
+// of the half as large workgroups of one-workgroup teams.  Every variant holds
+// as many by its registers (two waves per SIMD) and the pool of rows in LDS.  Asking the runtime loads the variant's code object: 2 to 6 ms
+// each, 24 for the six variants that a plan may come to, of which it runs one.
+// So a plan asks for that one alone (step_max_coresident).  First advance of a
+// process, one instance of 9,801 rows, ms: 12 to 16 with the three variants
+// before rows were kept in LDS, 28 asking for all six, 11 so.
+int step_plan_blocks(int k, int inner_fp32, int kr, int* teamed, int* alone) {
+  if (!pick_kernel(k, inner_fp32, kr, 0, 0)) {
+    set_error("unsupported kernel configuration (number of right-hand sides must be 1, 2, 4 or 16)");
+    return FEM_ERR_INVALID;
+  }
+  int dev = 0, cus = 0;
+  FEM_HIP(hipGetDevice(&dev));
+  FEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  *teamed = cus;
+  *alone = cus * (kTeamBlock / kBlock);
+  return 0;
+}
+
+// Workgroups of one variant that the device holds at once.
 // coh: 0 plain (one-workgroup teams), 1 coherent, 2 fenced.
 int step_max_coresident(int k, int inner_fp32, int kr, int coh, int rows, int* blocks) {
   const void* fn = pick_kernel(k, inner_fp32, kr, coh, rows);
