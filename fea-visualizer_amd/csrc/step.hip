@@ -31,8 +31,8 @@ const void* pick_kernel(int k, int fp32, int kr, int coh, int rows) {
 // Threads per workgroup of the variants of one exchange mode.
 int team_block(int coh) { return coh == 0 ? kBlock : kTeamBlock; }
 
-// Workgroups of kernel `fn` (of `block` threads) that fit the current device at once.  Cached per
-// (device, kernel): the answer depends only on the code object.
+// Workgroups of kernel `fn` (of `block` threads) that fit the current device at
+// once.  Cached per (device, kernel): the answer depends only on the code object.
 int kernel_max_coresident(const void* fn, int block, int* blocks) {
   constexpr int kMaxDev = 16, kMaxFn = 128;
   struct Entry { const void* fn; int blocks; };
@@ -117,11 +117,12 @@ int step_graph_node(const StepLaunch& L, int nsteps, hipGraph_t g, hipGraphNode_
 
 // Workgroups that a plan is sized within: one per CU with teams of several, two
 // of the half as large workgroups of one-workgroup teams.  Every variant holds
-// as many by its registers (two waves per SIMD) and the pool of rows in LDS.  Asking the runtime loads the variant's code object: 2 to 6 ms
-// each, 24 for the six variants that a plan may come to, of which it runs one.
-// So a plan asks for that one alone (step_max_coresident).  First advance of a
-// process, one instance of 9,801 rows, ms: 12 to 16 with the three variants
-// before rows were kept in LDS, 28 asking for all six, 11 so.
+// as many by its registers (two waves per SIMD) and the pool of rows in LDS.
+// Asking the runtime loads the variant's code object: 2 to 6 ms each, 24 for the
+// six variants that a plan may come to, of which it runs one.  So a plan asks
+// for that one alone (step_max_coresident).  First advance of a process, one
+// instance of 9,801 rows, ms: 12 to 16 with the three variants before rows were
+// kept in LDS, 28 asking for all six, 11 so.
 int step_plan_blocks(int k, int inner_fp32, int kr, int* teamed, int* alone) {
   if (!pick_kernel(k, inner_fp32, kr, 0, 0)) {
     set_error("unsupported kernel configuration (number of right-hand sides must be 1, 2, 4 or 16)");
